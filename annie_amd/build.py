@@ -46,15 +46,26 @@ def _newer(target, sources):
 def build_hip(force=True):
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libannie_hip.so")
-    srcs = [os.path.join(CSRC, f) for f in ("kernels.hip", "engine.hip")]
-    deps = srcs + [os.path.join(CSRC, f) for f in ("arith.h", "plan.h", "kernels.h")]
+    srcs = [os.path.join(CSRC, f) for f in ("kernels.hip", "lazy.hip", "engine.hip")]
+    deps = srcs + [os.path.join(CSRC, f) for f in ("arith.h", "plan.h", "kernels.h", "lazy.h", "rounds.h")]
     deps.append(os.path.join(REPO, "include", "annie_hip.h"))
     if not force and not _newer(out, deps):
         return out
+    # One compiler per source, side by side.
+    objs = [os.path.join(LIBDIR, os.path.basename(f) + ".o") for f in srcs]
+    cmds = [[HIPCC, *HIP_FLAGS, "-c", "-I" + GMP_INC, "-I" + os.path.join(REPO, "include"), s, "-o", o]
+            for s, o in zip(srcs, objs)]
+    for cmd in cmds:
+        print(" ".join(cmd), flush=True)
+    procs = [subprocess.Popen(cmd) for cmd in cmds]
+    codes = [p.wait() for p in procs]
+    if any(codes):
+        raise RuntimeError("hipcc failed")
     tmp = out + ".tmp"
-    _run([HIPCC, *HIP_FLAGS, "-shared", "-I" + GMP_INC, "-I" + os.path.join(REPO, "include"),
-          *srcs, "-o", tmp, *GMP_LIB])
+    _run([HIPCC, *HIP_FLAGS, "-shared", *objs, "-o", tmp, *GMP_LIB])
     os.replace(tmp, out)
+    for o in objs:
+        os.remove(o)
     return out
 
 

@@ -19,6 +19,7 @@
 
 #include "../../include/annie_hip.h"
 #include "kernels.h"
+#include "lazy.h"
 #include "plan.h"
 
 namespace annie {
@@ -39,6 +40,19 @@ __global__ void k_copy_slots(uint32_t* base, size_t dst_off, size_t src_off, siz
                              size_t slot_stride);
 template <int M, int K, int QS>
 __global__ void k_sqr_run(const RunArgs R);
+template <int M, int LR, int MODE, int SRC>
+__global__ void k_lz_row(const LzNtt A);
+template <int M, int DL>
+__global__ void k_lz_colf(const LzNtt A);
+template <int M>
+__global__ void k_lz_coli(const LzNtt A);
+template <int KP, int L, int ND, int DL, bool NEGA>
+__global__ void k_lz_carry(const LzCarry A);
+__global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
+template <int K, int DL>
+__global__ void k_lz_import(const LzConv A);
+template <int K, int DL>
+__global__ void k_lz_export(const LzConv A);
 
 static thread_local std::string g_last_error;
 
@@ -88,8 +102,38 @@ struct Stage {
   bool pending[NSTAGE] = {};
 };
 
+// The short-prime path of a context (lazy.h).  A slot holds NLZ digit
+// registers of DL n words, the planes of N^-1 mod R and N, the work planes and
+// a block of flags (the sign of m').
+enum LzReg : int { LX0 = 0, LX1 = 1, LX2 = 2, LZ_ONE, LZ_SNAP, LZ_MP, LZ_GET, NLZ };
+enum LzPlanes : int { PNIR = 0, PNQ, PWR, PWQ, PMQ, PYR, PYQ, NPLANES };
+constexpr size_t LZ_FLAGS = 64;
+
+struct Lazy {
+  bool on = false;
+  LzShape sh{};
+  int LR = 3;  // log2 of the elements per thread of the row passes
+  std::vector<uint32_t> primes;
+  LzPrimes pc{};
+  int32_t scaleR[LZ_MAXP] = {}, scaleQ[LZ_MAXP] = {};  // of the transforms of N^-1 mod R and N
+  LzCarry cr{}, cq{};                                  // CRT constants of the cyclic / negacyclic planes
+  uint32_t* mem = nullptr;
+  uint32_t* tw = nullptr;  // roots: KR n cyclic forward, KR n inverse, KQ n negacyclic forward, KQ n inverse
+  size_t stride = 0, plane0 = 0;
+  // Registers that hold the constant 1 as set1 leaves it, whose external form
+  // has the non-negative digits of its residue.
+  bool is_one[3] = {false, false, false};
+  uint32_t last_a = 1;  // last multiplier found to fit
+};
+
 struct Ctx {
   Plan pl;
+  Lazy lz;
+  // The long-prime file below is set up (always without the short-prime
+  // path; with it, for diagnostics or on demotion).
+  bool long_ready = false;
+  // The last stage diagnostic is newer than the last product.
+  bool staged = false;
   int device = 0;
   int m1 = 0, m2 = 0;
   // Launch schedule of the NTT passes (0: the default): lines per row-pass
@@ -163,6 +207,14 @@ struct Ctx {
   const TwDev* invR() const { return tw + 1 * size_t(pl.K) * n; }
   const TwDev* fwdQ() const { return tw + 2 * size_t(pl.K) * n; }
   const TwDev* invQ() const { return tw + 3 * size_t(pl.K) * n; }
+
+  uint32_t* lzreg(int r) const { return lz.mem + size_t(r) * size_t(lz.sh.DL) * n; }
+  uint32_t* lzplane(int p) const {
+    const size_t kr = size_t(lz.sh.KR), kq = size_t(lz.sh.KQ);
+    const size_t at[NPLANES + 1] = {0, kr, kr + kq, 2 * kr + kq, 2 * kr + 2 * kq, 2 * kr + 3 * kq, 3 * kr + 3 * kq, 3 * kr + 4 * kq};
+    return lz.mem + lz.plane0 + at[p] * n;
+  }
+  uint32_t* lzflags() const { return lzplane(NPLANES); }
 };
 
 }  // namespace annie
@@ -186,12 +238,17 @@ static NttJob job(const uint32_t* src, uint32_t* dst, const TwDev* f, const TwDe
   return j;
 }
 
-// Records an event pair around the next launch when profiling is on.
+// Records an event pair around the next launch when profiling is on.  The
+// name, `base<m,mode>x<count>`, is only put together then.
 struct ProfScope {
   Ctx& c;
   size_t rec = size_t(-1);
-  ProfScope(Ctx& cc, const std::string& name) : c(cc) {
+  ProfScope(Ctx& cc, const char* base, int m, const char* mode, int count) : c(cc) {
     if (!c.profiling) return;
+    std::string name = std::string(base) + "<" + std::to_string(m);
+    if (mode != nullptr) name += std::string(",") + mode;
+    name += ">";
+    if (count > 0) name += "x" + std::to_string(count);
     int kind = -1;
     for (size_t i = 0; i < c.kinds.size(); ++i)
       if (c.kinds[i] == name) kind = int(i);
@@ -295,7 +352,7 @@ static int launch_row(Ctx& c, int mode, const NttJob* jobs, int nj) {
   A.cols = int(lines);
   const dim3 grid(rows / lines, c.pl.K, nj * c.nslots), block(lines * Tl);
   const size_t shm = size_t(lines) * (S + (S >> 5)) * sizeof(uint32_t);
-  ProfScope ps(c, "k_row<" + std::to_string(c.m2) + "," + row_mode_name(mode) + ">x" + std::to_string(nj));
+  ProfScope ps(c, "k_row", c.m2, row_mode_name(mode), nj);
   switch (c.m2) {
     case 4: launch_row_m<4>(mode, grid, block, shm, c.cur, A); break;
     case 5: launch_row_m<5>(mode, grid, block, shm, c.cur, A); break;
@@ -335,7 +392,7 @@ static int launch_col(Ctx& c, bool inverse, const NttJob* jobs, int nj) {
   A.cols = int(C);
   const dim3 grid(n2 / C, c.pl.K, nj * c.nslots), block(C * Tl);
   const size_t shm = size_t(wide ? C : C + 1) * S * sizeof(uint32_t);
-  ProfScope ps(c, std::string(inverse ? "k_col_inv<" : "k_col_fwd<") + std::to_string(c.m1) + ">x" + std::to_string(nj));
+  ProfScope ps(c, inverse ? "k_col_inv" : "k_col_fwd", c.m1, nullptr, nj);
   switch (c.m1) {
     case 7: launch_col_m<7>(inverse, grid, block, shm, c.cur, A); break;
     case 8: launch_col_m<8>(inverse, grid, block, shm, c.cur, A); break;
@@ -400,7 +457,7 @@ static int launch_carry(Ctx& c, const CarryJob* jobs, int nj, const uint32_t* a_
   const dim3 grid(unsigned((nb + CARRY_WG - 2) / (CARRY_WG - 1)), nj * c.nslots), block(CARRY_WG);
   const int qs = c.pl.cbits() >> 5;
   if (qs > 2) return fail(ANNIE_ERR_SIZE, "digit width above 95 bits");
-  ProfScope ps(c, "k_carry<" + std::to_string(c.pl.K) + ">x" + std::to_string(nj));
+  ProfScope ps(c, "k_carry", c.pl.K, nullptr, nj);
   switch (c.pl.K * 4 + qs) {
 #define ANNIE_CARRY_CASE(K, QS) \
   case K * 4 + QS: hipLaunchKernelGGL((k_carry<K, QS>), grid, block, 0, c.cur, A); break;
@@ -475,6 +532,17 @@ static int reduce(Ctx& c, uint32_t* dst, bool raw_out, const uint32_t* snap = nu
   return reduce(c, ctx_bufs(c), dst, raw_out, snap, join);
 }
 
+static int lz_square(Ctx& c, uint32_t a, const uint32_t* a_slot, bool bits);
+static int lz_mul(Ctx& c, int dst, int src);
+static int lz_copy(Ctx& c, int dst, int src);
+static int lz_get_values(Ctx& c, int src, const size_t* slots, const mpz_t* const* mods, mpz_t* const* zs, size_t count);
+static int lz_load_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv);
+static int lz_setup(Ctx& c);
+static bool lz_class_fits(const Plan& pl);
+
+// The short-prime register of a register index.
+static int lz_of(int r) { return r == RONE ? int(LZ_ONE) : r == RSNAP ? int(LZ_SNAP) : r; }
+
 // squareMMGW (src/transformGPU.h:556-568): B.y = a B.x^2.  a_slot: per-slot
 // multipliers of a batch operation (device array in slot-list order),
 // replacing a.
@@ -512,12 +580,14 @@ static int square_mul(Ctx& c, const SqBufs& B, uint32_t a, const uint32_t* a_slo
 }
 
 static int square_mul(Ctx& c, uint32_t a, const uint32_t* a_slot = nullptr, bool bits = false) {
+  if (c.lz.on) return lz_square(c, a, a_slot, bits);
   return square_mul(c, ctx_bufs(c), a, a_slot, bits);
 }
 
 // mulMMGW (src/transformGPU.h:540-554).
 static int mul(Ctx& c, int dst, int src) {
   int rc;
+  if (c.lz.on) return lz_mul(c, dst, lz_of(src));
   const NttJob f[2] = {job(c.reg(src), c.reg(RSR), c.fwdR(), c.invR()), job(c.reg(src), c.reg(RSQ), c.fwdQ(), c.invQ())};
   if ((rc = forward(c, f, 2))) return rc;
   const NttJob j[2] = {job(c.reg(dst), c.reg(RWR), c.fwdR(), c.invR(), c.reg(RSR)),
@@ -530,6 +600,7 @@ static int mul(Ctx& c, int dst, int src) {
 
 static int copy_reg(Ctx& c, int dst, int src) {
   if (dst == src) return ANNIE_OK;
+  if (c.lz.on) return lz_copy(c, dst, lz_of(src));
   const size_t len = size_t(c.pl.K) * c.n;
   if (c.slot_ids == nullptr) {
     HIPCHK(hipMemcpyAsync(c.reg(dst), c.reg(src), len * 4, hipMemcpyDeviceToDevice, c.stream));
@@ -542,8 +613,9 @@ static int copy_reg(Ctx& c, int dst, int src) {
   return ANNIE_OK;
 }
 
-// Signed digits (DIGIT_LIMBS planes, two's complement) -> integer sum d_i B^i.
-static void digits_to_mpz(const Ctx& c, const std::vector<uint32_t>& d, int cb, mpz_t z) {
+// Signed digits (at(i): digit i) -> integer sum d_i B^i.
+template <class At>
+static void digits_to_mpz(const Ctx& c, At at, int cb, mpz_t z) {
   const size_t n = c.n;
   const size_t nbits = n * size_t(cb);
   const size_t nl = nbits / 64 + 3;
@@ -552,11 +624,7 @@ static void digits_to_mpz(const Ctx& c, const std::vector<uint32_t>& d, int cb, 
   size_t pos = 0;
   const unsigned __int128 mask = (cb >= 128) ? ~(unsigned __int128)0 : (((unsigned __int128)1 << cb) - 1);
   for (size_t i = 0; i < n; ++i) {
-    const unsigned __int128 u =
-        (unsigned __int128)d[i] | ((unsigned __int128)d[n + i] << 32) | ((unsigned __int128)d[2 * n + i] << 64);
-    // sign-extend the 96-bit digit
-    __int128 v = (__int128)(u << 32) >> 32;
-    v += carry;
+    const __int128 v = __int128(at(i)) + carry;
     const unsigned __int128 dig = (unsigned __int128)v & mask;
     carry = v >> cb;
     // write dig (cb bits) at bit position pos
@@ -606,16 +674,10 @@ static void mpz_to_digit_planes(const Ctx& c, const mpz_t x, int cb, std::vector
   }
 }
 
-// set_mpz (src/transformGPU.h:323-360): the host splits x into digits, the
-// device encodes them into K residue planes.
-static int upload_mpz(Ctx& c, int r, const mpz_t x, size_t slot = 0) {
-  std::vector<uint32_t> h;
-  mpz_to_digit_planes(c, x, slot_cbits(c, slot), h);
-  uint32_t* digits = c.rawtmp() + slot * c.slot_stride;
-  HIPCHK(hipMemcpyAsync(digits, h.data(), h.size() * 4, hipMemcpyHostToDevice, c.stream));
+// RNS encode: DIGIT_LIMBS digit planes -> K residue planes.
+static int encode_digits(Ctx& c, const uint32_t* digits, uint32_t* dst) {
   CarryArgs A = c.cbase;
   const dim3 grid(unsigned((c.n / CARRY_L + 255) / 256)), block(256);
-  uint32_t* dst = slot_reg(c, r, slot);
   switch (c.pl.K) {
     case 2: hipLaunchKernelGGL(k_digits_to_res<2>, grid, block, 0, c.stream, digits, dst, A); break;
     case 3: hipLaunchKernelGGL(k_digits_to_res<3>, grid, block, 0, c.stream, digits, dst, A); break;
@@ -623,6 +685,17 @@ static int upload_mpz(Ctx& c, int r, const mpz_t x, size_t slot = 0) {
     default: hipLaunchKernelGGL(k_digits_to_res<5>, grid, block, 0, c.stream, digits, dst, A); break;
   }
   HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+// set_mpz (src/transformGPU.h:323-360): the host splits x into digits, the
+// device encodes them into K residue planes.
+static int upload_mpz(Ctx& c, int r, const mpz_t x, size_t slot = 0) {
+  std::vector<uint32_t> h;
+  mpz_to_digit_planes(c, x, slot_cbits(c, slot), h);
+  uint32_t* digits = c.rawtmp() + slot * c.slot_stride;
+  HIPCHK(hipMemcpyAsync(digits, h.data(), h.size() * 4, hipMemcpyHostToDevice, c.stream));
+  if (int rc = encode_digits(c, digits, slot_reg(c, r, slot))) return rc;
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
 }
@@ -637,12 +710,409 @@ static int scale_reg(Ctx& c, int r, size_t slot = 0) {
   return ANNIE_OK;
 }
 
+// ---------------------------------------------------------------------------
+// The short-prime path (lazy.h): products of digit registers.
+
+// Whether a class of plans (one K, LN and digit-width class; the digit width
+// and the base vary with N and a) runs on the short-prime path: its widest
+// digits have to fit.  A context whose multipliers or digits turn out not to
+// fit is demoted to the long primes.
+static bool lz_class_fits(const Plan& pl) {
+  const char* off = std::getenv("ANNIE_LONG_PRIMES");
+  if (off && off[0] == '1') return false;
+  if (pl.K < 3 || pl.LN < 8 || pl.LN > 20) return false;
+  double lp = -1.0;
+  for (int k = 0; k < pl.K; ++k) lp += std::log2(double(PRIMES[k]));
+  int cb = pl.cbits();
+  for (int b = cb + pl.pck; (b >> 5) == (pl.cbits() >> 5) && pl.LN + 2 * b < lp; b += pl.pck) cb = b;
+  return lz_fits(pl, cb, 1u, lz_primes(pl.LN, lz_shape(pl.K).KR)) && lz_fits(pl, pl.cbits(), 1u, lz_primes(pl.LN, lz_shape(pl.K).KR));
+}
+
+// Words of one slot.
+static size_t lz_slot_words(int K, size_t n) {
+  const LzShape sh = lz_shape(K);
+  return (size_t(NLZ) * size_t(sh.DL) + 3 * size_t(sh.KR) + 4 * size_t(sh.KQ)) * n + LZ_FLAGS;
+}
+
+static int32_t lz_signed(uint64_t v, uint32_t p) { return v > p / 2 ? int32_t(v) - int32_t(p) : int32_t(v); }
+
+// CRT constants of the first `count` primes on L limbs.
+static void lz_crt_consts(LzCarry& A, const std::vector<uint32_t>& primes, int count, int L) {
+  Mpz P, M, t;
+  mpz_set_ui(P.v, 1);
+  for (int k = 0; k < count; ++k) mpz_mul_ui(P.v, P.v, primes[k]);
+  auto limbs = [&](const mpz_t z, uint32_t* out) {
+    std::memset(out, 0, LZ_MAXL * 4);
+    mpz_export(out, nullptr, -1, 4, 0, 0, z);
+  };
+  for (int k = 0; k < count; ++k) {
+    const uint32_t p = primes[k];
+    mpz_divexact_ui(M.v, P.v, p);
+    limbs(M.v, A.M[k]);
+    A.p[k] = p;
+    A.q[k] = inv32(p);
+    A.inv[k] = float(1.0 / double(p));
+    A.c[k] = lz_signed(to_mont(invmod_plain(uint32_t(mpz_fdiv_ui(M.v, p)), p), p), p);
+  }
+  mpz_set_ui(t.v, 1);
+  mpz_mul_2exp(t.v, t.v, 32u * unsigned(L));
+  mpz_sub(t.v, t.v, P.v);
+  limbs(t.v, A.NP);
+}
+
+// Limbs of the carries' CRT values (as instantiated in lazy.hip).
+static int lz_limbs(int K, bool cyc) { return cyc ? (K == 3 ? 6 : K == 4 ? 7 : 8) : (K == 3 ? 4 : K == 4 ? 5 : 6); }
+
+static int lz_elements(const Ctx& c) {
+  if (const char* e = std::getenv("ANNIE_LZ_LR")) return std::atoi(e);
+  return (c.nslots_alloc << c.pl.LN) >= (size_t(1) << 17) ? 4 : 3;
+}
+
+static int lz_setup(Ctx& c) {
+  Lazy& z = c.lz;
+  const int LN = c.pl.LN, K = c.pl.K;
+  const size_t n = c.n;
+  z.sh = lz_shape(K);
+  z.primes = lz_primes(LN, z.sh.KR);
+  const int KR = z.sh.KR, KQ = z.sh.KQ, DL = z.sh.DL;
+  // Sixteen elements per thread where the launch fills the GPU (fewer LDS
+  // exchanges), eight where it leaves CUs idle (shorter chains per thread).
+  z.LR = lz_elements(c);
+  z.stride = lz_slot_words(K, n);
+  z.plane0 = size_t(NLZ) * size_t(DL) * n;
+  if (hipMalloc(&z.mem, c.nslots_alloc * z.stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
+  if (hipMalloc(&z.tw, (2 * size_t(KR) + 2 * size_t(KQ)) * n * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "roots");
+  HIPCHK(hipMemsetAsync(z.mem, 0, c.nslots_alloc * z.stride * 4, c.stream));
+  lz_crt_consts(z.cr, z.primes, KR, lz_limbs(K, true));
+  lz_crt_consts(z.cq, z.primes, KQ, lz_limbs(K, false));
+  // Powers psi^i, i < 2^s, and psi^{i 2^s} of a primitive 2n-th root psi of
+  // each prime; the device multiplies them into the tables.
+  const int s = (LN + 1) / 2, hi = LN + 1 - s;
+  const size_t per = (size_t(1) << s) + (size_t(1) << hi);
+  std::vector<uint32_t> pw(size_t(KR) * per);
+  for (int k = 0; k < KR; ++k) {
+    const uint32_t p = z.primes[k];
+    z.pc.p[k] = p;
+    z.pc.q[k] = inv32(p);
+    z.pc.bar[k] = uint32_t((uint64_t(1) << 58) / p);
+    const uint32_t ninv = invmod_plain(uint32_t(n % p), p), bi = pow2mod(32u * unsigned(DL - 1), p);  // 1 / b
+    const uint32_t ns = mulmod_plain(ninv, mulmod_plain(bi, bi, p), p);                                // n^-1 b^-2
+    z.pc.cq[k] = lz_signed(mulmod_plain(ns, pow2mod(96, p), p), p);
+    z.pc.one[k] = lz_signed(invmod_plain(bi, p), p);
+    z.scaleR[k] = lz_signed(mulmod_plain(mulmod_plain(ns, bi, p), pow2mod(96, p), p), p);
+    z.scaleQ[k] = lz_signed(mulmod_plain(ns, pow2mod(64, p), p), p);
+    const uint32_t psi = powmod_plain(lz_nonresidue(p), (uint64_t(p) - 1) >> (LN + 1), p);
+    uint32_t* w = pw.data() + size_t(k) * per;
+    uint32_t v = to_mont(1, p);
+    for (size_t i = 0; i < (size_t(1) << s); ++i, v = mulmod_plain(v, psi, p)) w[i] = v;
+    const uint32_t step = powmod_plain(psi, uint64_t(1) << s, p);
+    v = to_mont(1, p);
+    for (size_t i = 0; i < (size_t(1) << hi); ++i, v = mulmod_plain(v, step, p)) w[(size_t(1) << s) + i] = v;
+  }
+  uint32_t* dpw = c.lzplane(PWR);  // scratch: per < n words for every length of this path
+  HIPCHK(hipMemcpyAsync(dpw, pw.data(), pw.size() * 4, hipMemcpyHostToDevice, c.stream));
+  hipLaunchKernelGGL(k_lz_roots, dim3(unsigned((n + 255) / 256), unsigned(KR)), dim3(256), 0, c.stream, z.tw, dpw, LN, KR, KQ,
+                     z.pc);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(c.stream));
+  z.on = true;
+  return ANNIE_OK;
+}
+
+typedef void (*LzKernel)(const LzNtt);
+
+template <int M, int SRC>
+static LzKernel lz_row_kernel(int LR, int mode) {
+  if (LR == 3) return mode == LZ_SQR ? k_lz_row<M, 3, LZ_SQR, SRC> : mode == LZ_MULN ? k_lz_row<M, 3, LZ_MULN, SRC> : k_lz_row<M, 3, LZ_GEN, SRC>;
+  return mode == LZ_SQR ? k_lz_row<M, 4, LZ_SQR, SRC> : mode == LZ_MULN ? k_lz_row<M, 4, LZ_MULN, SRC> : k_lz_row<M, 4, LZ_GEN, SRC>;
+}
+
+// Rows of planes [A.pl0, A.pl0 + planes): the whole transform of a digit
+// register (single-pass lengths), or the row levels of planes in place.
+static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
+  const Lazy& z = c.lz;
+  const bool single = c.m1 == 0;
+  const uint32_t S = 1u << c.m2, T = S >> z.LR, rows = 1u << c.m1;
+  uint32_t lines = 1;
+  if (T < 64 && !single) {
+    lines = row_lines_default(c.m1, c.m2);
+    if (c.sched_lines != 0) lines = c.sched_lines;  // checked by annie_hip_set_schedule
+  }
+  A.cols = int(lines);
+  const dim3 grid(rows / lines, unsigned(planes), unsigned(c.nslots)), block(lines * T);
+  const size_t shm = size_t(lines) * (S + (S >> 5)) * 4;
+  LzKernel f = nullptr;
+  switch (single ? 100 * z.sh.DL + c.m2 : c.m2) {
+#define LZ_CASE1(M)                                           \
+  case 200 + M: f = lz_row_kernel<M, 2>(z.LR, mode); break; \
+  case 300 + M: f = lz_row_kernel<M, 3>(z.LR, mode); break;
+    LZ_CASE1(8)
+    LZ_CASE1(9)
+    LZ_CASE1(10)
+    LZ_CASE1(11)
+    LZ_CASE1(12)
+    LZ_CASE1(13)
+#undef LZ_CASE1
+    case 7: f = lz_row_kernel<7, 0>(z.LR, mode); break;
+    case 8: f = lz_row_kernel<8, 0>(z.LR, mode); break;
+    case 9: f = lz_row_kernel<9, 0>(z.LR, mode); break;
+    case 10: f = lz_row_kernel<10, 0>(z.LR, mode); break;
+    default: return fail(ANNIE_ERR_SIZE, "no row kernel for this length");
+  }
+  ProfScope ps(c, "k_lz_row", c.m2, mode == LZ_SQR ? "sqr" : mode == LZ_MULN ? "muln" : "gen", planes);
+  hipLaunchKernelGGL(f, grid, block, shm, c.stream, A);
+  HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
+  const bool wide = c.m1 >= 10;
+  const uint32_t S = 1u << c.m1, T = S / (wide ? 32u : 16u);
+  uint32_t C = col_cols_default(c.m1, c.pl.LN);
+  if (c.sched_cols != 0 && !wide) C = c.sched_cols;  // checked by annie_hip_set_schedule
+  if (wide && C != 8u) return fail(ANNIE_ERR_SIZE, "column pass geometry");
+  A.cols = int(C);
+  const dim3 grid(uint32_t(c.n >> c.m1) / C, unsigned(planes), unsigned(c.nslots)), block(C * T);
+  const size_t shm = size_t(wide ? C : C + 1) * S * 4;
+  LzKernel f = nullptr;
+  switch (c.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
+#define LZ_CASE(M)                                  \
+  case M * 4: f = k_lz_coli<M>; break;              \
+  case M * 4 + 2: f = k_lz_colf<M, 2>; break;       \
+  case M * 4 + 3: f = k_lz_colf<M, 3>; break;
+    LZ_CASE(7)
+    LZ_CASE(8)
+    LZ_CASE(9)
+    LZ_CASE(10)
+#undef LZ_CASE
+    default: return fail(ANNIE_ERR_SIZE, "no column kernel for this length");
+  }
+  ProfScope ps(c, inverse ? "k_lz_coli" : "k_lz_colf", c.m1, nullptr, planes);
+  hipLaunchKernelGGL(f, grid, block, shm, c.stream, A);
+  HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+// Transform passes: planes [pl0, pl0 + planes) forward from the digits A.x, the
+// pointwise step of `mode`, and the inverse of the first `back` of them.
+static int lz_transform(Ctx& c, LzNtt& A, int mode, int pl0, int planes, int back) {
+  int rc;
+  A.pl0 = pl0;
+  if (c.m1 > 0 && (rc = lz_col(c, A, false, planes))) return rc;
+  if ((rc = lz_row(c, A, mode, planes))) return rc;
+  if (c.m1 > 0 && back > 0 && (rc = lz_col(c, A, true, back))) return rc;
+  return ANNIE_OK;
+}
+
+static LzNtt lz_args(const Ctx& c) {
+  const Lazy& z = c.lz;
+  LzNtt A{};
+  A.c = z.pc;
+  const size_t n = c.n, KR = size_t(z.sh.KR), KQ = size_t(z.sh.KQ);
+  A.fwdR = z.tw;
+  A.invR = z.tw + KR * n;
+  A.fwdQ = z.tw + 2 * KR * n;
+  A.invQ = z.tw + (2 * KR + KQ) * n;
+  A.nir = c.lzplane(PNIR);
+  A.nq = c.lzplane(PNQ);
+  A.slot_ids = c.slot_ids;
+  A.slot_stride = z.stride;
+  A.LN = c.pl.LN;
+  A.m1 = c.m1;
+  A.KR = z.sh.KR;
+  A.mul.a = 1u;
+  return A;
+}
+
+static int lz_carry(Ctx& c, LzCarry& A, bool cyc) {
+  const int nd = cyc ? (c.pl.K == 3 ? 5 : 4) : 3;
+  const size_t waves = (c.n + size_t(63 - nd)) / size_t(64 - nd);
+  const dim3 grid(unsigned((waves + 3) / 4), unsigned(c.nslots)), block(256);
+  A.slot_ids = c.slot_ids;
+  A.slot_stride = c.lz.stride;
+  A.LN = c.pl.LN;
+  A.cbits = c.pl.cbits();
+  A.cbits_slot = c.cbits_dev;
+  ProfScope ps(c, cyc ? "k_lz_carryR" : "k_lz_carryQ", c.pl.K, nullptr, 1);
+  switch (c.pl.K * 2 + (cyc ? 1 : 0)) {
+    case 7: hipLaunchKernelGGL((k_lz_carry<6, 6, 5, 2, false>), grid, block, 0, c.stream, A); break;
+    case 6: hipLaunchKernelGGL((k_lz_carry<4, 4, 3, 2, true>), grid, block, 0, c.stream, A); break;
+    case 9: hipLaunchKernelGGL((k_lz_carry<7, 7, 4, 2, false>), grid, block, 0, c.stream, A); break;
+    case 8: hipLaunchKernelGGL((k_lz_carry<5, 5, 3, 2, true>), grid, block, 0, c.stream, A); break;
+    case 11: hipLaunchKernelGGL((k_lz_carry<9, 8, 4, 3, false>), grid, block, 0, c.stream, A); break;
+    case 10: hipLaunchKernelGGL((k_lz_carry<6, 6, 3, 3, true>), grid, block, 0, c.stream, A); break;
+    default: return fail(ANNIE_ERR_SIZE, "no carry kernel for this RNS size");
+  }
+  HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+// Buffers of one product: operand x, result y (digit registers; may be the
+// same), m' and its sign, and the work planes.
+struct LzBufs {
+  const uint32_t* x;
+  uint32_t* y;
+  uint32_t *mp, *neg, *wr, *wq, *mq;
+};
+
+static LzBufs lz_bufs(const Ctx& c, const uint32_t* x, uint32_t* y) {
+  return LzBufs{x, y, c.lzreg(LZ_MP), c.lzflags(), c.lzplane(PWR), c.lzplane(PWQ), c.lzplane(PMQ)};
+}
+
+// MMGW product y = a x v: v = x (LZ_SQR), or with LZ_GEN the register whose
+// transforms are in PYR / PYQ (op LZ_MULY) or 1 (LZ_MUL1).  mul: the multiplier
+// of each list position; snap / snapbits: positions whose result also goes to
+// LZ_SNAP.
+static int lz_product(Ctx& c, const LzBufs& B, int mode, int op, const LzMult& mul, const uint32_t* snap = nullptr,
+                      const uint32_t* snapbits = nullptr) {
+  const int KR = c.lz.sh.KR, KQ = c.lz.sh.KQ;
+  int rc;
+  c.staged = false;
+  LzNtt A = lz_args(c);
+  A.x = B.x;
+  A.wr = B.wr;
+  A.wq = B.wq;
+  A.yr = c.lzplane(PYR);
+  A.yq = c.lzplane(PYQ);
+  A.op = op;
+  A.mul = mul;
+  if ((rc = lz_transform(c, A, mode, 0, KR + KQ, KR))) return rc;
+  LzCarry& R = c.lz.cr;
+  R.src = B.wr;
+  R.dst = B.mp;
+  R.neg = B.neg;
+  R.mul = mul;
+  if ((rc = lz_carry(c, R, true))) return rc;
+  A.x = B.mp;
+  A.neg = B.neg;
+  A.wq = B.mq;
+  A.tq = B.wq;
+  if ((rc = lz_transform(c, A, LZ_MULN, KR, KQ, KQ))) return rc;
+  LzCarry& Q = c.lz.cq;
+  Q.src = B.mq;
+  Q.dst = B.y;
+  Q.dst2 = (snap != nullptr || snapbits != nullptr) ? c.lzreg(LZ_SNAP) : nullptr;
+  Q.snap = snap;
+  Q.mul.a = 1u;
+  Q.mul.bits_mode = snapbits != nullptr ? 2 : 0;
+  if (snapbits != nullptr) std::memcpy(Q.mul.bits, snapbits, sizeof(Q.mul.bits));
+  return lz_carry(c, Q, false);
+}
+
+static LzMult lz_by(uint32_t a) {
+  LzMult m{};
+  m.a = a;
+  return m;
+}
+
+// Transforms of the register y for a later product: PYR / PYQ.
+static int lz_operand(Ctx& c, const uint32_t* y) {
+  LzNtt A = lz_args(c);
+  A.x = y;
+  A.wr = c.lzplane(PYR);
+  A.wq = c.lzplane(PYQ);
+  A.op = LZ_FWD;
+  return lz_transform(c, A, LZ_GEN, 0, c.lz.sh.KR + c.lz.sh.KQ, 0);
+}
+
+static int lz_mul(Ctx& c, int dst, int src) {
+  int rc;
+  if (c.slot_ids == nullptr) c.lz.is_one[dst] = false;
+  if ((rc = lz_operand(c, c.lzreg(src)))) return rc;
+  return lz_product(c, lz_bufs(c, c.lzreg(dst), c.lzreg(dst)), LZ_GEN, LZ_MULY, lz_by(1u));
+}
+
+static int lz_copy(Ctx& c, int dst, int src) {
+  if (dst == src) return ANNIE_OK;
+  const size_t len = size_t(c.lz.sh.DL) * c.n;
+  if (c.slot_ids == nullptr) {
+    c.lz.is_one[dst] = src == LZ_ONE || (src < 3 && c.lz.is_one[src]);
+    HIPCHK(hipMemcpyAsync(c.lzreg(dst), c.lzreg(src), len * 4, hipMemcpyDeviceToDevice, c.stream));
+    return ANNIE_OK;
+  }
+  const unsigned blocks = unsigned(std::min<size_t>((len / 4 + 255) / 256, 64));
+  hipLaunchKernelGGL(k_copy_slots, dim3(blocks, c.nslots), dim3(256), 0, c.stream, c.lz.mem, size_t(dst) * len,
+                     size_t(src) * len, len, c.slot_ids, c.lz.stride);
+  HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+template <class F>
+static int lz_convert(Ctx& c, F kernel, int halo, const uint32_t* src, uint32_t* dst, const uint32_t* neg, int cbits) {
+  LzConv A{src, dst, neg, c.pl.LN, cbits};
+  const size_t waves = (c.n + size_t(63 - halo)) / size_t(64 - halo);
+  hipLaunchKernelGGL(kernel, dim3(unsigned((waves + 3) / 4)), dim3(256), 0, c.stream, A);
+  HIPCHK(hipGetLastError());
+  return ANNIE_OK;
+}
+
+// Digits -> the external register format (K residue planes), and back.  neg:
+// the register is m' with this sign (see k_lz_export).
+static int lz_export(Ctx& c, const uint32_t* digits, uint32_t* dst, int cbits, const uint32_t* neg = nullptr) {
+  switch (c.pl.K) {
+    case 3: return lz_convert(c, k_lz_export<3, 2>, 3, digits, dst, neg, cbits);
+    case 4: return lz_convert(c, k_lz_export<4, 2>, 3, digits, dst, neg, cbits);
+    default: return lz_convert(c, k_lz_export<5, 3>, 3, digits, dst, neg, cbits);
+  }
+}
+
+static int lz_import(Ctx& c, const uint32_t* src, uint32_t* digits, int cbits) {
+  switch (c.pl.K) {
+    case 3: return lz_convert(c, k_lz_import<3, 2>, 3, src, digits, nullptr, cbits);
+    case 4: return lz_convert(c, k_lz_import<4, 2>, 3, src, digits, nullptr, cbits);
+    default: return lz_convert(c, k_lz_import<5, 3>, 3, src, digits, nullptr, cbits);
+  }
+}
+
+// Balanced digits of x >= 0 in the register format; `wrap`: a carry out of the
+// top enters digit 0 (x mod B^n - 1).
+static void mpz_to_lz_digits(const Ctx& c, const mpz_t x, int cb, bool wrap, std::vector<uint32_t>& out) {
+  const size_t n = c.n;
+  const int DL = c.lz.sh.DL;
+  std::vector<uint32_t> pl;
+  mpz_to_digit_planes(c, x, cb, pl);
+  out.assign(size_t(DL) * n, 0);
+  const __int128 B = __int128(1) << cb, half = B >> 1;
+  int carry = 0;
+  auto put = [&](size_t i, __int128 v) {
+    out[2 * i] = uint32_t(v);
+    out[2 * i + 1] = uint32_t(v >> 32);
+    if (DL == 3) out[2 * n + i] = uint32_t(v >> 64);
+  };
+  auto digit = [&](size_t i) {
+    return __int128((unsigned __int128)pl[i] | ((unsigned __int128)pl[n + i] << 32) | ((unsigned __int128)pl[2 * n + i] << 64));
+  };
+  __int128 first = 0;
+  for (size_t i = 0; i < n; ++i) {
+    __int128 v = digit(i) + carry;
+    carry = v >= half ? 1 : 0;
+    if (carry) v -= B;
+    if (i == 0) first = v;
+    put(i, v);
+  }
+  if (wrap && carry) put(0, first + 1);
+}
+
+static int lz_upload(Ctx& c, uint32_t* dst, const mpz_t x, int cb, bool wrap) {
+  std::vector<uint32_t> h;
+  mpz_to_lz_digits(c, x, cb, wrap, h);
+  HIPCHK(hipMemcpyAsync(dst, h.data(), h.size() * 4, hipMemcpyHostToDevice, c.stream));
+  HIPCHK(hipStreamSynchronize(c.stream));
+  return ANNIE_OK;
+}
+
+// External form of user register r (0..2) or of 1 (r = LZ_ONE) into K planes
+// at dst (not PYR).  The constant 1 keeps the non-negative digits of its
+// residue there.
+static int lz_external(Ctx& c, int r, uint32_t* dst);
+
 // get() for every slot of the current list (slot 0 without a list): T_Q = src
 // as raw digits (a carry pass over its own residues), T_R = src, reduce to
 // raw digits, read back, digits -> integer mod N.  mods[i] is the modulus of
 // list position i; zs[i] receives the value.
 static int get_values(Ctx& c, int src, const size_t* slots, const mpz_t* const* mods, mpz_t* const* zs, size_t count) {
   int rc;
+  if (c.lz.on) return lz_get_values(c, src, slots, mods, zs, count);
   const CarryJob cj = cjob(c.reg(src), c.tq(), 1u, 1, 0, 1);
   if ((rc = launch_carry(c, &cj, 1))) return rc;
   if ((rc = copy_reg(c, RTR, src))) return rc;
@@ -654,8 +1124,14 @@ static int get_values(Ctx& c, int src, const size_t* slots, const mpz_t* const* 
                           c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
   for (size_t i = 0; i < count; ++i) {
-    const std::vector<uint32_t> di(d.begin() + i * w, d.begin() + (i + 1) * w);
-    digits_to_mpz(c, di, slot_cbits(c, slots[i]), *zs[i]);
+    const uint32_t* di = d.data() + i * w;
+    // DIGIT_LIMBS planes of two's complement limbs: sign-extend the 96 bits.
+    auto at = [&](size_t j) {
+      const unsigned __int128 u =
+          (unsigned __int128)di[j] | ((unsigned __int128)di[c.n + j] << 32) | ((unsigned __int128)di[2 * c.n + j] << 64);
+      return (__int128)(u << 32) >> 32;
+    };
+    digits_to_mpz(c, at, slot_cbits(c, slots[i]), *zs[i]);
     mpz_mod(*zs[i], *zs[i], *mods[i]);
   }
   return ANNIE_OK;
@@ -705,6 +1181,8 @@ static void destroy(annie_hip_t* h) {
   if (c.ev_join) (void)hipEventDestroy(c.ev_join);
   if (c.mem) (void)hipFree(c.mem);
   if (c.tw) (void)hipFree(c.tw);
+  if (c.lz.mem) (void)hipFree(c.lz.mem);
+  if (c.lz.tw) (void)hipFree(c.lz.tw);
   for (auto& g : c.graphs) (void)hipGraphExecDestroy(g.exec);
   if (c.graph_buf) (void)hipFree(c.graph_buf);
   if (c.cbits_dev) (void)hipFree(c.cbits_dev);
@@ -729,9 +1207,45 @@ static void plan_R(int cbits, int LN, mpz_t R) {
 
 static void plan_R(const Plan& pl, mpz_t R) { plan_R(pl.cbits(), pl.LN, R); }
 
-// Device state shared by the slots of a context: stream, register file of
-// `slots` slots, twiddle tables, kernel constants.
-static int setup_device(Ctx& c, int device, size_t slots) {
+// The long-prime part of a context: register file, roots, kernel constants.
+static int setup_long(Ctx& c) {
+  if (c.long_ready) return ANNIE_OK;
+  const size_t K = size_t(c.pl.K), n = c.n, slots = c.nslots_alloc;
+  c.slot_stride = size_t(NREG) * K * n + 2 * size_t(DIGIT_LIMBS) * n;
+  if (hipMalloc(&c.mem, slots * c.slot_stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
+  c.regs = c.mem;
+  c.raw = c.mem + size_t(NREG) * K * n;
+  if (hipMalloc(&c.tw, 4 * K * n * sizeof(TwDev)) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "twiddles");
+  HIPCHK(hipMemsetAsync(c.mem, 0, slots * c.slot_stride * 4, c.stream));
+
+  c.pc = make_consts(c.pl);
+  for (int k = 0; k < KMAX; ++k) {
+    c.nbase.p[k] = c.pc.p[k];
+    c.nbase.q[k] = c.pc.q[k];
+    c.nbase.sc[k] = c.pc.sq_scale[k];
+    c.nbase.scq[k] = c.pc.sq_scale_q[k];
+  }
+  c.nbase.njobs = c.cbase.njobs = 1;
+
+  std::vector<TwDev> host(4 * K * n);
+  for (size_t k = 0; k < K; ++k) {
+    const PrimeTables pt = make_tables(c.pl.LN, int(k));
+    for (size_t i = 0; i < n; ++i) {
+      host[(0 * K + k) * n + i] = pt.fwdR[i].w;
+      host[(1 * K + k) * n + i] = pt.invR[i].w;
+      host[(2 * K + k) * n + i] = pt.fwdQ[i].w;
+      host[(3 * K + k) * n + i] = pt.invQ[i].w;
+    }
+  }
+  HIPCHK(hipMemcpyAsync(c.tw, host.data(), host.size() * sizeof(TwDev), hipMemcpyHostToDevice, c.stream));
+  HIPCHK(hipStreamSynchronize(c.stream));
+  c.long_ready = true;
+  return ANNIE_OK;
+}
+
+// Device state shared by the slots of a context: stream, and the register
+// files, roots and kernel constants of `slots` slots of the path it takes.
+static int setup_device(Ctx& c, int device, size_t slots, bool want_lazy) {
   c.n = c.pl.n();
   c.m1 = (c.pl.LN <= 13) ? 0 : c.pl.LN / 2;
   c.m2 = c.pl.LN - c.m1;
@@ -754,46 +1268,17 @@ static int setup_device(Ctx& c, int device, size_t slots) {
     HIPCHK(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
   }
-  const size_t K = size_t(c.pl.K), n = c.n;
   c.nslots_alloc = slots;
-  c.slot_stride = size_t(NREG) * K * n + 2 * size_t(DIGIT_LIMBS) * n;
-  if (hipMalloc(&c.mem, slots * c.slot_stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
-  c.regs = c.mem;
-  c.raw = c.mem + size_t(NREG) * K * n;
-  if (hipMalloc(&c.tw, 4 * K * n * sizeof(TwDev)) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "twiddles");
-  HIPCHK(hipMemsetAsync(c.mem, 0, slots * c.slot_stride * 4, c.stream));
-
-  c.pc = make_consts(c.pl);
-  for (int k = 0; k < KMAX; ++k) {
-    c.nbase.p[k] = c.pc.p[k];
-    c.nbase.q[k] = c.pc.q[k];
-    c.nbase.sc[k] = c.pc.sq_scale[k];
-    c.nbase.scq[k] = c.pc.sq_scale_q[k];
-  }
   c.nbase.LN = c.cbase.LN = c.pl.LN;
   c.cbase.cbits = c.pl.cbits();
-  c.nbase.njobs = c.cbase.njobs = 1;
-
-  std::vector<TwDev> host(4 * K * n);
-  for (size_t k = 0; k < K; ++k) {
-    const PrimeTables pt = make_tables(c.pl.LN, int(k));
-    for (size_t i = 0; i < n; ++i) {
-      host[(0 * K + k) * n + i] = pt.fwdR[i].w;
-      host[(1 * K + k) * n + i] = pt.invR[i].w;
-      host[(2 * K + k) * n + i] = pt.fwdQ[i].w;
-      host[(3 * K + k) * n + i] = pt.invQ[i].w;
-    }
-  }
-  HIPCHK(hipMemcpyAsync(c.tw, host.data(), host.size() * sizeof(TwDev), hipMemcpyHostToDevice, c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
-  return ANNIE_OK;
+  return (want_lazy && lz_class_fits(c.pl)) ? lz_setup(c) : setup_long(c);
 }
 
 // Per-modulus constants of one slot: N_Q, the negacyclic transform of N, and
 // Ninv_R, the cyclic transform of N^-1 mod R (src/transformGPU.h:737-741),
 // both scaled by n^-1 2^32 for the pointwise step, and the MMGW form of 1,
 // R/2 mod N (src/transformGPU.h:743-747).  Ninv is N^-1 mod R.
-static int load_slot_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv) {
+static int load_long_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv) {
   int rc;
   const uint32_t* prev_ids = c.slot_ids;
   const int prev_n = c.nslots;
@@ -830,6 +1315,174 @@ static int load_slot_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv
   return done(ANNIE_OK);
 }
 
+// R / 2 mod N (+ N when odd), the MMGW form of 1 (src/transformGPU.h:743-747).
+static void mmgw_one(const Ctx& c, int cb, const mpz_t N, mpz_t t) {
+  Mpz R;
+  plan_R(cb, c.pl.LN, R.v);
+  mpz_mod(t, R.v, N);
+  if (mpz_odd_p(t)) mpz_add(t, t, N);
+  mpz_fdiv_q_2exp(t, t, 1);
+}
+
+static const mpz_t& modulus(const Ctx& c, size_t slot) { return c.slotN.empty() ? c.N : c.slotN[slot]->v; }
+
+// The constants of one slot on the short-prime path: the transforms of N^-1
+// mod R and N with the scales of the pointwise steps, and 1.  Balanced digits,
+// so that the coefficient bounds of lz_fits hold.
+static int lz_load_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv) {
+  Lazy& z = c.lz;
+  const uint32_t* prev_ids = c.slot_ids;
+  const int prev_n = c.nslots;
+  c.slot_ids = nullptr;  // the passes below address the slot directly
+  c.nslots = 1;
+  const size_t off = slot * z.stride;
+  const int cb = slot_cbits(c, slot);
+  int rc = lz_upload(c, c.lzreg(LZ_GET) + off, N, cb, false);
+  LzNtt A = lz_args(c);
+  A.x = c.lzreg(LZ_GET) + off;
+  A.wr = c.lzplane(PNIR) + off;
+  A.wq = c.lzplane(PNQ) + off;
+  A.op = LZ_FWD;
+  if (rc == ANNIE_OK) {
+    std::memcpy(A.scale, z.scaleQ, sizeof(A.scale));
+    rc = lz_transform(c, A, LZ_GEN, z.sh.KR, z.sh.KQ, 0);
+  }
+  if (rc == ANNIE_OK) rc = lz_upload(c, c.lzreg(LZ_GET) + off, Ninv, cb, true);
+  if (rc == ANNIE_OK) {
+    std::memcpy(A.scale, z.scaleR, sizeof(A.scale));
+    rc = lz_transform(c, A, LZ_GEN, 0, z.sh.KR, 0);
+  }
+  Mpz t;
+  mmgw_one(c, cb, N, t.v);
+  if (rc == ANNIE_OK) rc = lz_upload(c, c.lzreg(LZ_ONE) + off, t.v, cb, false);
+  c.slot_ids = prev_ids;
+  c.nslots = prev_n;
+  return rc;
+}
+
+static int lz_external(Ctx& c, int r, uint32_t* dst) {
+  const int cb = slot_cbits(c, 0);
+  if (r != LZ_ONE && !c.lz.is_one[r]) return lz_export(c, c.lzreg(r), dst, cb);
+  if (!c.slotN.empty() && !c.slotN[0]) return lz_export(c, c.lzreg(r), dst, cb);
+  Mpz t;
+  mmgw_one(c, cb, modulus(c, 0), t.v);
+  std::vector<uint32_t> h;
+  mpz_to_digit_planes(c, t.v, cb, h);
+  uint32_t* digits = c.lzplane(PYR);  // 3 n words
+  HIPCHK(hipMemcpyAsync(digits, h.data(), h.size() * 4, hipMemcpyHostToDevice, c.stream));
+  if (int rc = encode_digits(c, digits, dst)) return rc;
+  HIPCHK(hipStreamSynchronize(c.stream));
+  return ANNIE_OK;
+}
+
+// The long-prime file of a short-prime context (slot 0 only unless `all`):
+// set up, its constants loaded.
+static int ensure_long(Ctx& c, bool all) {
+  int rc;
+  const bool had = c.long_ready;
+  if ((rc = setup_long(c))) return rc;
+  if (had && !all) return ANNIE_OK;
+  Mpz R, t;
+  for (size_t s = 0; s < (all ? c.nslots_alloc : 1); ++s) {
+    if (!c.slotN.empty() && !c.slotN[s]) continue;
+    plan_R(slot_cbits(c, s), c.pl.LN, R.v);
+    if (mpz_invert(t.v, modulus(c, s), R.v) == 0) return fail(ANNIE_ERR, "modulus not invertible");
+    if ((rc = load_long_consts(c, s, modulus(c, s), t.v))) return rc;
+  }
+  return ANNIE_OK;
+}
+
+// Moves a context to the long primes for good: a multiplier or a slot's digit
+// width is outside what the short-prime carries take.
+static int lz_demote(Ctx& c) {
+  int rc;
+  if ((rc = ensure_long(c, true))) return rc;
+  for (auto& g : c.graphs) (void)hipGraphExecDestroy(g.exec);
+  c.graphs.clear();
+  for (size_t s = 0; s < c.nslots_alloc; ++s) {
+    if (!c.slotN.empty() && !c.slotN[s]) continue;
+    const int cb = slot_cbits(c, s);
+    const size_t off = s * c.lz.stride, to = s * c.slot_stride;
+    for (int r = 0; r < 3; ++r) {
+      rc = c.slotN.empty() ? lz_external(c, r, c.reg(r)) : lz_export(c, c.lzreg(r) + off, c.reg(r) + to, cb);
+      if (rc) return rc;
+    }
+    if ((rc = lz_export(c, c.lzreg(LZ_SNAP) + off, c.reg(RSNAP) + to, cb))) return rc;
+  }
+  HIPCHK(hipStreamSynchronize(c.stream));
+  c.lz.on = false;
+  (void)hipFree(c.lz.mem);
+  (void)hipFree(c.lz.tw);
+  c.lz.mem = c.lz.tw = nullptr;
+  return ANNIE_OK;
+}
+
+// Whether a multiplier fits the carries and CRT ranges of every slot.
+static bool lz_takes(const Ctx& c, uint32_t a) {
+  if (a == 1u) return true;
+  if (a > LZ_MAX_A) return false;
+  if (c.slot_cb.empty()) return lz_fits(c.pl, c.pl.cbits(), a, c.lz.primes);
+  int cb = 0;
+  for (size_t s = 0; s < c.slot_cb.size(); ++s)
+    if (c.slotN[s]) cb = std::max(cb, c.slot_cb[s]);
+  return lz_fits(c.pl, cb, a, c.lz.primes);
+}
+
+static int lz_square(Ctx& c, uint32_t a, const uint32_t* a_slot, bool bits) {
+  if (a_slot == nullptr && !bits) {
+    if (a != 1u && a != c.lz.last_a) {
+      if (!lz_takes(c, a)) {
+        const int rc = lz_demote(c);
+        return rc ? rc : square_mul(c, a);
+      }
+      c.lz.last_a = a;
+    }
+    c.lz.is_one[0] = false;
+  }
+  LzMult m = lz_by(a);
+  const LzBufs B = lz_bufs(c, c.lzreg(LX0), c.lzreg(LX0));
+  if (a_slot != nullptr) {
+    m.a_slot = a_slot;
+    return lz_product(c, B, LZ_SQR, 0, m, a_slot);
+  }
+  if (bits) {
+    m.bits_mode = 1;
+    m.slot_base = c.base_dev;
+    std::memcpy(m.bits, c.mulbits, sizeof(m.bits));
+    return lz_product(c, B, LZ_SQR, 0, m, nullptr, c.snapbits);
+  }
+  return lz_product(c, B, LZ_SQR, 0, m);
+}
+
+// get() on the short-prime path: the product by 1, read back as digits.
+static int lz_get_values(Ctx& c, int src, const size_t* slots, const mpz_t* const* mods, mpz_t* const* zs, size_t count) {
+  int rc;
+  if ((rc = lz_product(c, lz_bufs(c, c.lzreg(src), c.lzreg(LZ_GET)), LZ_GEN, LZ_MUL1, lz_by(1u)))) return rc;
+  const int DL = c.lz.sh.DL;
+  const size_t w = size_t(DL) * c.n;
+  std::vector<uint32_t> d(w * count);
+  for (size_t i = 0; i < count; ++i)
+    HIPCHK(hipMemcpyAsync(d.data() + i * w, c.lzreg(LZ_GET) + slots[i] * c.lz.stride, w * 4, hipMemcpyDeviceToHost,
+                          c.stream));
+  HIPCHK(hipStreamSynchronize(c.stream));
+  for (size_t i = 0; i < count; ++i) {
+    const uint32_t* di = d.data() + i * w;
+    auto at = [&](size_t j) {
+      const uint64_t lo = uint64_t(di[2 * j]) | (uint64_t(di[2 * j + 1]) << 32);
+      if (DL == 2) return __int128(int64_t(lo));
+      return __int128((unsigned __int128)lo | ((unsigned __int128)(__int128)int32_t(di[2 * c.n + j]) << 64));
+    };
+    digits_to_mpz(c, at, slot_cbits(c, slots[i]), *zs[i]);
+    mpz_mod(*zs[i], *zs[i], *mods[i]);
+  }
+  return ANNIE_OK;
+}
+
+static int load_slot_consts(Ctx& c, size_t slot, const mpz_t N, const mpz_t Ninv) {
+  if (c.lz.on) return lz_load_consts(c, slot, N, Ninv);
+  return load_long_consts(c, slot, N, Ninv);
+}
+
 static int create(const uint64_t* Nl, size_t nl, int32_t a, int device, int min_ln, annie_hip_t** out) {
   if (!out || !Nl || nl == 0) return fail(ANNIE_ERR_ARG, "null argument");
   *out = nullptr;
@@ -860,7 +1513,7 @@ static int create(const uint64_t* Nl, size_t nl, int32_t a, int device, int min_
     return ANNIE_INIT_FAILED;
   }
   int rc;
-  if ((rc = setup_device(c, device, 1))) return rc;
+  if ((rc = setup_device(c, device, 1, lz_fits(c.pl, c.pl.cbits(), uint32_t(a), lz_primes(c.pl.LN, LZ_MAXP))))) return rc;
   if ((rc = load_slot_consts(c, 0, c.N, t))) return rc;
   *out = h.release();
   return ANNIE_OK;
@@ -935,7 +1588,10 @@ static bool ready(const annie_hip_t* h) {
 // `scratch` only names the symbol; its device address on each GPU comes from
 // hipGetSymbolAddress, looked up once per device with that device current.
 constexpr size_t NOALLOC_KN_MAX = ANNIE_HIP_NOALLOC_MAX_KN;
-constexpr size_t SCRATCH_WORDS = 4 * NOALLOC_KN_MAX + size_t(DIGIT_LIMBS) * (NOALLOC_KN_MAX / 2);
+// Short primes: three digit registers, a block of flags and the work planes
+// (23 n words at K = 4, the largest: n <= 2^17 there, 2^16 at K = 5).
+constexpr size_t SCRATCH_WORDS = 23 * (NOALLOC_KN_MAX / 4) + LZ_FLAGS;
+static_assert(SCRATCH_WORDS >= 4 * NOALLOC_KN_MAX + size_t(DIGIT_LIMBS) * (NOALLOC_KN_MAX / 2), "long-prime work registers");
 static __device__ __align__(256) uint32_t scratch[SCRATCH_WORDS];
 
 constexpr int MAX_DEVICES = 64;
@@ -1059,6 +1715,16 @@ int annie_hip_square_mul_noalloc(annie_hip_t* h, const uint32_t* x, uint32_t* y,
   HIPCHK(hipSetDevice(c.device));
   int rc;
   if ((rc = scratch_on(c.device, &w))) return rc;
+  if (c.lz.on && !lz_takes(c, uint32_t(a)) && (rc = lz_demote(c))) return rc;
+  if (c.lz.on) {
+    const size_t n = c.n, dig = size_t(c.lz.sh.DL) * n, kr = size_t(c.lz.sh.KR) * n, kq = size_t(c.lz.sh.KQ) * n;
+    if (3 * dig + kr + 2 * kq + LZ_FLAGS > SCRATCH_WORDS) return fail(ANNIE_ERR_SIZE, "no-allocation work registers");
+    uint32_t *dx = w, *dy = w + dig, *mp = w + 2 * dig, *wr = w + 3 * dig, *wq = wr + kr, *mq = wq + kq, *neg = mq + kq;
+    if ((rc = lz_import(c, x, dx, c.pl.cbits()))) return rc;
+    const LzBufs B{dx, dy, mp, neg, wr, wq, mq};
+    if ((rc = lz_product(c, B, LZ_SQR, 0, lz_by(uint32_t(a))))) return rc;
+    return lz_export(c, dy, y, c.pl.cbits());
+  }
   const SqBufs B{x, y, w, w + kn, w + 2 * kn, w + 3 * kn, w + 4 * kn};
   // One stream: the two-stream squaring is only used above this size limit.
   hipStream_t aux = c.aux;
@@ -1095,6 +1761,21 @@ int annie_hip_get(annie_hip_t* h, size_t src, uint64_t* limbs, size_t cap, size_
   return rc;
 }
 
+// External form of r0 and r1 on the device.
+static int external_regs(Ctx& c, const uint32_t** r) {
+  if (!c.lz.on) {
+    r[0] = c.reg(R0);
+    r[1] = c.reg(R1);
+    return ANNIE_OK;
+  }
+  // r1 first: the constant 1 goes through PYR.
+  r[0] = c.lzplane(PWR);
+  r[1] = c.lzplane(PWQ);
+  int rc;
+  if ((rc = lz_external(c, LX1, c.lzplane(PWQ)))) return rc;
+  return lz_external(c, LX0, c.lzplane(PWR));
+}
+
 size_t annie_hip_checkpoint_size(const annie_hip_t* h) {
   if (!h) return 0;
   return 8 + 2 * size_t(h->c.pl.K) * h->c.n * 4;
@@ -1107,11 +1788,11 @@ int annie_hip_save_checkpoint(annie_hip_t* h, void* buf, size_t cap) {
   uint32_t* w = static_cast<uint32_t*>(buf);
   w[0] = uint32_t(c.pl.K);
   w[1] = uint32_t(c.n);
+  const uint32_t* r[2];
+  if (const int rc = external_regs(c, r)) return rc;
   for (int k = 0; k < c.pl.K; ++k) {
-    HIPCHK(hipMemcpyAsync(w + 2 + size_t(2 * k) * c.n, c.reg(R0) + size_t(k) * c.n, c.n * 4, hipMemcpyDeviceToHost,
-                          c.stream));
-    HIPCHK(hipMemcpyAsync(w + 2 + size_t(2 * k + 1) * c.n, c.reg(R1) + size_t(k) * c.n, c.n * 4,
-                          hipMemcpyDeviceToHost, c.stream));
+    HIPCHK(hipMemcpyAsync(w + 2 + size_t(2 * k) * c.n, r[0] + size_t(k) * c.n, c.n * 4, hipMemcpyDeviceToHost, c.stream));
+    HIPCHK(hipMemcpyAsync(w + 2 + size_t(2 * k + 1) * c.n, r[1] + size_t(k) * c.n, c.n * 4, hipMemcpyDeviceToHost, c.stream));
   }
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
@@ -1123,11 +1804,17 @@ int annie_hip_load_checkpoint(annie_hip_t* h, const void* buf, size_t size) {
   if (!buf || size < annie_hip_checkpoint_size(h)) return fail(ANNIE_ERR_ARG, "checkpoint too short");
   const uint32_t* w = static_cast<const uint32_t*>(buf);
   if (w[0] != uint32_t(c.pl.K) || w[1] != uint32_t(c.n)) return fail(ANNIE_ERR_ARG, "checkpoint of another transform");
+  uint32_t* r0 = c.lz.on ? c.lzplane(PWR) : c.reg(R0);
+  uint32_t* r1 = c.lz.on ? c.lzplane(PYR) : c.reg(R1);
   for (int k = 0; k < c.pl.K; ++k) {
-    HIPCHK(hipMemcpyAsync(c.reg(R0) + size_t(k) * c.n, w + 2 + size_t(2 * k) * c.n, c.n * 4, hipMemcpyHostToDevice,
-                          c.stream));
-    HIPCHK(hipMemcpyAsync(c.reg(R1) + size_t(k) * c.n, w + 2 + size_t(2 * k + 1) * c.n, c.n * 4,
-                          hipMemcpyHostToDevice, c.stream));
+    HIPCHK(hipMemcpyAsync(r0 + size_t(k) * c.n, w + 2 + size_t(2 * k) * c.n, c.n * 4, hipMemcpyHostToDevice, c.stream));
+    HIPCHK(hipMemcpyAsync(r1 + size_t(k) * c.n, w + 2 + size_t(2 * k + 1) * c.n, c.n * 4, hipMemcpyHostToDevice, c.stream));
+  }
+  if (c.lz.on) {
+    int rc;
+    if ((rc = lz_import(c, r0, c.lzreg(LX0), slot_cbits(c, 0)))) return rc;
+    if ((rc = lz_import(c, r1, c.lzreg(LX1), slot_cbits(c, 0)))) return rc;
+    c.lz.is_one[0] = c.lz.is_one[1] = false;
   }
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
@@ -1189,7 +1876,22 @@ int annie_hip_read_register(annie_hip_t* h, size_t reg, uint32_t* out, size_t ca
   Ctx& c = h->c;
   const size_t words = size_t(c.pl.K) * c.n;
   if (reg >= size_t(NREG) || !out || cap_words < words) return fail(ANNIE_ERR_ARG, "bad register read");
-  HIPCHK(hipMemcpyAsync(out, c.reg(int(reg)), words * 4, hipMemcpyDeviceToHost, c.stream));
+  const uint32_t* src = nullptr;
+  if (c.lz.on) {
+    int rc = ANNIE_OK;
+    src = c.lzplane(PWR);
+    if (reg <= RONE) {
+      rc = lz_external(c, lz_of(int(reg)), c.lzplane(PWR));
+    } else if (reg == RTR && !c.staged) {  // m' + 2 of the last product
+      rc = lz_export(c, c.lzreg(LZ_MP), c.lzplane(PWR), slot_cbits(c, 0), c.lzflags());
+    } else if ((rc = ensure_long(c, false)) == ANNIE_OK) {
+      src = c.reg(int(reg));
+    }
+    if (rc) return rc;
+  } else {
+    src = c.reg(int(reg));
+  }
+  HIPCHK(hipMemcpyAsync(out, src, words * 4, hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
 }
@@ -1198,7 +1900,12 @@ int annie_hip_write_register(annie_hip_t* h, size_t reg, const uint32_t* in, siz
   if (!ready(h)) return ANNIE_ERR_ARG;
   Ctx& c = h->c;
   if (reg > 2 || !in || words != size_t(c.pl.K) * c.n) return fail(ANNIE_ERR_ARG, "bad register write");
-  HIPCHK(hipMemcpyAsync(c.reg(int(reg)), in, words * 4, hipMemcpyHostToDevice, c.stream));
+  uint32_t* dst = c.lz.on ? c.lzplane(PWR) : c.reg(int(reg));
+  HIPCHK(hipMemcpyAsync(dst, in, words * 4, hipMemcpyHostToDevice, c.stream));
+  if (c.lz.on) {
+    if (const int rc = lz_import(c, dst, c.lzreg(int(reg)), slot_cbits(c, 0))) return rc;
+    c.lz.is_one[reg] = false;
+  }
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
 }
@@ -1267,6 +1974,11 @@ int annie_hip_debug_square_stage(annie_hip_t* h, int32_t a, int stage) {
   if (!ready(h)) return ANNIE_ERR_ARG;
   Ctx& c = h->c;
   int rc;
+  if (c.lz.on) {  // the long-prime stages, from the register as it is
+    if ((rc = ensure_long(c, false))) return rc;
+    if ((rc = lz_external(c, LX0, c.reg(R0)))) return rc;
+    c.staged = true;
+  }
   const NttJob j[2] = {job(c.reg(R0), c.reg(RWR), c.fwdR(), c.invR()), job(c.reg(R0), c.reg(RWQ), c.fwdQ(), c.invQ())};
   if ((rc = convolve(c, ROW_SQR, j, 2))) return rc;
   if (stage >= 2) {
@@ -1290,6 +2002,9 @@ int annie_hip_read_tq(annie_hip_t* h, uint32_t* out, size_t cap_words) {
   if (!ready(h)) return ANNIE_ERR_ARG;
   Ctx& c = h->c;
   if (!out || cap_words < size_t(DIGIT_LIMBS) * c.n) return fail(ANNIE_ERR_ARG, "buffer too small");
+  if (c.lz.on) {
+    if (const int rc = ensure_long(c, false)) return rc;
+  }
   HIPCHK(hipMemcpyAsync(out, c.tq(), size_t(DIGIT_LIMBS) * c.n * 4, hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
   return ANNIE_OK;
@@ -1314,7 +2029,7 @@ int annie_hip_batch_create(int K, int pck, int LN, int lbase, size_t slots, int 
   c.pl.LN = LN;
   c.pl.lbase = lbase;
   int rc;
-  if ((rc = setup_device(c, device, slots))) return rc;
+  if ((rc = setup_device(c, device, slots, true))) return rc;
   c.slotN.resize(slots);
   c.slot_cb.assign(slots, c.pl.cbits());
   c.slot_base.assign(slots, 1u);
@@ -1342,8 +2057,16 @@ int annie_hip_batch_bytes(int K, int LN, size_t* per_slot, size_t* fixed) {
   // setup_device's slot stride, the staging ring's two words per slot per
   // entry, the graph buffers' two words per slot and the per-slot width,
   // base and list words.
-  if (per_slot)
-    *per_slot = (size_t(NREG) * size_t(K) * n + 2 * size_t(DIGIT_LIMBS) * n) * 4 + NSTAGE * 2 * 4 + 2 * 4 + 3 * 4;
+  if (per_slot) {
+    // The larger of the two paths' slots; the short primes' root tables beyond
+    // `fixed` count with the slots, of which a batch has at least one.
+    size_t words = size_t(NREG) * size_t(K) * n + 2 * size_t(DIGIT_LIMBS) * n;
+    if (K >= 3 && LN >= 8 && LN <= 20) {
+      const LzShape sh = lz_shape(K);
+      words = std::max(words, lz_slot_words(K, n) + (2 * size_t(sh.KR + sh.KQ) - 4 * size_t(K)) * n);
+    }
+    *per_slot = words * 4 + NSTAGE * 2 * 4 + 2 * 4 + 3 * 4;
+  }
   if (fixed) *fixed = 4 * size_t(K) * n * sizeof(TwDev);
   return ANNIE_OK;
 }
@@ -1374,11 +2097,14 @@ int annie_hip_batch_load(annie_hip_t* h, size_t slot, const uint64_t* N, size_t 
   HIPCHK(hipSetDevice(c.device));
   c.slot_cb[slot] = pl.cbits();
   c.slot_base[slot] = uint32_t(a);
+  c.lz.last_a = 1u;
   const uint32_t cb = uint32_t(pl.cbits()), ab = uint32_t(a);
   HIPCHK(hipMemcpyAsync(c.cbits_dev + slot, &cb, 4, hipMemcpyHostToDevice, c.stream));
   HIPCHK(hipMemcpyAsync(c.base_dev + slot, &ab, 4, hipMemcpyHostToDevice, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
-  const int rc = load_slot_consts(c, slot, m->v, t);
+  int rc = ANNIE_OK;
+  if (c.lz.on && !lz_fits(pl, pl.cbits(), 1u, c.lz.primes)) rc = lz_demote(c);
+  if (rc == ANNIE_OK) rc = load_slot_consts(c, slot, m->v, t);
   mpz_clears(R, t, nullptr);
   if (rc) return rc;
   c.slotN[slot] = std::move(m);
@@ -1455,6 +2181,15 @@ int annie_hip_batch_square_mul(annie_hip_t* h, const uint32_t* slots, const uint
   if ((rc = check_slots(c, slots, count))) return rc;
   for (size_t i = 0; i < count; ++i)
     if ((a[i] & ~SLOT_SNAP) < 1) return fail(ANNIE_ERR_ARG, "multiplier must be in [1, 2^31)");
+  for (size_t i = 0; i < count && c.lz.on; ++i) {
+    const uint32_t m = a[i] & ~SLOT_SNAP;
+    if (m <= c.lz.last_a) continue;
+    if (!lz_takes(c, m)) {
+      if ((rc = lz_demote(c))) return rc;
+    } else {
+      c.lz.last_a = m;
+    }
+  }
   const uint32_t *d, *da;
   if (!c.use_graphs) {
     // Short lists whose multipliers are 1 or the slot's base: the multipliers
@@ -1550,6 +2285,20 @@ int annie_hip_batch_square_run(annie_hip_t* h, const uint32_t* slots, size_t cou
     for (size_t t = 0; t < len; ++t)
       if ((m[t] & SLOT_SNAP) && t + 1 != len) return fail(ANNIE_ERR_ARG, "snapshot before the end of a run");
   }
+  if (c.lz.on) {
+    // One launched squaring per step of the slots that still run: with the
+    // short primes' four or eight launches, faster than one workgroup per slot.
+    std::vector<uint32_t> ids, m;
+    for (size_t t = 0; t < steps; ++t) {
+      ids.clear();
+      m.clear();
+      for (size_t i = 0; i < count; ++i)
+        if (mult[i * steps + t] != 0u) ids.push_back(slots[i]), m.push_back(mult[i * steps + t]);
+      if (ids.empty()) break;
+      if ((rc = annie_hip_batch_square_mul(h, ids.data(), m.data(), ids.size()))) return rc;
+    }
+    return ANNIE_OK;
+  }
   Stage& st = c.run_stage;
   if (!st.dev) {
     st.cap = c.nslots_alloc * (ANNIE_HIP_RUN_MAX_STEPS + 1);
@@ -1597,7 +2346,7 @@ int annie_hip_batch_square_run(annie_hip_t* h, const uint32_t* slots, size_t cou
   const uint32_t S = 1u << c.pl.LN;
   const uint32_t lines = uint32_t(threads) / (S / NTT_R);
   const size_t shm = std::max<size_t>(size_t(lines) * (S + (S >> 5)), size_t(c.pl.K + 1) * (S / CARRY_L)) * 4;
-  ProfScope ps(c, "k_sqr_run<" + std::to_string(c.pl.LN) + "," + std::to_string(c.pl.K) + ">");
+  ProfScope ps(c, "k_sqr_run", c.pl.LN, nullptr, c.pl.K);
   hipLaunchKernelGGL(f, dim3(unsigned(count)), dim3(unsigned(threads)), shm, c.stream, R);
   HIPCHK(hipGetLastError());
   return ANNIE_OK;

@@ -1,0 +1,781 @@
+// gfx950 kernels of the short-prime path (lazy.h): transforms over 28-bit
+// primes on signed, lazily reduced residues, and CRT + carry passes between
+// residues and digit registers.
+//
+// Arithmetic.  A residue is any signed 32-bit word congruent to it.  With p <
+// 2^28.2 a word holds +-6.9 p.  The Montgomery product by a constant |w| <=
+// p / 2, hi(b w) - hi(lo(b w p^-1) p), is at most p / 2 + |b| p / 2^33 <= 0.75 p
+// in magnitude for every word b, so the forward butterfly (a, b) -> (a + t,
+// a - t) takes six instructions and no correction; it grows its values by
+// 0.5-0.75 p per level, and eight levels fit between reductions.  Measured on
+// a register-resident chain (2,048 workgroups of 256): 4.9 issue slots per
+// butterfly against 9.4 with the corrections that primes above 2^31 need.
+// The bounds are tracked at compile time, in units of p / 256 (lz_grow,
+// lz_fwd_red, lz_group_inv), and a reduction (quotient by multiplication,
+// three instructions) is placed where a value could leave its word.
+#include "lazy.h"
+#include "rounds.h"
+
+namespace annie {
+
+constexpr int LZ_LIM = 1766;   // 6.9 p (p < 2^28.2: 2^31 / p > 6.96)
+constexpr int LZ_RED = 264;    // a reduced value: [0, 1.03 p)
+constexpr int LZ_IN = 384;     // a digit's residue as loaded: 1.5 p
+constexpr int LZ_OUT = 410;    // what an inverse round starts from: 1.6 p
+
+// Bound of a +- t for |a|, |b| <= s.
+constexpr int lz_grow(int s) { return s + 129 + s * 37 / 1024; }
+
+// Whether round I of a line of 2^M elements, starting at bound s, has to
+// reduce its elements first; lz_fwd_end: the bound after all rounds.
+constexpr int lz_fwd_walk(int M, int LR, int s, int upto, bool want_red) {
+  for (int i = 0, left = M; left > 0; ++i) {
+    const int rr = left < LR ? left : LR;
+    left -= rr;
+    int e = s;
+    for (int l = 0; l < rr; ++l) e = lz_grow(e);
+    const bool red = e > LZ_LIM;
+    if (red) {
+      e = LZ_RED;
+      for (int l = 0; l < rr; ++l) e = lz_grow(e);
+    }
+    if (want_red && i == upto) return red ? 1 : 0;
+    s = e;
+  }
+  return s;
+}
+constexpr bool lz_fwd_red(int M, int LR, int s, int I) { return lz_fwd_walk(M, LR, s, I, true) != 0; }
+static_assert(lz_fwd_walk(13, 3, LZ_IN, -1, false) <= LZ_LIM && lz_fwd_walk(10, 5, LZ_IN, -1, false) <= LZ_LIM &&
+                  lz_fwd_walk(10, 4, LZ_LIM, -1, false) <= LZ_LIM && lz_fwd_walk(13, 4, LZ_IN, -1, false) <= LZ_LIM,
+              "a forward line leaves its words");
+
+struct LzP {
+  uint32_t p, q, bar;
+};
+
+__device__ __forceinline__ int32_t lz_mulc(int32_t b, int32_t w, uint32_t wq, uint32_t p) {
+  return __mulhi(b, w) - __mulhi(int32_t(uint32_t(b) * wq), int32_t(p));
+}
+__device__ __forceinline__ int32_t lz_mul(int32_t a, int32_t b, const LzP& P) {
+  const uint32_t lo = uint32_t(a) * uint32_t(b);
+  return __mulhi(a, b) - __mulhi(int32_t(lo * P.q), int32_t(P.p));
+}
+// x mod p in [0, 1.03 p): bar = floor(2^58 / p).
+__device__ __forceinline__ int32_t lz_red(int32_t x, const LzP& P) {
+  return x - int32_t(uint32_t(__mulhi(x, int32_t(P.bar)) >> 26) * P.p);
+}
+
+template <int LR, int RR>
+__device__ __forceinline__ void lz_round_fwd(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P) {
+#pragma unroll
+  for (int s = 0; s < RoundTw<LR, RR>::G; ++s)
+#pragma unroll
+    for (int e = 0; e < RR; ++e) {
+      const int half = (1 << RR) >> (e + 1);
+#pragma unroll
+      for (int blk = 0; blk < (1 << e); ++blk) {
+        const uint32_t r = T.w[s * RoundTw<LR, RR>::W + (1 << e) - 1 + blk], rq = r * P.q;
+#pragma unroll
+        for (int jj = 0; jj < half; ++jj) {
+          uint32_t& a = x[s * (1 << RR) + blk * 2 * half + jj];
+          uint32_t& b = x[s * (1 << RR) + blk * 2 * half + jj + half];
+          const uint32_t t = uint32_t(lz_mulc(int32_t(b), int32_t(r), rq, P.p));
+          b = a - t;
+          a = a + t;
+        }
+      }
+    }
+}
+
+// Inverse levels of a round; the elements start within LZ_OUT, and end there
+// too unless LAST (then within LZ_LIM).  bd: the bound of each element, a
+// compile-time constant after unrolling.
+template <int LR, int RR, bool LAST>
+__device__ __forceinline__ void lz_round_inv(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P) {
+#pragma unroll
+  for (int s = 0; s < RoundTw<LR, RR>::G; ++s) {
+    int bd[1 << RR];
+#pragma unroll
+    for (int j = 0; j < (1 << RR); ++j) bd[j] = LZ_OUT;
+    uint32_t* v = &x[s * (1 << RR)];
+#pragma unroll
+    for (int e = RR - 1; e >= 0; --e) {
+      const int half = (1 << RR) >> (e + 1);
+#pragma unroll
+      for (int blk = 0; blk < (1 << e); ++blk) {
+        const uint32_t r = T.w[s * RoundTw<LR, RR>::W + (1 << e) - 1 + blk], rq = r * P.q;
+#pragma unroll
+        for (int jj = 0; jj < half; ++jj) {
+          const int j = blk * 2 * half + jj, i = j + half;
+          if (bd[j] + bd[i] > LZ_LIM) {
+            if (bd[j] > LZ_RED) v[j] = uint32_t(lz_red(int32_t(v[j]), P)), bd[j] = LZ_RED;
+            if (bd[i] > LZ_RED) v[i] = uint32_t(lz_red(int32_t(v[i]), P)), bd[i] = LZ_RED;
+          }
+          const uint32_t d = v[j] - v[i];
+          v[j] = v[j] + v[i];
+          v[i] = uint32_t(lz_mulc(int32_t(d), int32_t(r), rq, P.p));
+          const int sum = bd[j] + bd[i];
+          bd[j] = sum;
+          bd[i] = 130 + sum * 37 / 1024;
+        }
+      }
+    }
+    if constexpr (!LAST) {
+#pragma unroll
+      for (int j = 0; j < (1 << RR); ++j)
+        if (bd[j] > LZ_OUT) v[j] = uint32_t(lz_red(int32_t(v[j]), P));
+    }
+  }
+}
+
+// The roots of all rounds of a line, loaded before its first element arrives
+// (lines of eight elements per thread: at most 32 words each way).
+template <int M, int LR, int I>
+struct LzRoots {
+  SchedTw<M, LR, I> t;
+  LzRoots<M, LR, I + 1> next;
+  __device__ __forceinline__ void load(uint32_t tg, uint32_t lineRoot, const uint32_t* tw) {
+    round_tw(t, M, LR * I, tg, lineRoot, tw);
+    if constexpr (I + 1 < Sched<M, LR>::NR) next.load(tg, lineRoot, tw);
+  }
+  template <int J>
+  __device__ __forceinline__ const SchedTw<M, LR, J>& get() const {
+    if constexpr (J == I) return t;
+    else return next.template get<J>();
+  }
+};
+template <int M, int LR>
+struct LzRoots<M, LR, (M + LR - 1) / LR> {};
+
+// Forward rounds I.. .  ROOTS: 0 each round loads its own roots (from LDS), 1
+// one round ahead (`cur` holds round I's), 2 all loaded (`all`).
+template <int M, int LR, int I, int ROOTS, int S0, class GLd, class LLd, class LSt, class Hook>
+__device__ __forceinline__ void lz_fwd(uint32_t (&x)[1 << LR], uint32_t tg, uint32_t lineRoot, const uint32_t* tw,
+                                       const LzP& P, GLd& gld, LLd& lld, LSt& lst, const SchedTw<M, LR, I>& cur,
+                                       const LzRoots<M, LR, 0>& all, Hook&& at_last) {
+  constexpr int RR = Sched<M, LR>::template rr<I>();
+  constexpr bool END = I + 1 == Sched<M, LR>::NR;
+  SchedTw<M, LR, I> own;
+  if constexpr (ROOTS == 0) round_tw(own, M, LR * I, tg, lineRoot, tw);
+  SchedTw<M, LR, END ? I : I + 1> nxt;
+  if constexpr (ROOTS == 1 && !END) round_tw(nxt, M, LR * (I + 1), tg, lineRoot, tw);
+  if constexpr (END) at_last();
+  if constexpr (I > 0) round_load<LR, RR>(x, M, LR * I, tg, lld);
+  if constexpr (lz_fwd_red(M, LR, S0, I)) {
+#pragma unroll
+    for (int i = 0; i < (1 << LR); ++i) x[i] = uint32_t(lz_red(int32_t(x[i]), P));
+  }
+  if constexpr (ROOTS == 0) lz_round_fwd<LR, RR>(x, own, P);
+  else if constexpr (ROOTS == 1) lz_round_fwd<LR, RR>(x, cur, P);
+  else lz_round_fwd<LR, RR>(x, all.template get<I>(), P);
+  if constexpr (!END) {
+    round_store<LR, RR>(x, M, LR * I, tg, lst);
+    __syncthreads();
+    lz_fwd<M, LR, I + 1, ROOTS, S0>(x, tg, lineRoot, tw, P, gld, lld, lst, nxt, all, at_last);
+  }
+}
+
+// Inverse rounds I down to 0, from the elements of round NR - 1 in x.  FINAL:
+// the values go to a carry, which takes any word.
+template <int M, int LR, int I, int ROOTS, bool FINAL, class GSt, class LLd, class LSt>
+__device__ __forceinline__ void lz_inv(uint32_t (&x)[1 << LR], uint32_t tg, uint32_t lineRoot, const uint32_t* tw,
+                                       const LzP& P, GSt& gst, LLd& lld, LSt& lst, const SchedTw<M, LR, I>& cur,
+                                       const LzRoots<M, LR, 0>& all) {
+  constexpr int RR = Sched<M, LR>::template rr<I>();
+  SchedTw<M, LR, I> own;
+  if constexpr (ROOTS == 0) round_tw(own, M, LR * I, tg, lineRoot, tw);
+  SchedTw<M, LR, I == 0 ? 0 : I - 1> nxt;
+  if constexpr (ROOTS == 1 && I > 0) round_tw(nxt, M, LR * (I - 1), tg, lineRoot, tw);
+  if constexpr (I + 1 < Sched<M, LR>::NR) round_load<LR, RR>(x, M, LR * I, tg, lld);
+  constexpr bool LAST = I == 0 && FINAL;
+  if constexpr (ROOTS == 0) lz_round_inv<LR, RR, LAST>(x, own, P);
+  else if constexpr (ROOTS == 1) lz_round_inv<LR, RR, LAST>(x, cur, P);
+  else lz_round_inv<LR, RR, LAST>(x, all.template get<I>(), P);
+  if constexpr (I > 0) {
+    round_store<LR, RR>(x, M, LR * I, tg, lst);
+    __syncthreads();
+    lz_inv<M, LR, I - 1, ROOTS, FINAL>(x, tg, lineRoot, tw, P, gst, lld, lst, nxt, all);
+  } else {
+    round_store<LR, RR>(x, M, 0, tg, gst);
+  }
+}
+
+// Residue of digit i of a register times b = 2^{-32 (DL - 1)}: one Montgomery
+// reduction per limb below the top one.  A digit has at most 59 (DL = 2) or
+// 76 bits, so the result is within 1.5 p.
+template <int DL>
+__device__ __forceinline__ int32_t lz_digit(const uint32_t* x, size_t n, uint32_t i, const LzP& P) {
+  const uint2 d = reinterpret_cast<const uint2*>(x)[i];
+  const uint32_t g = __umulhi(d.x * P.q, P.p);
+  if constexpr (DL == 2) return int32_t(d.y - g);
+  const uint32_t h = x[2 * n + i];
+  uint32_t lo;
+  const bool br = __builtin_sub_overflow(d.y, g, &lo);
+  return int32_t(h - (br ? 1u : 0u) - __umulhi(lo * P.q, P.p));
+}
+
+__device__ __forceinline__ uint32_t lz_slot(const uint32_t* ids, uint32_t pos) { return ids ? ids[pos] : 0u; }
+
+__device__ __forceinline__ uint32_t lz_multiplier(const LzMult& m, uint32_t pos, uint32_t slot) {
+  if (m.a_slot != nullptr) return m.a_slot[pos] & ~SLOT_SNAP;
+  if (m.bits_mode == 1) return ((m.bits[pos >> 5] >> (pos & 31u)) & 1u) ? m.slot_base[slot] : 1u;
+  return m.a;
+}
+
+// Lines of fewer than 64 threads run several to a block, up to 1,024 threads.
+constexpr int lz_row_threads(int M, int LR) { return (1 << M >> LR) > 512 || (1 << M >> LR) < 64 ? 1024 : 512; }
+
+// Row pass (the whole transform of lengths up to 2^13, SRC = limbs of a digit;
+// the levels from m1 on of longer ones, SRC = 0: planes in place).  What stays
+// between transforms (y^, n^, N^, t^) is kept in the order in which the
+// threads hold it, element e of thread tg at e T + tg, so that its loads and
+// stores are consecutive.
+// Grid: (rows / lines, planes, slots); block: lines of 2^M / 2^LR threads.
+template <int M, int LR, int MODE, int SRC>
+__global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A) {
+  extern __shared__ uint32_t lds[];
+  constexpr uint32_t S = 1u << M, T = S >> LR;
+  constexpr int NR = Sched<M, LR>::NR, RL = Sched<M, LR>::template rr<NR - 1>();
+  constexpr int ROOTS = LR <= 3 ? 2 : 1;
+  constexpr int S0 = SRC ? LZ_IN : LZ_LIM;
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.z);
+  const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
+  const int pl = A.pl0 + int(blockIdx.y);
+  const bool cyc = MODE != LZ_MULN && pl < A.KR;
+  const int k = cyc ? pl : pl - A.KR;
+  const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
+  constexpr bool ONE = T >= 64;
+  const uint32_t line = ONE ? 0u : threadIdx.x / T, tg = ONE ? threadIdx.x : threadIdx.x % T;
+  const uint32_t row = SRC ? 0u : (ONE ? blockIdx.x : blockIdx.x * uint32_t(A.cols) + line);
+  const uint32_t lineRoot = SRC ? 1u : (1u << A.m1) + row;
+  const size_t base = so + size_t(k) * n + size_t(row) * S;
+  uint32_t* X = lds + line * (S + (S >> 5));
+  uint32_t* w = (cyc ? A.wr : A.wq) + base;
+  const uint32_t* twf = (cyc ? A.fwdR : A.fwdQ) + size_t(k) * n;
+  const uint32_t* twi = (cyc ? A.invR : A.invQ) + size_t(k) * n;
+
+  auto gld = [&](uint32_t i) {
+    if constexpr (SRC == 0) return ld_w(w, i);
+    else return uint32_t(lz_digit<SRC>(A.x + so, n, i, P));
+  };
+  auto gst = [&](uint32_t i, uint32_t v) { st_w(w, i, v); };
+  auto lld = [&](uint32_t i) { return X[lpad(i)]; };
+  auto lst = [&](uint32_t i, uint32_t v) { X[lpad(i)] = v; };
+
+  uint32_t x[1 << LR], op[1 << LR], oy[1 << LR];
+  LzRoots<M, LR, 0> rf, ri;
+  SchedTw<M, LR, 0> t0;
+  SchedTw<M, LR, NR - 1> ti;
+  const bool back = MODE == LZ_MULN || (cyc && (MODE == LZ_SQR || A.op != LZ_FWD));
+  if constexpr (ROOTS == 2) rf.load(tg, lineRoot, twf);
+  else round_tw(t0, M, 0, tg, lineRoot, twf);
+  round_load<LR, Sched<M, LR>::template rr<0>()>(x, M, 0, tg, gld);
+  if constexpr (MODE == LZ_MULN && SRC != 0) {
+    // m' + 2, or m' + R + 2 = m' for a negative m': R N = -2 N mod Q.
+    if (tg == 0u && A.neg != nullptr && A.neg[so] == 0u)
+      x[0] = uint32_t(lz_red(int32_t(x[0] + 2u * uint32_t(A.c.one[k])), P));
+  }
+  if constexpr (ROOTS == 2) {
+    if (back) ri.load(tg, lineRoot, twi);
+  }
+  auto prefetch = [&] {
+    if constexpr (ROOTS == 1) {
+      if (back) round_tw(ti, M, LR * (NR - 1), tg, lineRoot, twi);
+    }
+    if (back) {
+      const uint32_t* o = (MODE == LZ_MULN ? A.nq : A.nir) + base;
+#pragma unroll
+      for (int e = 0; e < (1 << LR); ++e) op[e] = ld_w(o, uint32_t(e) * T + tg);
+    }
+    if constexpr (MODE == LZ_MULN) {
+      const uint32_t* o = A.tq + base;
+#pragma unroll
+      for (int e = 0; e < (1 << LR); ++e) oy[e] = ld_w(o, uint32_t(e) * T + tg);
+    }
+  };
+  lz_fwd<M, LR, 0, ROOTS, S0>(x, tg, lineRoot, twf, P, gld, lld, lst, t0, rf, prefetch);
+
+  if constexpr (MODE == LZ_GEN) {
+    if (A.op == LZ_MULY) {
+      const uint32_t* o = (cyc ? A.yr : A.yq) + base;
+#pragma unroll
+      for (int e = 0; e < (1 << LR); ++e) oy[e] = ld_w(o, uint32_t(e) * T + tg);
+    } else {
+#pragma unroll
+      for (int e = 0; e < (1 << LR); ++e) oy[e] = uint32_t(A.c.one[k]);
+    }
+  }
+  if (back) {
+#pragma unroll
+    for (int e = 0; e < (1 << LR); ++e) {
+      if constexpr (MODE == LZ_MULN) {
+        x[e] = uint32_t(lz_mul(int32_t(x[e]), int32_t(op[e]), P)) - oy[e];
+      } else {
+        const int32_t y = MODE == LZ_SQR ? int32_t(x[e]) : int32_t(oy[e]);
+        x[e] = uint32_t(lz_mul(lz_mul(int32_t(x[e]), y, P), int32_t(op[e]), P));
+      }
+    }
+    // Single-pass values go to the carry; a column pass follows otherwise.
+    lz_inv<M, LR, NR - 1, ROOTS, SRC != 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
+  } else {
+    int32_t c = A.scale[k];
+    if (MODE == LZ_SQR || A.op != LZ_FWD) {
+      const uint32_t a = lz_multiplier(A.mul, blockIdx.z, slot);
+      c = lz_mulc(int32_t(a), A.c.cq[k], uint32_t(A.c.cq[k]) * P.q, P.p);
+    }
+    const uint32_t cp = uint32_t(c) * P.q;
+#pragma unroll
+    for (int e = 0; e < (1 << LR); ++e) {
+      int32_t v = int32_t(x[e]);
+      if constexpr (MODE == LZ_SQR) {
+        v = lz_mulc(lz_mul(v, v, P), c, cp, P.p);
+      } else {
+        if (A.op != LZ_FWD) v = lz_mul(v, int32_t(oy[e]), P);
+        if (c != 0) v = lz_mulc(v, c, cp, P.p);
+      }
+      st_w(w, uint32_t(e) * T + tg, uint32_t(v));
+    }
+    (void)RL;
+  }
+}
+
+// Column passes of lengths from 2^14 on: the first M = m1 levels on columns of
+// stride n2 = n / 2^M, A.cols (8 for M = 10) consecutive columns per block,
+// interleaved and XOR-swizzled in LDS as the passes over the long primes.
+// Forward reads digits, so that the planes of one column group share them.
+template <int M>
+struct LzCol {
+  static constexpr int LR = (M >= 10) ? 5 : 4;
+  static constexpr bool LDS_ROOTS = (LR == 4);
+  static constexpr int THREADS = (M >= 10) ? 256 : 1024;
+  static constexpr int WAVES = (M >= 10) ? 4 : 4;
+};
+
+template <int M, int DL>
+__global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(const LzNtt A) {
+  extern __shared__ uint32_t lds[];
+  constexpr int LR = LzCol<M>::LR;
+  constexpr uint32_t S = 1u << M;
+  constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.z);
+  const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
+  const int pl = A.pl0 + int(blockIdx.y);
+  const bool cyc = pl < A.KR;
+  const int k = cyc ? pl : pl - A.KR;
+  const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
+  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const uint32_t line = threadIdx.x % C, tg = threadIdx.x / C;
+  const uint32_t n2 = uint32_t(n >> M), col0 = col_group(C) * C;
+  uint32_t* dst = (cyc ? A.wr : A.wq) + so + size_t(k) * n + col0;
+  const uint32_t* twf = (cyc ? A.fwdR : A.fwdQ) + size_t(k) * n;
+  const uint32_t* xd = A.x + so;
+
+  auto gld = [&](uint32_t i) { return uint32_t(lz_digit<DL>(xd, n, col0 + line + i * n2, P)); };
+  auto gst = [&](uint32_t i, uint32_t v) { dst[line + i * n2] = v; };
+  auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
+  auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
+
+  uint32_t x[1 << LR];
+  LzRoots<M, LR, 0> none;
+  SchedTw<M, LR, 0> t0;
+  if constexpr (!LzCol<M>::LDS_ROOTS) round_tw(t0, M, 0, tg, 1u, twf);
+  round_load<LR, Sched<M, LR>::template rr<0>()>(x, M, 0, tg, gld);
+  if (A.neg != nullptr && threadIdx.x == 0u && col0 == 0u && A.neg[so] == 0u)
+    x[0] = uint32_t(lz_red(int32_t(x[0] + 2u * uint32_t(A.c.one[k])), P));  // m' + 2, as in k_lz_row
+  if constexpr (LzCol<M>::LDS_ROOTS) {
+    uint32_t* roots = lds + C * S;
+    for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twf[i];
+    __syncthreads();
+    lz_fwd<M, LR, 0, 0, LZ_IN>(x, tg, 1u, roots, P, gld, lld, lst, t0, none, [] {});
+  } else {
+    lz_fwd<M, LR, 0, 1, LZ_IN>(x, tg, 1u, twf, P, gld, lld, lst, t0, none, [] {});
+  }
+  round_store<LR, RL>(x, M, DLV, tg, gst);
+}
+
+template <int M>
+__global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(const LzNtt A) {
+  extern __shared__ uint32_t lds[];
+  constexpr int LR = LzCol<M>::LR;
+  constexpr uint32_t S = 1u << M;
+  constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
+  const size_t so = size_t(lz_slot(A.slot_ids, blockIdx.z)) * A.slot_stride, n = size_t(1) << A.LN;
+  const int pl = A.pl0 + int(blockIdx.y);
+  const bool cyc = pl < A.KR;
+  const int k = cyc ? pl : pl - A.KR;
+  const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
+  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const uint32_t line = threadIdx.x % C, tg = threadIdx.x / C;
+  const uint32_t n2 = uint32_t(n >> M);
+  uint32_t* w = (cyc ? A.wr : A.wq) + so + size_t(k) * n + size_t(col_group(C)) * C;
+  const uint32_t* twi = (cyc ? A.invR : A.invQ) + size_t(k) * n;
+
+  auto gld = [&](uint32_t i) { return w[line + i * n2]; };
+  auto gst = [&](uint32_t i, uint32_t v) { w[line + i * n2] = v; };
+  auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
+  auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
+
+  uint32_t x[1 << LR];
+  LzRoots<M, LR, 0> none;
+  SchedTw<M, LR, NR - 1> ti;
+  round_load<LR, RL>(x, M, DLV, tg, gld);
+  if constexpr (LzCol<M>::LDS_ROOTS) {
+    uint32_t* roots = lds + C * S;
+    for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twi[i];
+    __syncthreads();
+    lz_inv<M, LR, NR - 1, 0, true>(x, tg, 1u, roots, P, gst, lld, lst, ti, none);
+  } else {
+    round_tw(ti, M, DLV, tg, 1u, twi);
+    lz_inv<M, LR, NR - 1, 1, true>(x, tg, 1u, twi, P, gst, lld, lst, ti, none);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// CRT + carry, one coefficient per thread.
+//
+// A wave takes 64 consecutive coefficients and finishes the last 64 - ND; the
+// first ND are the previous wave's, computed again for what they carry over,
+// so no wave waits for another and neighbours exchange by lane shifts.  A
+// coefficient V is cut into ND base-B digits d_0 .. d_{ND-1} (the last one
+// signed); the sum s_i = d_0 + B-aligned digits of the ND - 1 coefficients
+// below it is formed by ND - 1 shift-and-add steps; s_i = q B + r with r in
+// [-B/2, B/2), and the digit is r + q of the coefficient below.  Values are
+// kept exactly: what leaves lane i is what lane i + 1 adds, and what crosses
+// the top of the number enters digit 0, negated modulo B^n + 1.  Digits lie in
+// [-B/2 - 16, B/2 + 16).
+// ---------------------------------------------------------------------------
+
+template <int DL>
+struct LzDig;
+template <>
+struct LzDig<2> {
+  int64_t v;
+};
+template <>
+struct LzDig<3> {
+  uint64_t v;
+  int32_t h;
+};
+
+// The value of the lane below (lane 0: 0).
+__device__ __forceinline__ uint32_t lz_shr1(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x138, 0xf, 0xf, false));  // wave_shr:1
+}
+__device__ __forceinline__ LzDig<2> lz_below(const LzDig<2>& d) {
+  const uint64_t u = uint64_t(d.v);
+  return {int64_t(uint64_t(lz_shr1(uint32_t(u))) | (uint64_t(lz_shr1(uint32_t(u >> 32))) << 32))};
+}
+__device__ __forceinline__ LzDig<3> lz_below(const LzDig<3>& d) {
+  return {uint64_t(lz_shr1(uint32_t(d.v))) | (uint64_t(lz_shr1(uint32_t(d.v >> 32))) << 32),
+          int32_t(lz_shr1(uint32_t(d.h)))};
+}
+__device__ __forceinline__ LzDig<2> lz_add(const LzDig<2>& a, const LzDig<2>& b) { return {a.v + b.v}; }
+__device__ __forceinline__ LzDig<3> lz_add(const LzDig<3>& a, const LzDig<3>& b) {
+  const uint64_t v = a.v + b.v;
+  return {v, a.h + b.h + (v < a.v ? 1 : 0)};
+}
+__device__ __forceinline__ LzDig<2> lz_neg(const LzDig<2>& a) { return {-a.v}; }
+__device__ __forceinline__ LzDig<3> lz_neg(const LzDig<3>& a) { return {0ull - a.v, ~a.h + (a.v == 0 ? 1 : 0)}; }
+__device__ __forceinline__ LzDig<2> lz_small(LzDig<2>, int32_t v) { return {int64_t(v)}; }
+__device__ __forceinline__ LzDig<3> lz_small(LzDig<3>, int32_t v) { return {uint64_t(int64_t(v)), v >> 31}; }
+__device__ __forceinline__ bool lz_zero(const LzDig<2>& a) { return a.v == 0; }
+__device__ __forceinline__ bool lz_zero(const LzDig<3>& a) { return a.v == 0 && a.h == 0; }
+__device__ __forceinline__ bool lz_minus(const LzDig<2>& a) { return a.v < 0; }
+__device__ __forceinline__ bool lz_minus(const LzDig<3>& a) { return a.h < 0; }
+
+// s = q B + r, r in [-B/2, B/2): returns q, leaves r in s.  sh = cbits mod 32
+// (DL = 2: B = 2^(32 + sh), sh > 0; DL = 3: B = 2^(64 + sh)).
+__device__ __forceinline__ int32_t lz_split(LzDig<2>& s, uint32_t sh) {
+  const int64_t q = (s.v + (int64_t(1) << (31 + sh))) >> (32 + sh);
+  s.v -= q << (32 + sh);
+  return int32_t(q);
+}
+__device__ __forceinline__ int32_t lz_split(LzDig<3>& s, uint32_t sh) {
+  // Adding B/2 = 2^(63 + sh) carries from bit 63 when sh = 0.
+  const int32_t top = sh == 0u ? s.h + int32_t(s.v >> 63) : s.h + (int32_t(1) << (sh - 1u));
+  const int32_t q = top >> sh;
+  s.h -= int32_t(uint32_t(q) << sh);
+  return q;
+}
+
+template <int DL>
+__device__ __forceinline__ LzDig<DL> lz_load_digit(const uint32_t* x, size_t n, uint32_t i) {
+  const uint2 d = reinterpret_cast<const uint2*>(x)[i];
+  LzDig<DL> r;
+  r.v = uint64_t(d.x) | (uint64_t(d.y) << 32);
+  if constexpr (DL == 3) r.h = int32_t(x[2 * n + i]);
+  return r;
+}
+template <int DL>
+__device__ __forceinline__ void lz_store_digit(uint32_t* x, size_t n, uint32_t i, const LzDig<DL>& d) {
+  const uint64_t u = uint64_t(d.v);
+  reinterpret_cast<uint2*>(x)[i] = make_uint2(uint32_t(u), uint32_t(u >> 32));
+  if constexpr (DL == 3) x[2 * n + i] = uint32_t(d.h);
+}
+
+// The lowest digit of the two's complement limbs v, which move down by B
+// (their count L drops by DL - 1); the top digit is what is left.
+template <int DL, int L>
+__device__ __forceinline__ LzDig<DL> lz_take(uint32_t (&v)[LZ_MAXL], uint32_t sh) {
+  const uint32_t mask = (1u << sh) - 1u;
+  LzDig<DL> d;
+  if constexpr (DL == 2) {
+    d.v = int64_t(uint64_t(v[0]) | (uint64_t(v[1] & mask) << 32));
+  } else {
+    d.v = uint64_t(v[0]) | (uint64_t(v[1]) << 32);
+    d.h = int32_t(v[2] & mask);
+  }
+#pragma unroll
+  for (int j = 0; j + DL < L; ++j) v[j] = __builtin_amdgcn_alignbit(v[j + DL], v[j + DL - 1], sh);
+  v[L - DL] = uint32_t(int32_t(v[L - 1]) >> sh);
+  return d;
+}
+template <int DL, int L>
+__device__ __forceinline__ LzDig<DL> lz_top(const uint32_t (&v)[LZ_MAXL]) {
+  LzDig<DL> d;
+  const uint32_t s1 = uint32_t(int32_t(v[L - 1]) >> 31);
+  d.v = uint64_t(v[0]) | (uint64_t(L > 1 ? v[1] : s1) << 32);
+  if constexpr (DL == 3) d.h = int32_t(L > 2 ? v[2] : s1);
+  return d;
+}
+
+// d_J .. d_{ND-1} of v, then s = d_J + (what the lane below has from d_{J+1} on).
+template <int DL, int L, int ND, bool NEGA, int J>
+__device__ __forceinline__ LzDig<DL> lz_horner(uint32_t (&v)[LZ_MAXL], uint32_t sh, bool wrap) {
+  if constexpr (J == ND - 1) {
+    return lz_top<DL, L>(v);
+  } else {
+    const LzDig<DL> d = lz_take<DL, L>(v, sh);
+    LzDig<DL> up = lz_below(lz_horner<DL, L - (DL - 1), ND, NEGA, J + 1>(v, sh, wrap));
+    if (NEGA && wrap) up = lz_neg(up);
+    return lz_add(d, up);
+  }
+}
+
+template <int DL, int L, int ND, bool NEGA>
+__device__ __forceinline__ LzDig<DL> lz_finish(uint32_t (&v)[LZ_MAXL], uint32_t sh, bool wrap) {
+  LzDig<DL> s = lz_horner<DL, L, ND, NEGA, 0>(v, sh, wrap);
+  const int32_t q = lz_split(s, sh);
+  int32_t c = int32_t(lz_shr1(uint32_t(q)));
+  if (NEGA && wrap) c = -c;
+  return lz_add(s, lz_small(s, c));
+}
+
+// The coefficient as two's complement limbs.  The products of column l are
+// below 9 2^(28.2 + 32) < 2^63.4, so 64-bit sums hold them.
+template <int KP, int L>
+__device__ __forceinline__ void lz_crt(const LzCarry& A, const uint32_t* src, size_t n, uint32_t i, uint32_t (&v)[LZ_MAXL]) {
+  uint64_t col[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) col[l] = 0;
+  float f = 0.5f;
+  int32_t r[KP];
+#pragma unroll
+  for (int k = 0; k < KP; ++k) r[k] = int32_t(ld_w(src + size_t(k) * n, i));
+#pragma unroll
+  for (int k = 0; k < KP; ++k) {
+    int32_t y = lz_mulc(r[k], A.c[k], uint32_t(A.c[k]) * A.q[k], A.p[k]);
+    y += (y >> 31) & int32_t(A.p[k]);
+    f += float(y) * A.inv[k];
+#pragma unroll
+    for (int l = 0; l < L; ++l) col[l] += uint64_t(uint32_t(y)) * A.M[k][l];
+  }
+  const uint32_t q = uint32_t(f);
+  uint64_t t = 0;
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    t += col[l];
+    const uint64_t u = uint64_t(q) * A.NP[l];
+    // col + carry < 2^63.5 and q NP < 2^36: no overflow.
+    t += u;
+    v[l] = uint32_t(t);
+    t >>= 32;
+  }
+}
+
+// Grid: (ceil(waves / 4), slots); block 256.
+template <int KP, int L, int ND, int DL, bool NEGA>
+__global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
+  constexpr int W = 64 - ND;
+  const size_t n = size_t(1) << A.LN;
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
+  const size_t so = size_t(slot) * A.slot_stride;
+  const uint32_t cbits = A.cbits_slot ? A.cbits_slot[slot] : uint32_t(A.cbits);
+  const uint32_t sh = cbits & 31u;
+  const uint32_t a = lz_multiplier(A.mul, blockIdx.y, slot);
+  bool snap = false;
+  if (A.dst2 != nullptr) {
+    snap = A.snap != nullptr ? (A.snap[blockIdx.y] & SLOT_SNAP) != 0u
+                             : (A.mul.bits_mode == 2 && ((A.mul.bits[blockIdx.y >> 5] >> (blockIdx.y & 31u)) & 1u));
+  }
+  const int lane = int(threadIdx.x & 63u);
+  const int wave = int(blockIdx.x * 4u + (threadIdx.x >> 6));
+  const int top = int((n - 1) / W);
+  if (wave > top) return;
+  for (int w = wave;; --w) {
+    const int i = w * W + lane - ND;
+    const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
+    uint32_t v[LZ_MAXL];
+    lz_crt<KP, L>(A, A.src + so, n, idx, v);
+    if (a != 1u) {
+      uint64_t t = 0;
+#pragma unroll
+      for (int l = 0; l < L; ++l) {
+        t += uint64_t(v[l]) * a;
+        v[l] = uint32_t(t);
+        t >>= 32;
+      }
+    }
+    const LzDig<DL> d = lz_finish<DL, L, ND, NEGA>(v, sh, i == 0);
+    const bool own = lane >= ND && uint32_t(i) < n;
+    if (w == wave && own) {
+      lz_store_digit<DL>(A.dst + so, n, uint32_t(i), d);
+      if (snap) lz_store_digit<DL>(A.dst2 + so, n, uint32_t(i), d);
+    }
+    if (A.neg == nullptr || wave != top) return;
+    // The sign of the number is that of its highest nonzero digit: nearly
+    // always the top one; the last wave goes on downwards if its digits are
+    // all zero.
+    const uint64_t nz = __ballot(own && !lz_zero(d));
+    const uint64_t mi = __ballot(own && lz_minus(d));
+    if (nz != 0ull || w == 0) {
+      if (lane == 0) A.neg[so] = nz != 0ull ? uint32_t((mi >> (63 - __clzll((long long)(nz)))) & 1ull) : 0u;
+      return;
+    }
+  }
+}
+
+// Residues of the plan's K primes -> digits (mod B^n + 1, which keeps every
+// register): the CRT value of each coefficient, carried as above.
+template <int K, int DL>
+__global__ void __launch_bounds__(256) k_lz_import(const LzConv A) {
+  constexpr int ND = 3, W = 64 - ND, L = K + 1;
+  const size_t n = size_t(1) << A.LN;
+  const int lane = int(threadIdx.x & 63u), w = int(blockIdx.x * 4u + (threadIdx.x >> 6));
+  const int i = w * W + lane - ND;
+  if (w * W >= int(n)) return;
+  const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
+  uint32_t r[K], acc[L], v[LZ_MAXL];
+#pragma unroll
+  for (int k = 0; k < K; ++k) r[k] = ld_w(A.src + size_t(k) * n, idx);
+  garner<K, L>(r, acc);
+#pragma unroll
+  for (int l = 0; l < L; ++l) v[l] = acc[l];
+  const LzDig<DL> d = lz_finish<DL, L, ND, true>(v, uint32_t(A.cbits) & 31u, i == 0);
+  if (lane >= ND && uint32_t(i) < n) lz_store_digit<DL>(A.dst, n, uint32_t(i), d);
+}
+
+// Digits -> residues of the plan's K primes, of the balanced digits in
+// [-B/2, B/2) (three carry steps: a longer run of carries would need three
+// digits at the edge of their range in a row, and keeps the value all the
+// same).  neg: the register is m' (mod B^n - 1) of that sign, exported as the
+// squaring defines it: m' + 2, plus R = B^n - 1 when negative.
+template <int K, int DL>
+__global__ void __launch_bounds__(256) k_lz_export(const LzConv A) {
+  constexpr int H = 3, W = 64 - H;
+  const size_t n = size_t(1) << A.LN;
+  const int lane = int(threadIdx.x & 63u), w = int(blockIdx.x * 4u + (threadIdx.x >> 6));
+  const int i = w * W + lane - H;
+  if (w * W >= int(n)) return;
+  const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
+  const uint32_t sh = uint32_t(A.cbits) & 31u;
+  LzDig<DL> s = lz_load_digit<DL>(A.src, n, idx);
+#pragma unroll
+  for (int step = 0; step < H; ++step) {
+    const int32_t q = lz_split(s, sh);
+    int32_t c = int32_t(lz_shr1(uint32_t(q)));
+    if (A.neg == nullptr && i == 0) c = -c;
+    s = lz_add(s, lz_small(s, c));
+  }
+  if (lane < H || uint32_t(i) >= n) return;
+  if (A.neg != nullptr) {
+    const bool neg = A.neg[0] != 0u;
+    if (i == 0) s = lz_add(s, lz_small(s, neg ? 1 : 2));
+    if (neg && uint32_t(i) == n - 1) {
+      if constexpr (DL == 2) s.v += int64_t(1) << (32 + sh);
+      else s.h += int32_t(1) << sh;
+    }
+  }
+  uint32_t d[DIGIT_LIMBS];
+  const uint64_t u = uint64_t(s.v);
+  d[0] = uint32_t(u);
+  d[1] = uint32_t(u >> 32);
+  if constexpr (DL == 3) d[2] = uint32_t(s.h);
+  else d[2] = uint32_t(int32_t(d[1]) >> 31);
+#pragma unroll
+  for (int k = 0; k < K; ++k) st_w(A.dst + size_t(k) * n, uint32_t(i), digit_residue_wide(d, k));
+}
+
+// Root tables (heap-indexed as make_tables in plan.h) in signed Montgomery form,
+// |w| <= p / 2: entry 2^l + b is psi^e with e = 2 h brv_l(b) (cyclic) or h (2
+// brv_l(b) + 1) (negacyclic), h = n / 2^{l+1}, or its inverse psi^{2n - e}.  pw
+// holds psi^i for i < 2^s, then psi^{i 2^s}, per prime (s = ceil(LN / 2)).
+__global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C) {
+  const uint32_t n = 1u << LN, idx = blockIdx.x * 256u + threadIdx.x;
+  const int k = int(blockIdx.y);
+  if (idx >= n) return;
+  const LzP P{C.p[k], C.q[k], C.bar[k]};
+  const int s = (LN + 1) / 2;
+  const uint32_t* w = pw + size_t(k) * ((1u << s) + (1u << (LN + 1 - s)));
+  const int l = idx == 0u ? 0 : 31 - __clz(int(idx));
+  const uint32_t b = idx == 0u ? 0u : idx - (1u << l);
+  const uint32_t br = l == 0 ? 0u : __brev(b) >> (32 - l), h = n >> (l + 1), mask = 2u * n - 1u;
+  auto root = [&](uint32_t e) {
+    const int32_t lo = int32_t(w[e & ((1u << s) - 1u)]), hi = int32_t(w[(1u << s) + (e >> s)]);
+    uint32_t v = uint32_t(lz_red(lz_mul(lo, hi, P), P));
+    if (v >= P.p) v -= P.p;
+    return v > P.p / 2 ? v - P.p : v;
+  };
+  const uint32_t eR = idx == 0u ? 0u : (2u * h * br) & mask, eQ = idx == 0u ? 0u : (h * (2u * br + 1u)) & mask;
+  tw[size_t(k) * n + idx] = root(eR);
+  tw[(size_t(KR) + k) * n + idx] = root((2u * n - eR) & mask);
+  if (k < KQ) {
+    tw[(2 * size_t(KR) + k) * n + idx] = root(eQ);
+    tw[(2 * size_t(KR) + KQ + k) * n + idx] = root((2u * n - eQ) & mask);
+  }
+}
+
+// Instantiations, looked up by the host engine.  Eight elements per thread
+// (LR = 3) for short launches, sixteen where they fill the GPU.
+#define LZ_ROW(M, LR, SRC)                                             \
+  template __global__ void k_lz_row<M, LR, LZ_SQR, SRC>(const LzNtt);  \
+  template __global__ void k_lz_row<M, LR, LZ_MULN, SRC>(const LzNtt); \
+  template __global__ void k_lz_row<M, LR, LZ_GEN, SRC>(const LzNtt);
+#define LZ_ROW1(M)  \
+  LZ_ROW(M, 3, 2) \
+  LZ_ROW(M, 3, 3) \
+  LZ_ROW(M, 4, 2) \
+  LZ_ROW(M, 4, 3)
+LZ_ROW1(8)
+LZ_ROW1(9)
+LZ_ROW1(10)
+LZ_ROW1(11)
+LZ_ROW1(12)
+LZ_ROW1(13)
+#define LZ_ROW2(M) LZ_ROW(M, 3, 0) LZ_ROW(M, 4, 0)
+LZ_ROW2(7)
+LZ_ROW2(8)
+LZ_ROW2(9)
+LZ_ROW2(10)
+#define LZ_COL(M)                                          \
+  template __global__ void k_lz_colf<M, 2>(const LzNtt);   \
+  template __global__ void k_lz_colf<M, 3>(const LzNtt);   \
+  template __global__ void k_lz_coli<M>(const LzNtt);
+LZ_COL(7)
+LZ_COL(8)
+LZ_COL(9)
+LZ_COL(10)
+template __global__ void k_lz_carry<6, 6, 5, 2, false>(const LzCarry);
+template __global__ void k_lz_carry<4, 4, 3, 2, true>(const LzCarry);
+template __global__ void k_lz_carry<7, 7, 4, 2, false>(const LzCarry);
+template __global__ void k_lz_carry<5, 5, 3, 2, true>(const LzCarry);
+template __global__ void k_lz_carry<9, 8, 4, 3, false>(const LzCarry);
+template __global__ void k_lz_carry<6, 6, 3, 3, true>(const LzCarry);
+#define LZ_CONV(K, DL)                                        \
+  template __global__ void k_lz_import<K, DL>(const LzConv);  \
+  template __global__ void k_lz_export<K, DL>(const LzConv);
+LZ_CONV(3, 2)
+LZ_CONV(4, 2)
+LZ_CONV(5, 3)
+
+}  // namespace annie

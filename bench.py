@@ -79,6 +79,16 @@ def alg_bytes(kind, U, K=5):
     """
     name, jobs = kind.rsplit("x", 1)
     jobs = int(jobs)
+    if name.startswith("k_lz_"):
+        # Short primes: planes of W = 4 n bytes (`jobs` of them); 6, 7 or 9 of
+        # them cyclic, digits of 2 or 3 words.
+        W, cyclic, limbs = U // K, {3: 6, 4: 7, 5: 9}[K], 3 if K == 5 else 2
+        if name.startswith("k_lz_row"):
+            mode = name.split(",")[1].rstrip(">")
+            return W * (4 * jobs if mode == "muln" else 2 * jobs + (cyclic if mode == "sqr" else 0))
+        if name.startswith("k_lz_carry"):
+            return W * ((cyclic if name.startswith("k_lz_carryR") else cyclic - 2 if K < 5 else 6) + limbs)
+        return W * (limbs + jobs if name.startswith("k_lz_colf") else 2 * jobs)
     digits = 3 * U // K
     if name.startswith("k_row"):
         mode = name.split(",")[1].rstrip(">")
