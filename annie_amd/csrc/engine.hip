@@ -49,6 +49,8 @@ __global__ void k_lz_coli(const LzNtt A);
 template <int KP, int L, int ND, int DL, bool NEGA>
 __global__ void k_lz_carry(const LzCarry A);
 __global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
+template <int DL>
+__global__ void k_lz_pack(const LzPack A);
 template <int K, int DL>
 __global__ void k_lz_import(const LzConv A);
 template <int K, int DL>
@@ -108,6 +110,7 @@ struct Stage {
 enum LzReg : int { LX0 = 0, LX1 = 1, LX2 = 2, LZ_ONE, LZ_SNAP, LZ_MP, LZ_GET, NLZ };
 enum LzPlanes : int { PNIR = 0, PNQ, PWR, PWQ, PMQ, PYR, PYQ, NPLANES };
 constexpr size_t LZ_FLAGS = 64;
+constexpr size_t LZ_PACK_WORDS = size_t(1) << 22;  // get() staging of a context (more only where one value needs it)
 
 struct Lazy {
   bool on = false;
@@ -124,6 +127,9 @@ struct Lazy {
   // has the non-negative digits of its residue.
   bool is_one[3] = {false, false, false};
   uint32_t last_a = 1;  // last multiplier found to fit
+  // Staging of get(): packed words on the device and in pinned memory.
+  uint32_t *pack = nullptr, *pack_host = nullptr;
+  size_t pack_words = 0;
 };
 
 struct Ctx {
@@ -765,7 +771,9 @@ static int lz_limbs(int K, bool cyc) { return cyc ? (K == 3 ? 6 : K == 4 ? 7 : 8
 
 static int lz_elements(const Ctx& c) {
   if (const char* e = std::getenv("ANNIE_LZ_LR")) return std::atoi(e);
-  return (c.nslots_alloc << c.pl.LN) >= (size_t(1) << 17) ? 4 : 3;
+  // Lines of 2^9 and shorter would leave half a wave idle at sixteen.
+  const int M = c.pl.LN <= 13 ? c.pl.LN : c.pl.LN - c.pl.LN / 2;
+  return (c.nslots_alloc << c.pl.LN) >= (size_t(1) << 17) && M >= 10 ? 4 : 3;
 }
 
 static int lz_setup(Ctx& c) {
@@ -839,7 +847,7 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
     if (c.sched_lines != 0) lines = c.sched_lines;  // checked by annie_hip_set_schedule
   }
   A.cols = int(lines);
-  const dim3 grid(rows / lines, unsigned(planes), unsigned(c.nslots)), block(lines * T);
+  const dim3 grid(rows / lines, unsigned(c.nslots), unsigned(planes)), block(lines * T);
   const size_t shm = size_t(lines) * (S + (S >> 5)) * 4;
   LzKernel f = nullptr;
   switch (single ? 100 * z.sh.DL + c.m2 : c.m2) {
@@ -872,7 +880,7 @@ static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
   if (c.sched_cols != 0 && !wide) C = c.sched_cols;  // checked by annie_hip_set_schedule
   if (wide && C != 8u) return fail(ANNIE_ERR_SIZE, "column pass geometry");
   A.cols = int(C);
-  const dim3 grid(uint32_t(c.n >> c.m1) / C, unsigned(planes), unsigned(c.nslots)), block(C * T);
+  const dim3 grid(uint32_t(c.n >> c.m1) / C, unsigned(c.nslots), unsigned(planes)), block(C * T);
   const size_t shm = size_t(wide ? C : C + 1) * S * 4;
   LzKernel f = nullptr;
   switch (c.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
@@ -1183,6 +1191,8 @@ static void destroy(annie_hip_t* h) {
   if (c.tw) (void)hipFree(c.tw);
   if (c.lz.mem) (void)hipFree(c.lz.mem);
   if (c.lz.tw) (void)hipFree(c.lz.tw);
+  if (c.lz.pack) (void)hipFree(c.lz.pack);
+  if (c.lz.pack_host) (void)hipHostFree(c.lz.pack_host);
   for (auto& g : c.graphs) (void)hipGraphExecDestroy(g.exec);
   if (c.graph_buf) (void)hipFree(c.graph_buf);
   if (c.cbits_dev) (void)hipFree(c.cbits_dev);
@@ -1454,26 +1464,49 @@ static int lz_square(Ctx& c, uint32_t a, const uint32_t* a_slot, bool bits) {
   return lz_product(c, B, LZ_SQR, 0, m);
 }
 
-// get() on the short-prime path: the product by 1, read back as digits.
+// get() on the short-prime path: the product by 1, packed into binary words on
+// the device and read back through pinned memory, as many list positions at a
+// time as the context's staging words hold.  The product is below 4 N, so
+// that a few subtractions reduce it.
 static int lz_get_values(Ctx& c, int src, const size_t* slots, const mpz_t* const* mods, mpz_t* const* zs, size_t count) {
   int rc;
   if ((rc = lz_product(c, lz_bufs(c, c.lzreg(src), c.lzreg(LZ_GET)), LZ_GEN, LZ_MUL1, lz_by(1u)))) return rc;
-  const int DL = c.lz.sh.DL;
-  const size_t w = size_t(DL) * c.n;
-  std::vector<uint32_t> d(w * count);
-  for (size_t i = 0; i < count; ++i)
-    HIPCHK(hipMemcpyAsync(d.data() + i * w, c.lzreg(LZ_GET) + slots[i] * c.lz.stride, w * 4, hipMemcpyDeviceToHost,
-                          c.stream));
-  HIPCHK(hipStreamSynchronize(c.stream));
-  for (size_t i = 0; i < count; ++i) {
-    const uint32_t* di = d.data() + i * w;
-    auto at = [&](size_t j) {
-      const uint64_t lo = uint64_t(di[2 * j]) | (uint64_t(di[2 * j + 1]) << 32);
-      if (DL == 2) return __int128(int64_t(lo));
-      return __int128((unsigned __int128)lo | ((unsigned __int128)(__int128)int32_t(di[2 * c.n + j]) << 64));
-    };
-    digits_to_mpz(c, at, slot_cbits(c, slots[i]), *zs[i]);
-    mpz_mod(*zs[i], *zs[i], *mods[i]);
+  Lazy& z = c.lz;
+  int cb = 0;
+  for (size_t i = 0; i < count; ++i) cb = std::max(cb, slot_cbits(c, slots[i]));
+  const size_t per = (c.n / 32) * size_t(cb), chunk = std::min(count, std::max<size_t>(1, LZ_PACK_WORDS / per));
+  if (z.pack_words < chunk * per) {
+    HIPCHK(hipStreamSynchronize(c.stream));
+    if (z.pack) (void)hipFree(z.pack);
+    if (z.pack_host) (void)hipHostFree(z.pack_host);
+    z.pack = z.pack_host = nullptr;
+    z.pack_words = 0;
+    if (hipMalloc(&z.pack, chunk * per * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "packed words");
+    if (hipHostMalloc(&z.pack_host, chunk * per * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "pinned words");
+    z.pack_words = chunk * per;
+  }
+  for (size_t i0 = 0; i0 < count; i0 += chunk) {
+    const size_t m = std::min(chunk, count - i0);
+    LzPack A{c.lzreg(LZ_GET), z.pack, c.slot_ids ? c.slot_ids + i0 : nullptr, z.stride, per, c.pl.LN, c.pl.cbits(), c.cbits_dev};
+    const dim3 grid(unsigned(c.n / 256), unsigned(m)), block(256);
+    if (z.sh.DL == 2) hipLaunchKernelGGL(k_lz_pack<2>, grid, block, 0, c.stream, A);
+    else hipLaunchKernelGGL(k_lz_pack<3>, grid, block, 0, c.stream, A);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(z.pack_host, z.pack, m * per * 4, hipMemcpyDeviceToHost, c.stream));
+    HIPCHK(hipStreamSynchronize(c.stream));
+    for (size_t i = 0; i < m; ++i) {
+      mpz_t& v = *zs[i0 + i];
+      const mpz_t& N = *mods[i0 + i];
+      const size_t words = (c.n / 32) * size_t(slot_cbits(c, slots[i0 + i]));
+      mpz_import(v, words, -1, 4, 0, 0, z.pack_host + i * per);
+      if (mpz_tstbit(v, mp_bitcnt_t(words) * 32 - 1)) {  // negative: only from a register that holds no residue
+        Mpz top;
+        mpz_setbit(top.v, mp_bitcnt_t(words) * 32);
+        mpz_sub(v, v, top.v);
+      }
+      if (mpz_sgn(v) < 0 || mpz_sizeinbase(v, 2) > mpz_sizeinbase(N, 2) + 2) mpz_mod(v, v, N);
+      while (mpz_cmp(v, N) >= 0) mpz_sub(v, v, N);
+    }
   }
   return ANNIE_OK;
 }

@@ -80,7 +80,7 @@ enum LzOp : int {
   LZ_MUL1 = 2,   // as LZ_SQR with x^ 1^
 };
 
-// One NTT pass over planes [pl0, pl0 + gridDim.y): plane k < KR is the cyclic
+// One NTT pass over planes [pl0, pl0 + gridDim.z): plane k < KR is the cyclic
 // transform of prime k, plane KR + k the negacyclic one.  Pointers address
 // slot 0; slot s lies at + s * slot_stride words.
 struct LzNtt {
@@ -124,6 +124,16 @@ struct LzConv {
   uint32_t* dst;
   const uint32_t* neg;  // export of m': + 2 (and + R - 2 + ... when negative), or null
   int LN, cbits;
+};
+
+// Digits -> binary words.
+struct LzPack {
+  const uint32_t* src;
+  uint32_t* dst;  // out_stride words per list position
+  const uint32_t* slot_ids;
+  size_t slot_stride, out_stride;
+  int LN, cbits;
+  const uint32_t* cbits_slot;
 };
 
 // The transform primes of length 2^LN: the largest primes k 2^e + 1 below

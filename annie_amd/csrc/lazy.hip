@@ -230,7 +230,9 @@ constexpr int lz_row_threads(int M, int LR) { return (1 << M >> LR) > 512 || (1 
 // between transforms (y^, n^, N^, t^) is kept in the order in which the
 // threads hold it, element e of thread tg at e T + tg, so that its loads and
 // stores are consecutive.
-// Grid: (rows / lines, planes, slots); block: lines of 2^M / 2^LR threads.
+// Grid: (rows / lines, slots, planes), so that the cyclic planes, which go
+// forward and back, start before the negacyclic ones, which only go forward
+// here; block: lines of 2^M / 2^LR threads.
 template <int M, int LR, int MODE, int SRC>
 __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A) {
   extern __shared__ uint32_t lds[];
@@ -238,9 +240,9 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
   constexpr int NR = Sched<M, LR>::NR, RL = Sched<M, LR>::template rr<NR - 1>();
   constexpr int ROOTS = LR <= 3 ? 2 : 1;
   constexpr int S0 = SRC ? LZ_IN : LZ_LIM;
-  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.z);
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
-  const int pl = A.pl0 + int(blockIdx.y);
+  const int pl = A.pl0 + int(blockIdx.z);
   const bool cyc = MODE != LZ_MULN && pl < A.KR;
   const int k = cyc ? pl : pl - A.KR;
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
@@ -320,7 +322,7 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
   } else {
     int32_t c = A.scale[k];
     if (MODE == LZ_SQR || A.op != LZ_FWD) {
-      const uint32_t a = lz_multiplier(A.mul, blockIdx.z, slot);
+      const uint32_t a = lz_multiplier(A.mul, blockIdx.y, slot);
       c = lz_mulc(int32_t(a), A.c.cq[k], uint32_t(A.c.cq[k]) * P.q, P.p);
     }
     const uint32_t cp = uint32_t(c) * P.q;
@@ -357,9 +359,9 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   constexpr int LR = LzCol<M>::LR;
   constexpr uint32_t S = 1u << M;
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
-  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.z);
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
-  const int pl = A.pl0 + int(blockIdx.y);
+  const int pl = A.pl0 + int(blockIdx.z);
   const bool cyc = pl < A.KR;
   const int k = cyc ? pl : pl - A.KR;
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
@@ -399,8 +401,8 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(
   constexpr int LR = LzCol<M>::LR;
   constexpr uint32_t S = 1u << M;
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
-  const size_t so = size_t(lz_slot(A.slot_ids, blockIdx.z)) * A.slot_stride, n = size_t(1) << A.LN;
-  const int pl = A.pl0 + int(blockIdx.y);
+  const size_t so = size_t(lz_slot(A.slot_ids, blockIdx.y)) * A.slot_stride, n = size_t(1) << A.LN;
+  const int pl = A.pl0 + int(blockIdx.z);
   const bool cyc = pl < A.KR;
   const int k = cyc ? pl : pl - A.KR;
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
@@ -706,6 +708,57 @@ __global__ void __launch_bounds__(256) k_lz_export(const LzConv A) {
   for (int k = 0; k < K; ++k) st_w(A.dst + size_t(k) * n, uint32_t(i), digit_residue_wide(d, k));
 }
 
+// A register that holds a non-negative number below B^n / 2, as binary words: 2
+// cbits words per wave of 64 digits, list position after list position.  Digit
+// i borrows from digit i + 1 when the highest nonzero digit at or below it is
+// negative: a ballot finds it in the wave, and the digits before the wave are
+// searched 64 at a time (one step unless they are all zero).
+// Grid: (ceil(n / 256), positions); block 256; digits from `count` on are zero.
+template <int DL>
+__global__ void __launch_bounds__(256) k_lz_pack(const LzPack A) {
+  __shared__ uint32_t u[4][64 * DL + 1];
+  const size_t n = size_t(1) << A.LN;
+  const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
+  const uint32_t* x = A.src + size_t(slot) * A.slot_stride;
+  const uint32_t cb = A.cbits_slot ? A.cbits_slot[slot] : uint32_t(A.cbits), sh = cb & 31u;
+  const int lane = int(threadIdx.x & 63u), wv = int(threadIdx.x >> 6);
+  const uint32_t w0 = blockIdx.x * 256u + uint32_t(wv) * 64u;
+  LzDig<DL> d = lz_load_digit<DL>(x, n, w0 + uint32_t(lane));
+  const uint64_t nz = __ballot(!lz_zero(d)), mi = __ballot(lz_minus(d));
+  uint32_t below = 0;  // whether the digits before the wave are a negative number
+  for (uint32_t b = w0; b != 0u; b -= 64u) {
+    const LzDig<DL> e = lz_load_digit<DL>(x, n, b - 64u + uint32_t(lane));
+    const uint64_t ez = __ballot(!lz_zero(e)), em = __ballot(lz_minus(e));
+    if (ez != 0ull) {
+      below = uint32_t((em >> (63 - __clzll((long long)ez))) & 1ull);
+      break;
+    }
+  }
+  const uint64_t under = nz & ((1ull << lane) - 1ull);
+  const uint32_t borrow = under != 0ull ? uint32_t((mi >> (63 - __clzll((long long)under))) & 1ull) : below;
+  d = lz_add(d, lz_small(d, -int32_t(borrow)));
+  if (lz_minus(d)) {
+    if constexpr (DL == 2) d.v += int64_t(1) << (32 + sh);
+    else d.h += int32_t(1) << sh;
+  }
+  u[wv][lane * DL] = uint32_t(uint64_t(d.v));
+  u[wv][lane * DL + 1] = uint32_t(uint64_t(d.v) >> 32);
+  if constexpr (DL == 3) u[wv][lane * DL + 2] = uint32_t(d.h);
+  if (lane == 0) u[wv][64 * DL] = 0u;
+  __syncthreads();
+  uint32_t* out = A.dst + size_t(blockIdx.y) * A.out_stride + size_t(w0 / 32u) * cb;
+  for (uint32_t w = uint32_t(lane); w < 2u * cb; w += 64u) {
+    // Bits [32 w, 32 w + 32) of the wave's digits: at most two digits (cb >= 32).
+    const uint32_t i = (32u * w) / cb, off = 32u * w - i * cb, k = off >> 5, r = off & 31u;
+    const uint32_t* p = &u[wv][i * DL];
+    uint32_t v = p[k] >> r;
+    if (r != 0u && int(k) + 1 < DL) v |= p[k + 1] << (32u - r);
+    const uint32_t have = cb - off;  // bits of digit i from off on
+    if (have < 32u) v = (v & ((1u << have) - 1u)) | (i < 63u ? p[DL] << have : 0u);
+    out[w] = v;
+  }
+}
+
 // Root tables (heap-indexed as make_tables in plan.h) in signed Montgomery form,
 // |w| <= p / 2: entry 2^l + b is psi^e with e = 2 h brv_l(b) (cyclic) or h (2
 // brv_l(b) + 1) (negacyclic), h = n / 2^{l+1}, or its inverse psi^{2n - e}.  pw
@@ -774,6 +827,8 @@ template __global__ void k_lz_carry<6, 6, 3, 3, true>(const LzCarry);
 #define LZ_CONV(K, DL)                                        \
   template __global__ void k_lz_import<K, DL>(const LzConv);  \
   template __global__ void k_lz_export<K, DL>(const LzConv);
+template __global__ void k_lz_pack<2>(const LzPack);
+template __global__ void k_lz_pack<3>(const LzPack);
 LZ_CONV(3, 2)
 LZ_CONV(4, 2)
 LZ_CONV(5, 3)
