@@ -40,13 +40,13 @@ __global__ void k_copy_slots(uint32_t* base, size_t dst_off, size_t src_off, siz
                              size_t slot_stride);
 template <int M, int K, int QS>
 __global__ void k_sqr_run(const RunArgs R);
-template <int M, int LR, int MODE, int SRC>
+template <int M, int LR, int MODE, int SRC, int W>
 __global__ void k_lz_row(const LzNtt A);
-template <int M, int DL>
+template <int M, int DL, int W>
 __global__ void k_lz_colf(const LzNtt A);
-template <int M>
+template <int M, int W>
 __global__ void k_lz_coli(const LzNtt A);
-template <int KP, int L, int ND, int DL, bool NEGA>
+template <int SET, int KP, int L, int ND, int DL, bool NEGA>
 __global__ void k_lz_carry(const LzCarry A);
 __global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
 template <int DL>
@@ -119,7 +119,6 @@ struct Lazy {
   std::vector<uint32_t> primes;
   LzPrimes pc{};
   int32_t scaleR[LZ_MAXP] = {}, scaleQ[LZ_MAXP] = {};  // of the transforms of N^-1 mod R and N
-  LzCarry cr{}, cq{};                                  // CRT constants of the cyclic / negacyclic planes
   uint32_t* mem = nullptr;
   uint32_t* tw = nullptr;  // roots: KR n cyclic forward, KR n inverse, KQ n negacyclic forward, KQ n inverse
   size_t stride = 0, plane0 = 0;
@@ -726,7 +725,7 @@ static int scale_reg(Ctx& c, int r, size_t slot = 0) {
 static bool lz_class_fits(const Plan& pl) {
   const char* off = std::getenv("ANNIE_LONG_PRIMES");
   if (off && off[0] == '1') return false;
-  if (pl.K < 3 || pl.LN < 8 || pl.LN > 20) return false;
+  if (pl.K < 3 || pl.LN < 8 || pl.LN > LZ_MAX_LN) return false;
   double lp = -1.0;
   for (int k = 0; k < pl.K; ++k) lp += std::log2(double(PRIMES[k]));
   int cb = pl.cbits();
@@ -741,33 +740,6 @@ static size_t lz_slot_words(int K, size_t n) {
 }
 
 static int32_t lz_signed(uint64_t v, uint32_t p) { return v > p / 2 ? int32_t(v) - int32_t(p) : int32_t(v); }
-
-// CRT constants of the first `count` primes on L limbs.
-static void lz_crt_consts(LzCarry& A, const std::vector<uint32_t>& primes, int count, int L) {
-  Mpz P, M, t;
-  mpz_set_ui(P.v, 1);
-  for (int k = 0; k < count; ++k) mpz_mul_ui(P.v, P.v, primes[k]);
-  auto limbs = [&](const mpz_t z, uint32_t* out) {
-    std::memset(out, 0, LZ_MAXL * 4);
-    mpz_export(out, nullptr, -1, 4, 0, 0, z);
-  };
-  for (int k = 0; k < count; ++k) {
-    const uint32_t p = primes[k];
-    mpz_divexact_ui(M.v, P.v, p);
-    limbs(M.v, A.M[k]);
-    A.p[k] = p;
-    A.q[k] = inv32(p);
-    A.inv[k] = float(1.0 / double(p));
-    A.c[k] = lz_signed(to_mont(invmod_plain(uint32_t(mpz_fdiv_ui(M.v, p)), p), p), p);
-  }
-  mpz_set_ui(t.v, 1);
-  mpz_mul_2exp(t.v, t.v, 32u * unsigned(L));
-  mpz_sub(t.v, t.v, P.v);
-  limbs(t.v, A.NP);
-}
-
-// Limbs of the carries' CRT values (as instantiated in lazy.hip).
-static int lz_limbs(int K, bool cyc) { return cyc ? (K == 3 ? 6 : K == 4 ? 7 : 8) : (K == 3 ? 4 : K == 4 ? 5 : 6); }
 
 static int lz_elements(const Ctx& c) {
   if (const char* e = std::getenv("ANNIE_LZ_LR")) return std::atoi(e);
@@ -791,8 +763,6 @@ static int lz_setup(Ctx& c) {
   if (hipMalloc(&z.mem, c.nslots_alloc * z.stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
   if (hipMalloc(&z.tw, (2 * size_t(KR) + 2 * size_t(KQ)) * n * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "roots");
   HIPCHK(hipMemsetAsync(z.mem, 0, c.nslots_alloc * z.stride * 4, c.stream));
-  lz_crt_consts(z.cr, z.primes, KR, lz_limbs(K, true));
-  lz_crt_consts(z.cq, z.primes, KQ, lz_limbs(K, false));
   // Powers psi^i, i < 2^s, and psi^{i 2^s} of a primitive 2n-th root psi of
   // each prime; the device multiplies them into the tables.
   const int s = (LN + 1) / 2, hi = LN + 1 - s;
@@ -829,10 +799,15 @@ static int lz_setup(Ctx& c) {
 
 typedef void (*LzKernel)(const LzNtt);
 
+template <int M, int LR, int SRC, int W>
+static LzKernel lz_row_mode(int mode) {
+  return mode == LZ_SQR    ? k_lz_row<M, LR, LZ_SQR, SRC, W>
+         : mode == LZ_MULN ? k_lz_row<M, LR, LZ_MULN, SRC, W>
+                           : k_lz_row<M, LR, LZ_GEN, SRC, W>;
+}
 template <int M, int SRC>
 static LzKernel lz_row_kernel(int LR, int mode) {
-  if (LR == 3) return mode == LZ_SQR ? k_lz_row<M, 3, LZ_SQR, SRC> : mode == LZ_MULN ? k_lz_row<M, 3, LZ_MULN, SRC> : k_lz_row<M, 3, LZ_GEN, SRC>;
-  return mode == LZ_SQR ? k_lz_row<M, 4, LZ_SQR, SRC> : mode == LZ_MULN ? k_lz_row<M, 4, LZ_MULN, SRC> : k_lz_row<M, 4, LZ_GEN, SRC>;
+  return LR == 3 ? lz_row_mode<M, 3, SRC, 0>(mode) : lz_row_mode<M, 4, SRC, 0>(mode);
 }
 
 // Rows of planes [A.pl0, A.pl0 + planes): the whole transform of a digit
@@ -865,6 +840,7 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
     case 8: f = lz_row_kernel<8, 0>(z.LR, mode); break;
     case 9: f = lz_row_kernel<9, 0>(z.LR, mode); break;
     case 10: f = lz_row_kernel<10, 0>(z.LR, mode); break;
+    case 11: f = lz_width(lz_set(c.pl.LN)) == 1 ? lz_row_mode<11, 4, 0, 1>(mode) : lz_row_mode<11, 4, 0, 2>(mode); break;
     default: return fail(ANNIE_ERR_SIZE, "no row kernel for this length");
   }
   ProfScope ps(c, "k_lz_row", c.m2, mode == LZ_SQR ? "sqr" : mode == LZ_MULN ? "muln" : "gen", planes);
@@ -875,23 +851,29 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
 
 static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
   const bool wide = c.m1 >= 10;
-  const uint32_t S = 1u << c.m1, T = S / (wide ? 32u : 16u);
+  const uint32_t S = 1u << c.m1, T = S / (wide ? 32u : 16u), n2 = uint32_t(c.n >> c.m1);
   uint32_t C = col_cols_default(c.m1, c.pl.LN);
   if (c.sched_cols != 0 && !wide) C = c.sched_cols;  // checked by annie_hip_set_schedule
   if (wide && C != 8u) return fail(ANNIE_ERR_SIZE, "column pass geometry");
   A.cols = int(C);
-  const dim3 grid(uint32_t(c.n >> c.m1) / C, unsigned(c.nslots), unsigned(planes)), block(C * T);
+  // From 2^10 on the planes go with the column groups (lz_tile in lazy.hip, in
+  // units of four groups over eight XCDs: n2 >= 2^10 columns are whole units).
+  if (wide && n2 % 256u != 0) return fail(ANNIE_ERR_SIZE, "column pass geometry");
+  A.planes = planes;
+  const dim3 grid(n2 / C * (wide ? unsigned(planes) : 1u), unsigned(c.nslots), wide ? 1u : unsigned(planes)), block(C * T);
   const size_t shm = size_t(wide ? C : C + 1) * S * 4;
   LzKernel f = nullptr;
-  switch (c.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
-#define LZ_CASE(M)                                  \
-  case M * 4: f = k_lz_coli<M>; break;              \
-  case M * 4 + 2: f = k_lz_colf<M, 2>; break;       \
-  case M * 4 + 3: f = k_lz_colf<M, 3>; break;
-    LZ_CASE(7)
-    LZ_CASE(8)
-    LZ_CASE(9)
-    LZ_CASE(10)
+  switch (100 * lz_width(lz_set(c.pl.LN)) + c.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
+#define LZ_CASE(M, W)                                        \
+  case 100 * W + M * 4: f = k_lz_coli<M, W>; break;          \
+  case 100 * W + M * 4 + 2: f = k_lz_colf<M, 2, W>; break;   \
+  case 100 * W + M * 4 + 3: f = k_lz_colf<M, 3, W>; break;
+    LZ_CASE(7, 0)
+    LZ_CASE(8, 0)
+    LZ_CASE(9, 0)
+    LZ_CASE(10, 0)
+    LZ_CASE(10, 1)
+    LZ_CASE(11, 2)
 #undef LZ_CASE
     default: return fail(ANNIE_ERR_SIZE, "no column kernel for this length");
   }
@@ -942,13 +924,19 @@ static int lz_carry(Ctx& c, LzCarry& A, bool cyc) {
   A.cbits = c.pl.cbits();
   A.cbits_slot = c.cbits_dev;
   ProfScope ps(c, cyc ? "k_lz_carryR" : "k_lz_carryQ", c.pl.K, nullptr, 1);
-  switch (c.pl.K * 2 + (cyc ? 1 : 0)) {
-    case 7: hipLaunchKernelGGL((k_lz_carry<6, 6, 5, 2, false>), grid, block, 0, c.stream, A); break;
-    case 6: hipLaunchKernelGGL((k_lz_carry<4, 4, 3, 2, true>), grid, block, 0, c.stream, A); break;
-    case 9: hipLaunchKernelGGL((k_lz_carry<7, 7, 4, 2, false>), grid, block, 0, c.stream, A); break;
-    case 8: hipLaunchKernelGGL((k_lz_carry<5, 5, 3, 2, true>), grid, block, 0, c.stream, A); break;
-    case 11: hipLaunchKernelGGL((k_lz_carry<9, 8, 4, 3, false>), grid, block, 0, c.stream, A); break;
-    case 10: hipLaunchKernelGGL((k_lz_carry<6, 6, 3, 3, true>), grid, block, 0, c.stream, A); break;
+  switch (10 * lz_set(c.pl.LN) + c.pl.K * 2 + (cyc ? 1 : 0) - 6) {
+#define LZ_CASE(SET)                                                                                                  \
+  case 10 * SET + 1: hipLaunchKernelGGL((k_lz_carry<SET, 6, 6, 5, 2, false>), grid, block, 0, c.stream, A); break; \
+  case 10 * SET + 0: hipLaunchKernelGGL((k_lz_carry<SET, 4, 4, 3, 2, true>), grid, block, 0, c.stream, A); break;  \
+  case 10 * SET + 3: hipLaunchKernelGGL((k_lz_carry<SET, 7, 7, 4, 2, false>), grid, block, 0, c.stream, A); break; \
+  case 10 * SET + 2: hipLaunchKernelGGL((k_lz_carry<SET, 5, 5, 3, 2, true>), grid, block, 0, c.stream, A); break;  \
+  case 10 * SET + 5: hipLaunchKernelGGL((k_lz_carry<SET, 9, 8, 4, 3, false>), grid, block, 0, c.stream, A); break; \
+  case 10 * SET + 4: hipLaunchKernelGGL((k_lz_carry<SET, 6, 6, 3, 3, true>), grid, block, 0, c.stream, A); break;
+    LZ_CASE(0)
+    LZ_CASE(1)
+    LZ_CASE(2)
+    LZ_CASE(3)
+#undef LZ_CASE
     default: return fail(ANNIE_ERR_SIZE, "no carry kernel for this RNS size");
   }
   HIPCHK(hipGetLastError());
@@ -985,7 +973,7 @@ static int lz_product(Ctx& c, const LzBufs& B, int mode, int op, const LzMult& m
   A.op = op;
   A.mul = mul;
   if ((rc = lz_transform(c, A, mode, 0, KR + KQ, KR))) return rc;
-  LzCarry& R = c.lz.cr;
+  LzCarry R{};
   R.src = B.wr;
   R.dst = B.mp;
   R.neg = B.neg;
@@ -996,7 +984,7 @@ static int lz_product(Ctx& c, const LzBufs& B, int mode, int op, const LzMult& m
   A.wq = B.mq;
   A.tq = B.wq;
   if ((rc = lz_transform(c, A, LZ_MULN, KR, KQ, KQ))) return rc;
-  LzCarry& Q = c.lz.cq;
+  LzCarry Q{};
   Q.src = B.mq;
   Q.dst = B.y;
   Q.dst2 = (snap != nullptr || snapbits != nullptr) ? c.lzreg(LZ_SNAP) : nullptr;
@@ -2094,7 +2082,7 @@ int annie_hip_batch_bytes(int K, int LN, size_t* per_slot, size_t* fixed) {
     // The larger of the two paths' slots; the short primes' root tables beyond
     // `fixed` count with the slots, of which a batch has at least one.
     size_t words = size_t(NREG) * size_t(K) * n + 2 * size_t(DIGIT_LIMBS) * n;
-    if (K >= 3 && LN >= 8 && LN <= 20) {
+    if (K >= 3 && LN >= 8 && LN <= LZ_MAX_LN) {
       const LzShape sh = lz_shape(K);
       words = std::max(words, lz_slot_words(K, n) + (2 * size_t(sh.KR + sh.KQ) - 4 * size_t(K)) * n);
     }

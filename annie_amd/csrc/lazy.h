@@ -13,8 +13,8 @@
 // inverse transform and the carry of T_Q out (src/transformGPU.h:523-568 does
 // each product on its own).
 //
-// The primes are below 2^28.2, so that a signed 32-bit word holds +-6.9 p and
-// a butterfly needs no correction: see lazy.hip.  More planes (7 + 5 instead of
+// The primes are below 2^28.2 (slightly wider above 2^20), so that a signed
+// 32-bit word holds +-6.9 p and a butterfly needs no correction: see lazy.hip.  More planes (7 + 5 instead of
 // 4 per transform at K = 4) and fewer transforms come to 29 plane transforms a
 // squaring instead of 32, each at half the instructions, in four launches
 // (lengths up to 2^13) or eight instead of six or twelve.
@@ -22,8 +22,8 @@
 // Measured against the passes over the long primes, one squaring: 2^10 (K =
 // 4) 43.9 -> 16.8 us, 2^13 61.7 -> 31.5, 2^14 (K = 5) 77.4 -> 35.5, 2^16 78.7
 // -> 41.7, 2^19 154 -> 101; one tick of a batch: 130 slots of 2^12 138 -> 89,
-// 300 slots of 2^9 (K = 5) 124 -> 82, nine of 2^13 71 -> 39.  Lengths above
-// 2^20 have too few such primes and stay on the long ones.
+// 300 slots of 2^9 (K = 5) 124 -> 82, nine of 2^13 71 -> 39.  2^23 has
+// too few such primes and stays on the long ones.
 #pragma once
 #include <cmath>
 #include <cstddef>
@@ -38,7 +38,21 @@ namespace annie {
 constexpr int LZ_MAXP = 9;     // prime planes of a transform
 constexpr int LZ_MAXL = 8;     // 32-bit limbs of a CRT value
 constexpr uint32_t LZ_MAX_A = 4095;  // largest multiplier that the carries have room for
-constexpr double LZ_LOG2_P = 28.2;   // the primes are below 2^28.2 and above 2^27
+constexpr int LZ_MAX_LN = 22;
+
+// The primes, k 2^e + 1: set 0 (e = 20, below 2^28.2) serves lengths up to 2^19,
+// sets 1 - 3 (e = 21, 22, 23, below 2^28.2, 2^29.3, 2^29.9) 2^20 - 2^22: the
+// negacyclic transform needs 2^{LN + 1}-th roots of unity, and these are the
+// largest such primes below the fewest bits that leave enough of them.  Fixed
+// sets make the CRT's constants instruction literals.
+constexpr int LZ_SETS = 4;
+constexpr uint32_t LZ_K[LZ_SETS][LZ_MAXP] = {{291, 277, 262, 258, 246, 238, 235, 220, 211},
+                                             {131, 129, 123, 119, 110, 101, 95, 89, 81},
+                                             {154, 142, 112, 99, 90, 55, 40, 39, 37},
+                                             {119, 107, 105, 90, 77, 71, 56, 45, 20}};
+constexpr int lz_set(int LN) { return LN <= 19 ? 0 : LN - 19; }
+constexpr int lz_width(int set) { return set <= 1 ? 0 : set - 1; }  // W in lazy.hip
+constexpr uint32_t lz_prime(int set, int k) { return (LZ_K[set][k] << (20 + set)) + 1u; }
 
 // Planes and limbs of RNS size K of the plan (K = 3, 4, 5).
 struct LzShape {
@@ -94,18 +108,13 @@ struct LzNtt {
   const uint32_t* neg;                        // first pass over m': its sign (null: x is no m')
   const uint32_t* slot_ids;
   size_t slot_stride;
-  int LN, m1, KR, pl0, cols, op;
+  int LN, m1, KR, pl0, planes, cols, op;
   int32_t scale[LZ_MAXP];                     // LZ_FWD: scale of each prime's planes (0: none)
   LzMult mul;
 };
 
-// CRT of KP planes and carry.  V = sum y_i M_i - round(sum y_i / p_i) P with
-// y_i = r_i c_i mod p_i, M_i = P / p_i, c_i = M_i^-1 mod p_i.
+// CRT of the planes and carry.
 struct LzCarry {
-  uint32_t p[LZ_MAXP], q[LZ_MAXP];
-  int32_t c[LZ_MAXP];
-  float inv[LZ_MAXP];
-  uint32_t M[LZ_MAXP][LZ_MAXL], NP[LZ_MAXL];  // M_i; -P mod 2^{32 L}
   const uint32_t* src;                        // planes
   uint32_t* dst;                              // digits
   uint32_t* dst2;                             // snapshot of flagged positions, or null
@@ -136,35 +145,58 @@ struct LzPack {
   const uint32_t* cbits_slot;
 };
 
-// The transform primes of length 2^LN: the largest primes k 2^e + 1 below
-// 2^28.2, e = max(LN + 1, 16) (the negacyclic transform needs 2^{LN + 1}-th
-// roots of unity).
-static inline bool lz_is_prime(uint32_t n) {
-  if (n < 4) return n > 1;
-  uint32_t d = n - 1, s = 0;
-  while (!(d & 1u)) d >>= 1, ++s;
-  for (uint32_t a : {2u, 3u, 5u, 7u}) {  // deterministic below 3,215,031,751
-    uint32_t x = powmod_plain(a, d, n);
-    if (x == 1 || x == n - 1) continue;
-    bool comp = true;
-    for (uint32_t r = 1; r < s && comp; ++r) {
-      x = mulmod_plain(x, x, n);
-      if (x == n - 1) comp = false;
-    }
-    if (comp) return false;
-  }
-  return true;
+static inline std::vector<uint32_t> lz_primes(int LN, int count) {
+  std::vector<uint32_t> out;
+  for (int k = 0; k < count && LN <= LZ_MAX_LN; ++k) out.push_back(lz_prime(lz_set(LN), k));
+  return out;
 }
 
-static inline std::vector<uint32_t> lz_primes(int LN, int count) {
-  const int e = LN + 1 > 16 ? LN + 1 : 16;
-  std::vector<uint32_t> out;
-  for (uint32_t k = uint32_t(std::pow(2.0, LZ_LOG2_P)) >> e; k > 0 && int(out.size()) < count; --k) {
-    const uint32_t p = (k << e) + 1;
-    if (p < (1u << 27)) break;
-    if (lz_is_prime(p)) out.push_back(p);
+// CRT constants of the first KP primes of a set, on L limbs (modulo 2^{32 L}):
+// V = sum y_i M_i - round(sum y_i / p_i) P with y_i = r_i M_i^-1 mod p_i, M_i = P /
+// p_i; c: M_i^-1 in signed Montgomery form, cq = c p^-1 mod 2^32, NP = -P.
+template <int KP, int L>
+struct LzCrt {
+  uint32_t p[KP], cq[KP], M[KP][L], NP[L];
+  int32_t c[KP];
+  float inv[KP];
+};
+
+template <int SET, int KP, int L>
+constexpr LzCrt<KP, L> lz_make_crt() {
+  LzCrt<KP, L> t{};
+  auto times = [](uint32_t (&v)[L], uint32_t m) {
+    uint64_t c = 0;
+    for (int l = 0; l < L; ++l) {
+      c += uint64_t(v[l]) * m;
+      v[l] = uint32_t(c);
+      c >>= 32;
+    }
+  };
+  uint32_t P[L] = {1};
+  for (int k = 0; k < KP; ++k) times(P, lz_prime(SET, k));
+  uint64_t borrow = 0;
+  for (int l = 0; l < L; ++l) {
+    const uint64_t v = 0 - uint64_t(P[l]) - borrow;
+    t.NP[l] = uint32_t(v);
+    borrow = (v >> 32) ? 1 : 0;
   }
-  return out;
+  for (int k = 0; k < KP; ++k) {
+    const uint32_t p = lz_prime(SET, k);
+    uint32_t M[L] = {1};
+    uint64_t r = 1;
+    for (int j = 0; j < KP; ++j)
+      if (j != k) {
+        times(M, lz_prime(SET, j));
+        r = r * lz_prime(SET, j) % p;
+      }
+    for (int l = 0; l < L; ++l) t.M[k][l] = M[l];
+    const uint32_t c = uint32_t((uint64_t(cx_powmod(uint32_t(r), uint64_t(p) - 2, p)) << 32) % p);
+    t.p[k] = p;
+    t.c[k] = c > p / 2 ? int32_t(c) - int32_t(p) : int32_t(c);
+    t.cq[k] = uint32_t(t.c[k]) * cx_inv32(p);
+    t.inv[k] = float(1.0 / double(p));
+  }
+  return t;
 }
 
 // A generator of the 2-part: g with g^((p-1)/2) = -1 (any quadratic
@@ -182,7 +214,7 @@ static inline uint32_t lz_nonresidue(uint32_t p) {
 // (1 + a) n (B/2)^2 (both by a factor 1 + 2^-20); with 0.4 bits to spare the
 // quotient sum y_i / p_i, exact to 2^-19 in single precision, rounds right.
 static inline bool lz_fits(const Plan& pl, int cbits, uint32_t a, const std::vector<uint32_t>& primes) {
-  if (pl.K < 3 || pl.K > 5 || pl.LN < 8 || pl.LN > 20 || a > LZ_MAX_A) return false;
+  if (pl.K < 3 || pl.K > 5 || pl.LN < 8 || pl.LN > LZ_MAX_LN || a > LZ_MAX_A) return false;
   const LzShape sh = lz_shape(pl.K);
   if (pl.K == 5 ? (cbits < 64 || cbits > 76) : (cbits < 34 || cbits > 59)) return false;
   if (int(primes.size()) < sh.KR) return false;

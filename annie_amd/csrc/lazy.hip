@@ -2,51 +2,68 @@
 // primes on signed, lazily reduced residues, and CRT + carry passes between
 // residues and digit registers.
 //
-// Arithmetic.  A residue is any signed 32-bit word congruent to it.  With p <
-// 2^28.2 a word holds +-6.9 p.  The Montgomery product by a constant |w| <=
-// p / 2, hi(b w) - hi(lo(b w p^-1) p), is at most p / 2 + |b| p / 2^33 <= 0.75 p
-// in magnitude for every word b, so the forward butterfly (a, b) -> (a + t,
-// a - t) takes six instructions and no correction; it grows its values by
-// 0.5-0.75 p per level, and eight levels fit between reductions.  Measured on
-// a register-resident chain (2,048 workgroups of 256): 4.9 issue slots per
+// Arithmetic.  A residue is any signed 32-bit word congruent to it.  The
+// Montgomery product by a constant |w| <= p / 2, hi(b w) - hi(lo(b w p^-1) p), is
+// at most p / 2 + |b| p / 2^33 <= 0.75 p in magnitude for every word b, so the
+// forward butterfly (a, b) -> (a + t, a - t) takes six instructions and no
+// correction while its values fit: they grow by 0.5-0.75 p per level.  Measured
+// on a register-resident chain (2,048 workgroups of 256): 4.9 issue slots per
 // butterfly against 9.4 with the corrections that primes above 2^31 need.
-// The bounds are tracked at compile time, in units of p / 256 (lz_grow,
-// lz_fwd_red, lz_group_inv), and a reduction (quotient by multiplication,
-// three instructions) is placed where a value could leave its word.
+//
+// Three sets of primes (lazy.h), W: 0 below 2^28.2 (a word holds +-6.9 p: eight
+// levels between reductions), 1 below 2^29.3 (2^21, +-3.2 p) and 2 below 2^29.9
+// (2^22, +-2.1 p), as few primes with roots of order 2^{LN + 1} are smaller at
+// the longest lengths.  W = 0 reduces by a quotient (lz_red), a whole round at a
+// time; W > 0 takes one p off by the sign (lz_cond), where a sum would not fit.
+// The bounds are tracked at compile time in units of p / 256 (lz_walk,
+// lz_round_inv).
 #include "lazy.h"
 #include "rounds.h"
 
 namespace annie {
 
-constexpr int LZ_LIM = 1766;   // 6.9 p (p < 2^28.2: 2^31 / p > 6.96)
-constexpr int LZ_RED = 264;    // a reduced value: [0, 1.03 p)
-constexpr int LZ_IN = 384;     // a digit's residue as loaded: 1.5 p
-constexpr int LZ_OUT = 410;    // what an inverse round starts from: 1.6 p
+constexpr int lz_lim(int W) { return W == 0 ? 1766 : W == 1 ? 828 : 545; }   // floor(256 2^31 / p)
+constexpr int lz_gain(int W) { return W == 0 ? 37 : W == 1 ? 80 : 121; }     // 1024 p / 2^33
+constexpr int LZ_RED = 264;                                                   // lz_red: [0, 1.03 p)
+constexpr int lz_in(int W) { return W == 0 ? 384 : 262; }                     // a digit's residue as loaded
+constexpr int lz_out(int W) { return W == 0 ? 410 : 256; }                    // what an inverse round starts from
+constexpr int lz_less(int s) { return s > 512 ? s - 256 : 256; }              // lz_cond of a value within s
 
-// Bound of a +- t for |a|, |b| <= s.
-constexpr int lz_grow(int s) { return s + 129 + s * 37 / 1024; }
-
-// Whether round I of a line of 2^M elements, starting at bound s, has to
-// reduce its elements first; lz_fwd_end: the bound after all rounds.
-constexpr int lz_fwd_walk(int M, int LR, int s, int upto, bool want_red) {
+// Forward bounds: lz_level is the bound after one level from bound s (the
+// sums' first operand is reduced when `c`), lz_level_cond whether it has to be;
+// lz_walk the bound at the start of round `upto` of a line of 2^M elements (or
+// at its end), and lz_fwd_red whether round I reduces its elements first.
+constexpr bool lz_level_cond(int W, int s) { return W > 0 && s + 129 + s * lz_gain(W) / 1024 > lz_lim(W); }
+constexpr int lz_level(int W, int s) { return (lz_level_cond(W, s) ? lz_less(s) : s) + 129 + s * lz_gain(W) / 1024; }
+constexpr int lz_levels(int W, int s, int rr) {
+  for (int l = 0; l < rr; ++l) s = lz_level(W, s);
+  return s;
+}
+constexpr int lz_walk(int W, int M, int LR, int s, int upto) {
   for (int i = 0, left = M; left > 0; ++i) {
     const int rr = left < LR ? left : LR;
     left -= rr;
-    int e = s;
-    for (int l = 0; l < rr; ++l) e = lz_grow(e);
-    const bool red = e > LZ_LIM;
-    if (red) {
-      e = LZ_RED;
-      for (int l = 0; l < rr; ++l) e = lz_grow(e);
-    }
-    if (want_red && i == upto) return red ? 1 : 0;
-    s = e;
+    if (W == 0 && lz_levels(W, s, rr) > lz_lim(W)) s = LZ_RED;
+    if (i == upto) return s;
+    s = lz_levels(W, s, rr);
   }
   return s;
 }
-constexpr bool lz_fwd_red(int M, int LR, int s, int I) { return lz_fwd_walk(M, LR, s, I, true) != 0; }
-static_assert(lz_fwd_walk(13, 3, LZ_IN, -1, false) <= LZ_LIM && lz_fwd_walk(10, 5, LZ_IN, -1, false) <= LZ_LIM &&
-                  lz_fwd_walk(10, 4, LZ_LIM, -1, false) <= LZ_LIM && lz_fwd_walk(13, 4, LZ_IN, -1, false) <= LZ_LIM,
+constexpr bool lz_fwd_red(int W, int M, int LR, int s, int I) {
+  int at = s;
+  for (int i = 0, left = M; i < I; ++i) {
+    const int rr = left < LR ? left : LR;
+    left -= rr;
+    if (W == 0 && lz_levels(W, at, rr) > lz_lim(W)) at = LZ_RED;
+    at = lz_levels(W, at, rr);
+  }
+  const int left = M - LR * I;
+  return W == 0 && lz_levels(W, at, left < LR ? left : LR) > lz_lim(W);
+}
+constexpr bool lz_safe(int W, int M, int LR, int s) { return lz_walk(W, M, LR, s, -1) <= lz_lim(W); }
+static_assert(lz_safe(0, 13, 3, lz_in(0)) && lz_safe(0, 13, 4, lz_in(0)) && lz_safe(0, 10, 5, lz_in(0)) &&
+                  lz_safe(0, 10, 4, lz_lim(0)) && lz_safe(0, 10, 3, lz_lim(0)) && lz_safe(1, 10, 5, lz_in(1)) &&
+                  lz_safe(1, 11, 4, lz_lim(1)) && lz_safe(2, 11, 5, lz_in(2)) && lz_safe(2, 11, 4, lz_lim(2)),
               "a forward line leaves its words");
 
 struct LzP {
@@ -65,12 +82,21 @@ __device__ __forceinline__ int32_t lz_red(int32_t x, const LzP& P) {
   return x - int32_t(uint32_t(__mulhi(x, int32_t(P.bar)) >> 26) * P.p);
 }
 
-template <int LR, int RR>
-__device__ __forceinline__ void lz_round_fwd(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P) {
+// x - p or x + p by the sign: within max(p, |x| - p).
+__device__ __forceinline__ uint32_t lz_cond(uint32_t x, const LzP& P) {
+  return x + (uint32_t(int32_t(x) >> 31) & (2u * P.p)) - P.p;
+}
+
+// The levels of one round from elements within s.
+template <int LR, int RR, int W>
+__device__ __forceinline__ void lz_round_fwd(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P, int s0) {
 #pragma unroll
-  for (int s = 0; s < RoundTw<LR, RR>::G; ++s)
+  for (int s = 0; s < RoundTw<LR, RR>::G; ++s) {
+    int bound = s0;
 #pragma unroll
     for (int e = 0; e < RR; ++e) {
+      const bool cond = lz_level_cond(W, bound);
+      bound = lz_level(W, bound);
       const int half = (1 << RR) >> (e + 1);
 #pragma unroll
       for (int blk = 0; blk < (1 << e); ++blk) {
@@ -80,23 +106,31 @@ __device__ __forceinline__ void lz_round_fwd(uint32_t (&x)[1 << LR], const Round
           uint32_t& a = x[s * (1 << RR) + blk * 2 * half + jj];
           uint32_t& b = x[s * (1 << RR) + blk * 2 * half + jj + half];
           const uint32_t t = uint32_t(lz_mulc(int32_t(b), int32_t(r), rq, P.p));
+          if (cond) a = lz_cond(a, P);
           b = a - t;
           a = a + t;
         }
       }
     }
+  }
 }
 
-// Inverse levels of a round; the elements start within LZ_OUT, and end there
-// too unless LAST (then within LZ_LIM).  bd: the bound of each element, a
+// Inverse levels of a round; the elements start within lz_out, and end there
+// too unless LAST (then within their words).  bd: the bound of each element, a
 // compile-time constant after unrolling.
-template <int LR, int RR, bool LAST>
+template <int W>
+__device__ __forceinline__ void lz_less_inv(uint32_t& x, int& bd, const LzP& P) {
+  if (W == 0 && bd > LZ_RED) x = uint32_t(lz_red(int32_t(x), P)), bd = LZ_RED;
+  if (W > 0 && bd > 256) x = lz_cond(x, P), bd = lz_less(bd);
+}
+
+template <int LR, int RR, int W, bool LAST>
 __device__ __forceinline__ void lz_round_inv(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P) {
 #pragma unroll
   for (int s = 0; s < RoundTw<LR, RR>::G; ++s) {
     int bd[1 << RR];
 #pragma unroll
-    for (int j = 0; j < (1 << RR); ++j) bd[j] = LZ_OUT;
+    for (int j = 0; j < (1 << RR); ++j) bd[j] = lz_out(W);
     uint32_t* v = &x[s * (1 << RR)];
 #pragma unroll
     for (int e = RR - 1; e >= 0; --e) {
@@ -107,23 +141,23 @@ __device__ __forceinline__ void lz_round_inv(uint32_t (&x)[1 << LR], const Round
 #pragma unroll
         for (int jj = 0; jj < half; ++jj) {
           const int j = blk * 2 * half + jj, i = j + half;
-          if (bd[j] + bd[i] > LZ_LIM) {
-            if (bd[j] > LZ_RED) v[j] = uint32_t(lz_red(int32_t(v[j]), P)), bd[j] = LZ_RED;
-            if (bd[i] > LZ_RED) v[i] = uint32_t(lz_red(int32_t(v[i]), P)), bd[i] = LZ_RED;
+          if (bd[j] + bd[i] > lz_lim(W)) {
+            lz_less_inv<W>(v[j], bd[j], P);
+            lz_less_inv<W>(v[i], bd[i], P);
           }
           const uint32_t d = v[j] - v[i];
           v[j] = v[j] + v[i];
           v[i] = uint32_t(lz_mulc(int32_t(d), int32_t(r), rq, P.p));
           const int sum = bd[j] + bd[i];
           bd[j] = sum;
-          bd[i] = 130 + sum * 37 / 1024;
+          bd[i] = 130 + sum * lz_gain(W) / 1024;
         }
       }
     }
     if constexpr (!LAST) {
 #pragma unroll
       for (int j = 0; j < (1 << RR); ++j)
-        if (bd[j] > LZ_OUT) v[j] = uint32_t(lz_red(int32_t(v[j]), P));
+        if (bd[j] > lz_out(W)) lz_less_inv<W>(v[j], bd[j], P);
     }
   }
 }
@@ -149,7 +183,7 @@ struct LzRoots<M, LR, (M + LR - 1) / LR> {};
 
 // Forward rounds I.. .  ROOTS: 0 each round loads its own roots (from LDS), 1
 // one round ahead (`cur` holds round I's), 2 all loaded (`all`).
-template <int M, int LR, int I, int ROOTS, int S0, class GLd, class LLd, class LSt, class Hook>
+template <int W, int M, int LR, int I, int ROOTS, int S0, class GLd, class LLd, class LSt, class Hook>
 __device__ __forceinline__ void lz_fwd(uint32_t (&x)[1 << LR], uint32_t tg, uint32_t lineRoot, const uint32_t* tw,
                                        const LzP& P, GLd& gld, LLd& lld, LSt& lst, const SchedTw<M, LR, I>& cur,
                                        const LzRoots<M, LR, 0>& all, Hook&& at_last) {
@@ -161,23 +195,24 @@ __device__ __forceinline__ void lz_fwd(uint32_t (&x)[1 << LR], uint32_t tg, uint
   if constexpr (ROOTS == 1 && !END) round_tw(nxt, M, LR * (I + 1), tg, lineRoot, tw);
   if constexpr (END) at_last();
   if constexpr (I > 0) round_load<LR, RR>(x, M, LR * I, tg, lld);
-  if constexpr (lz_fwd_red(M, LR, S0, I)) {
+  if constexpr (lz_fwd_red(W, M, LR, S0, I)) {
 #pragma unroll
     for (int i = 0; i < (1 << LR); ++i) x[i] = uint32_t(lz_red(int32_t(x[i]), P));
   }
-  if constexpr (ROOTS == 0) lz_round_fwd<LR, RR>(x, own, P);
-  else if constexpr (ROOTS == 1) lz_round_fwd<LR, RR>(x, cur, P);
-  else lz_round_fwd<LR, RR>(x, all.template get<I>(), P);
+  constexpr int S = lz_walk(W, M, LR, S0, I);
+  if constexpr (ROOTS == 0) lz_round_fwd<LR, RR, W>(x, own, P, S);
+  else if constexpr (ROOTS == 1) lz_round_fwd<LR, RR, W>(x, cur, P, S);
+  else lz_round_fwd<LR, RR, W>(x, all.template get<I>(), P, S);
   if constexpr (!END) {
     round_store<LR, RR>(x, M, LR * I, tg, lst);
     __syncthreads();
-    lz_fwd<M, LR, I + 1, ROOTS, S0>(x, tg, lineRoot, tw, P, gld, lld, lst, nxt, all, at_last);
+    lz_fwd<W, M, LR, I + 1, ROOTS, S0>(x, tg, lineRoot, tw, P, gld, lld, lst, nxt, all, at_last);
   }
 }
 
 // Inverse rounds I down to 0, from the elements of round NR - 1 in x.  FINAL:
 // the values go to a carry, which takes any word.
-template <int M, int LR, int I, int ROOTS, bool FINAL, class GSt, class LLd, class LSt>
+template <int W, int M, int LR, int I, int ROOTS, bool FINAL, class GSt, class LLd, class LSt>
 __device__ __forceinline__ void lz_inv(uint32_t (&x)[1 << LR], uint32_t tg, uint32_t lineRoot, const uint32_t* tw,
                                        const LzP& P, GSt& gst, LLd& lld, LSt& lst, const SchedTw<M, LR, I>& cur,
                                        const LzRoots<M, LR, 0>& all) {
@@ -188,13 +223,13 @@ __device__ __forceinline__ void lz_inv(uint32_t (&x)[1 << LR], uint32_t tg, uint
   if constexpr (ROOTS == 1 && I > 0) round_tw(nxt, M, LR * (I - 1), tg, lineRoot, tw);
   if constexpr (I + 1 < Sched<M, LR>::NR) round_load<LR, RR>(x, M, LR * I, tg, lld);
   constexpr bool LAST = I == 0 && FINAL;
-  if constexpr (ROOTS == 0) lz_round_inv<LR, RR, LAST>(x, own, P);
-  else if constexpr (ROOTS == 1) lz_round_inv<LR, RR, LAST>(x, cur, P);
-  else lz_round_inv<LR, RR, LAST>(x, all.template get<I>(), P);
+  if constexpr (ROOTS == 0) lz_round_inv<LR, RR, W, LAST>(x, own, P);
+  else if constexpr (ROOTS == 1) lz_round_inv<LR, RR, W, LAST>(x, cur, P);
+  else lz_round_inv<LR, RR, W, LAST>(x, all.template get<I>(), P);
   if constexpr (I > 0) {
     round_store<LR, RR>(x, M, LR * I, tg, lst);
     __syncthreads();
-    lz_inv<M, LR, I - 1, ROOTS, FINAL>(x, tg, lineRoot, tw, P, gst, lld, lst, nxt, all);
+    lz_inv<W, M, LR, I - 1, ROOTS, FINAL>(x, tg, lineRoot, tw, P, gst, lld, lst, nxt, all);
   } else {
     round_store<LR, RR>(x, M, 0, tg, gst);
   }
@@ -233,13 +268,13 @@ constexpr int lz_row_threads(int M, int LR) { return (1 << M >> LR) > 512 || (1 
 // Grid: (rows / lines, slots, planes), so that the cyclic planes, which go
 // forward and back, start before the negacyclic ones, which only go forward
 // here; block: lines of 2^M / 2^LR threads.
-template <int M, int LR, int MODE, int SRC>
+template <int M, int LR, int MODE, int SRC, int W>
 __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A) {
   extern __shared__ uint32_t lds[];
   constexpr uint32_t S = 1u << M, T = S >> LR;
   constexpr int NR = Sched<M, LR>::NR, RL = Sched<M, LR>::template rr<NR - 1>();
   constexpr int ROOTS = LR <= 3 ? 2 : 1;
-  constexpr int S0 = SRC ? LZ_IN : LZ_LIM;
+  constexpr int S0 = SRC ? lz_in(W) : lz_lim(W);
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
   const int pl = A.pl0 + int(blockIdx.z);
@@ -295,7 +330,7 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
       for (int e = 0; e < (1 << LR); ++e) oy[e] = ld_w(o, uint32_t(e) * T + tg);
     }
   };
-  lz_fwd<M, LR, 0, ROOTS, S0>(x, tg, lineRoot, twf, P, gld, lld, lst, t0, rf, prefetch);
+  lz_fwd<W, M, LR, 0, ROOTS, S0>(x, tg, lineRoot, twf, P, gld, lld, lst, t0, rf, prefetch);
 
   if constexpr (MODE == LZ_GEN) {
     if (A.op == LZ_MULY) {
@@ -311,14 +346,16 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
 #pragma unroll
     for (int e = 0; e < (1 << LR); ++e) {
       if constexpr (MODE == LZ_MULN) {
+        // Within 0.88 p + 0.72 p.
         x[e] = uint32_t(lz_mul(int32_t(x[e]), int32_t(op[e]), P)) - oy[e];
+        if constexpr (W > 0) x[e] = lz_cond(x[e], P);
       } else {
         const int32_t y = MODE == LZ_SQR ? int32_t(x[e]) : int32_t(oy[e]);
         x[e] = uint32_t(lz_mul(lz_mul(int32_t(x[e]), y, P), int32_t(op[e]), P));
       }
     }
     // Single-pass values go to the carry; a column pass follows otherwise.
-    lz_inv<M, LR, NR - 1, ROOTS, SRC != 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
+    lz_inv<W, M, LR, NR - 1, ROOTS, SRC != 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
   } else {
     int32_t c = A.scale[k];
     if (MODE == LZ_SQR || A.op != LZ_FWD) {
@@ -342,18 +379,36 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
 }
 
 // Column passes of lengths from 2^14 on: the first M = m1 levels on columns of
-// stride n2 = n / 2^M, A.cols (8 for M = 10) consecutive columns per block,
+// stride n2 = n / 2^M, A.cols (8 for M >= 10) consecutive columns per block,
 // interleaved and XOR-swizzled in LDS as the passes over the long primes.
-// Forward reads digits, so that the planes of one column group share them.
+// Grid: (column groups, slots, planes); from 2^10 on (column groups x planes,
+// slots): a unit of four column groups covers whole 128-byte lines and goes to
+// one XCD (id mod 8) with all its planes in turn, so that the digits are read
+// from memory once for all planes (25 MB instead of 15 times that at 2^21).
 template <int M>
 struct LzCol {
   static constexpr int LR = (M >= 10) ? 5 : 4;
   static constexpr bool LDS_ROOTS = (LR == 4);
-  static constexpr int THREADS = (M >= 10) ? 256 : 1024;
+  static constexpr int THREADS = (M >= 10) ? (8 << (M - LR)) : 1024;
   static constexpr int WAVES = (M >= 10) ? 4 : 4;
 };
 
-template <int M, int DL>
+struct LzTile {
+  int pl;
+  uint32_t col0;
+};
+template <int M>
+__device__ __forceinline__ LzTile lz_tile(const LzNtt& A, uint32_t C) {
+  if constexpr (M < 10) {
+    return {A.pl0 + int(blockIdx.z), col_group(C) * C};
+  } else {
+    const uint32_t per = 4u * uint32_t(A.planes), t = blockIdx.x >> 3;
+    const uint32_t unit = (t / per) * 8u + (blockIdx.x & 7u), r = t % per;
+    return {A.pl0 + int(r >> 2), (unit * 4u + (r & 3u)) * C};
+  }
+}
+
+template <int M, int DL, int W>
 __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(const LzNtt A) {
   extern __shared__ uint32_t lds[];
   constexpr int LR = LzCol<M>::LR;
@@ -361,13 +416,14 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
-  const int pl = A.pl0 + int(blockIdx.z);
+  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const LzTile tile = lz_tile<M>(A, C);
+  const int pl = tile.pl;
   const bool cyc = pl < A.KR;
   const int k = cyc ? pl : pl - A.KR;
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
-  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
   const uint32_t line = threadIdx.x % C, tg = threadIdx.x / C;
-  const uint32_t n2 = uint32_t(n >> M), col0 = col_group(C) * C;
+  const uint32_t n2 = uint32_t(n >> M), col0 = tile.col0;
   uint32_t* dst = (cyc ? A.wr : A.wq) + so + size_t(k) * n + col0;
   const uint32_t* twf = (cyc ? A.fwdR : A.fwdQ) + size_t(k) * n;
   const uint32_t* xd = A.x + so;
@@ -377,10 +433,12 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
   auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
 
+  // Roots of 2^10 one round ahead from the table; 2^11 would spill.
+  constexpr int ROOTS = M == 10 ? 1 : 0;
   uint32_t x[1 << LR];
   LzRoots<M, LR, 0> none;
   SchedTw<M, LR, 0> t0;
-  if constexpr (!LzCol<M>::LDS_ROOTS) round_tw(t0, M, 0, tg, 1u, twf);
+  if constexpr (ROOTS == 1) round_tw(t0, M, 0, tg, 1u, twf);
   round_load<LR, Sched<M, LR>::template rr<0>()>(x, M, 0, tg, gld);
   if (A.neg != nullptr && threadIdx.x == 0u && col0 == 0u && A.neg[so] == 0u)
     x[0] = uint32_t(lz_red(int32_t(x[0] + 2u * uint32_t(A.c.one[k])), P));  // m' + 2, as in k_lz_row
@@ -388,28 +446,29 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
     uint32_t* roots = lds + C * S;
     for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twf[i];
     __syncthreads();
-    lz_fwd<M, LR, 0, 0, LZ_IN>(x, tg, 1u, roots, P, gld, lld, lst, t0, none, [] {});
+    lz_fwd<W, M, LR, 0, 0, lz_in(W)>(x, tg, 1u, roots, P, gld, lld, lst, t0, none, [] {});
   } else {
-    lz_fwd<M, LR, 0, 1, LZ_IN>(x, tg, 1u, twf, P, gld, lld, lst, t0, none, [] {});
+    lz_fwd<W, M, LR, 0, ROOTS, lz_in(W)>(x, tg, 1u, twf, P, gld, lld, lst, t0, none, [] {});
   }
   round_store<LR, RL>(x, M, DLV, tg, gst);
 }
 
-template <int M>
+template <int M, int W>
 __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(const LzNtt A) {
   extern __shared__ uint32_t lds[];
   constexpr int LR = LzCol<M>::LR;
   constexpr uint32_t S = 1u << M;
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
   const size_t so = size_t(lz_slot(A.slot_ids, blockIdx.y)) * A.slot_stride, n = size_t(1) << A.LN;
-  const int pl = A.pl0 + int(blockIdx.z);
+  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const LzTile tile = lz_tile<M>(A, C);
+  const int pl = tile.pl;
   const bool cyc = pl < A.KR;
   const int k = cyc ? pl : pl - A.KR;
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
-  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
   const uint32_t line = threadIdx.x % C, tg = threadIdx.x / C;
   const uint32_t n2 = uint32_t(n >> M);
-  uint32_t* w = (cyc ? A.wr : A.wq) + so + size_t(k) * n + size_t(col_group(C)) * C;
+  uint32_t* w = (cyc ? A.wr : A.wq) + so + size_t(k) * n + tile.col0;
   const uint32_t* twi = (cyc ? A.invR : A.invQ) + size_t(k) * n;
 
   auto gld = [&](uint32_t i) { return w[line + i * n2]; };
@@ -417,6 +476,8 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(
   auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
   auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
 
+  // Roots of 2^10 one round ahead from the table; 2^11 would spill.
+  constexpr int ROOTS = M == 10 ? 1 : 0;
   uint32_t x[1 << LR];
   LzRoots<M, LR, 0> none;
   SchedTw<M, LR, NR - 1> ti;
@@ -425,10 +486,10 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(
     uint32_t* roots = lds + C * S;
     for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twi[i];
     __syncthreads();
-    lz_inv<M, LR, NR - 1, 0, true>(x, tg, 1u, roots, P, gst, lld, lst, ti, none);
+    lz_inv<W, M, LR, NR - 1, 0, true>(x, tg, 1u, roots, P, gst, lld, lst, ti, none);
   } else {
-    round_tw(ti, M, DLV, tg, 1u, twi);
-    lz_inv<M, LR, NR - 1, 1, true>(x, tg, 1u, twi, P, gst, lld, lst, ti, none);
+    if constexpr (ROOTS == 1) round_tw(ti, M, DLV, tg, 1u, twi);
+    lz_inv<W, M, LR, NR - 1, ROOTS, true>(x, tg, 1u, twi, P, gst, lld, lst, ti, none);
   }
 }
 
@@ -563,40 +624,57 @@ __device__ __forceinline__ LzDig<DL> lz_finish(uint32_t (&v)[LZ_MAXL], uint32_t 
   return lz_add(s, lz_small(s, c));
 }
 
-// The coefficient as two's complement limbs.  The products of column l are
-// below 9 2^(28.2 + 32) < 2^63.4, so 64-bit sums hold them.
-template <int KP, int L>
-__device__ __forceinline__ void lz_crt(const LzCarry& A, const uint32_t* src, size_t n, uint32_t i, uint32_t (&v)[LZ_MAXL]) {
-  uint64_t col[L];
+// The coefficient as two's complement limbs.  Column l sums KP products below p
+// 2^32: 9 2^(28.2 + 32) < 2^63.4 for the shortest primes; with the wider ones
+// (WIDE) the sums are kept in two halves of at most five products, below
+// 2^64.
+template <int SET, int KP, int L>
+__device__ __forceinline__ void lz_crt(const uint32_t* src, size_t n, uint32_t i, uint32_t (&v)[LZ_MAXL]) {
+  constexpr LzCrt<KP, L> C = lz_make_crt<SET, KP, L>();
+  constexpr bool WIDE = lz_width(SET) > 0;
+  constexpr int H = WIDE ? 4 : KP;  // products of the first half: 4 2^(29.9 + 32) < 2^64
+  uint64_t col[L], cob[WIDE ? L : 1];
 #pragma unroll
   for (int l = 0; l < L; ++l) col[l] = 0;
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int l = 0; l < L; ++l) cob[l] = 0;
+  }
   float f = 0.5f;
   int32_t r[KP];
 #pragma unroll
   for (int k = 0; k < KP; ++k) r[k] = int32_t(ld_w(src + size_t(k) * n, i));
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
-    int32_t y = lz_mulc(r[k], A.c[k], uint32_t(A.c[k]) * A.q[k], A.p[k]);
-    y += (y >> 31) & int32_t(A.p[k]);
-    f += float(y) * A.inv[k];
+    int32_t y = lz_mulc(r[k], C.c[k], C.cq[k], C.p[k]);
+    y += (y >> 31) & int32_t(C.p[k]);
+    f += float(y) * C.inv[k];
 #pragma unroll
-    for (int l = 0; l < L; ++l) col[l] += uint64_t(uint32_t(y)) * A.M[k][l];
+    for (int l = 0; l < L; ++l) {
+      if (k < H) col[l] += uint64_t(uint32_t(y)) * C.M[k][l];
+      else cob[WIDE ? l : 0] += uint64_t(uint32_t(y)) * C.M[k][l];
+    }
   }
   const uint32_t q = uint32_t(f);
   uint64_t t = 0;
 #pragma unroll
   for (int l = 0; l < L; ++l) {
-    t += col[l];
-    const uint64_t u = uint64_t(q) * A.NP[l];
-    // col + carry < 2^63.5 and q NP < 2^36: no overflow.
-    t += u;
-    v[l] = uint32_t(t);
-    t >>= 32;
+    if constexpr (WIDE) {
+      const uint64_t lo = (col[l] & 0xffffffffull) + (cob[l] & 0xffffffffull) + (t & 0xffffffffull) + uint64_t(q) * C.NP[l];
+      v[l] = uint32_t(lo);
+      t = (col[l] >> 32) + (cob[l] >> 32) + (t >> 32) + (lo >> 32);
+    } else {
+      // col + carry < 2^63.5 and q NP < 2^36: no overflow.
+      t += col[l];
+      t += uint64_t(q) * C.NP[l];
+      v[l] = uint32_t(t);
+      t >>= 32;
+    }
   }
 }
 
 // Grid: (ceil(waves / 4), slots); block 256.
-template <int KP, int L, int ND, int DL, bool NEGA>
+template <int SET, int KP, int L, int ND, int DL, bool NEGA>
 __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   constexpr int W = 64 - ND;
   const size_t n = size_t(1) << A.LN;
@@ -618,7 +696,7 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
     const int i = w * W + lane - ND;
     const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
     uint32_t v[LZ_MAXL];
-    lz_crt<KP, L>(A, A.src + so, n, idx, v);
+    lz_crt<SET, KP, L>(A.src + so, n, idx, v);
     if (a != 1u) {
       uint64_t t = 0;
 #pragma unroll
@@ -790,45 +868,54 @@ __global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* 
 
 // Instantiations, looked up by the host engine.  Eight elements per thread
 // (LR = 3) for short launches, sixteen where they fill the GPU.
-#define LZ_ROW(M, LR, SRC)                                             \
-  template __global__ void k_lz_row<M, LR, LZ_SQR, SRC>(const LzNtt);  \
-  template __global__ void k_lz_row<M, LR, LZ_MULN, SRC>(const LzNtt); \
-  template __global__ void k_lz_row<M, LR, LZ_GEN, SRC>(const LzNtt);
-#define LZ_ROW1(M)  \
-  LZ_ROW(M, 3, 2) \
-  LZ_ROW(M, 3, 3) \
-  LZ_ROW(M, 4, 2) \
-  LZ_ROW(M, 4, 3)
+#define LZ_ROW(M, LR, SRC, W)                                             \
+  template __global__ void k_lz_row<M, LR, LZ_SQR, SRC, W>(const LzNtt);  \
+  template __global__ void k_lz_row<M, LR, LZ_MULN, SRC, W>(const LzNtt); \
+  template __global__ void k_lz_row<M, LR, LZ_GEN, SRC, W>(const LzNtt);
+#define LZ_ROW1(M)   \
+  LZ_ROW(M, 3, 2, 0) \
+  LZ_ROW(M, 3, 3, 0) \
+  LZ_ROW(M, 4, 2, 0) \
+  LZ_ROW(M, 4, 3, 0)
 LZ_ROW1(8)
 LZ_ROW1(9)
 LZ_ROW1(10)
 LZ_ROW1(11)
 LZ_ROW1(12)
 LZ_ROW1(13)
-#define LZ_ROW2(M) LZ_ROW(M, 3, 0) LZ_ROW(M, 4, 0)
+#define LZ_ROW2(M) LZ_ROW(M, 3, 0, 0) LZ_ROW(M, 4, 0, 0)
 LZ_ROW2(7)
 LZ_ROW2(8)
 LZ_ROW2(9)
 LZ_ROW2(10)
-#define LZ_COL(M)                                          \
-  template __global__ void k_lz_colf<M, 2>(const LzNtt);   \
-  template __global__ void k_lz_colf<M, 3>(const LzNtt);   \
-  template __global__ void k_lz_coli<M>(const LzNtt);
-LZ_COL(7)
-LZ_COL(8)
-LZ_COL(9)
-LZ_COL(10)
-template __global__ void k_lz_carry<6, 6, 5, 2, false>(const LzCarry);
-template __global__ void k_lz_carry<4, 4, 3, 2, true>(const LzCarry);
-template __global__ void k_lz_carry<7, 7, 4, 2, false>(const LzCarry);
-template __global__ void k_lz_carry<5, 5, 3, 2, true>(const LzCarry);
-template __global__ void k_lz_carry<9, 8, 4, 3, false>(const LzCarry);
-template __global__ void k_lz_carry<6, 6, 3, 3, true>(const LzCarry);
+LZ_ROW(11, 4, 0, 1)
+LZ_ROW(11, 4, 0, 2)
+#define LZ_COL(M, W)                                          \
+  template __global__ void k_lz_colf<M, 2, W>(const LzNtt);   \
+  template __global__ void k_lz_colf<M, 3, W>(const LzNtt);   \
+  template __global__ void k_lz_coli<M, W>(const LzNtt);
+LZ_COL(7, 0)
+LZ_COL(8, 0)
+LZ_COL(9, 0)
+LZ_COL(10, 0)
+LZ_COL(10, 1)
+LZ_COL(11, 2)
+#define LZ_CARRY(SET)                                                            \
+  template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true>(const LzCarry);  \
+  template __global__ void k_lz_carry<SET, 7, 7, 4, 2, false>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true>(const LzCarry);  \
+  template __global__ void k_lz_carry<SET, 9, 8, 4, 3, false>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true>(const LzCarry);
+LZ_CARRY(0)
+LZ_CARRY(1)
+LZ_CARRY(2)
+LZ_CARRY(3)
+template __global__ void k_lz_pack<2>(const LzPack);
+template __global__ void k_lz_pack<3>(const LzPack);
 #define LZ_CONV(K, DL)                                        \
   template __global__ void k_lz_import<K, DL>(const LzConv);  \
   template __global__ void k_lz_export<K, DL>(const LzConv);
-template __global__ void k_lz_pack<2>(const LzPack);
-template __global__ void k_lz_pack<3>(const LzPack);
 LZ_CONV(3, 2)
 LZ_CONV(4, 2)
 LZ_CONV(5, 3)

@@ -17,9 +17,10 @@ pytestmark = pytest.mark.gpu
 P = [(125 << 25) + 1, (243 << 24) + 1, (235 << 24) + 1, (29 << 27) + 1, (13 << 28) + 1]
 
 # Bits of N: K = 3, 4, 5 at the single-pass lengths 2^8 .. 2^13 and the two-pass
-# lengths from 2^14 (seven column levels) to 2^20 (ten).
+# lengths from 2^14 (seven column levels) to 2^20 (ten); the wider primes of
+# 2^21 and 2^22.
 SIZES = [10000, 13000, 17500, 38000, 55000, 70000, 200000, 324619, 430000, 560000, 1000003, 3100000, 8600000, 27000000,
-         50000000, 60000000]
+         50000000, 60000000, 100000000, 130000000, 200000000, 250000000]
 
 
 def _words(x, t):
