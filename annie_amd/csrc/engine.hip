@@ -40,13 +40,13 @@ __global__ void k_copy_slots(uint32_t* base, size_t dst_off, size_t src_off, siz
                              size_t slot_stride);
 template <int M, int K, int QS>
 __global__ void k_sqr_run(const RunArgs R);
-template <int M, int LR, int MODE, int SRC, int W>
+template <int M, int LR, int MODE, int SRC, int W, int SP>
 __global__ void k_lz_row(const LzNtt A);
 template <int M, int DL, int W>
 __global__ void k_lz_colf(const LzNtt A);
 template <int M, int W>
 __global__ void k_lz_coli(const LzNtt A);
-template <int SET, int KP, int L, int ND, int DL, bool NEGA>
+template <int SET, int KP, int L, int ND, int DL, bool NEGA, int SP>
 __global__ void k_lz_carry(const LzCarry A);
 __global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
 template <int DL>
@@ -116,6 +116,9 @@ struct Lazy {
   bool on = false;
   LzShape sh{};
   int LR = 3;  // log2 of the elements per thread of the row passes
+  // Levels of the column passes (0: single-pass), or of a single-pass transform
+  // split over 2^sp workgroups, and of the rows.
+  int m1 = 0, sp = 0, m2 = 0;
   std::vector<uint32_t> primes;
   LzPrimes pc{};
   int32_t scaleR[LZ_MAXP] = {}, scaleQ[LZ_MAXP] = {};  // of the transforms of N^-1 mod R and N
@@ -718,15 +721,19 @@ static int scale_reg(Ctx& c, int r, size_t slot = 0) {
 // ---------------------------------------------------------------------------
 // The short-prime path (lazy.h): products of digit registers.
 
-// Whether a class of plans (one K, LN and digit-width class; the digit width
-// and the base vary with N and a) runs on the short-prime path: its widest
-// digits have to fit.  A context whose multipliers or digits turn out not to
-// fit is demoted to the long primes.
-static bool lz_class_fits(const Plan& pl) {
+// ANNIE_LONG_PRIMES=1 keeps every context on the long primes.
+static bool lz_wanted() {
   const char* off = std::getenv("ANNIE_LONG_PRIMES");
-  if (off && off[0] == '1') return false;
-  if (pl.K < 3 || pl.LN < 8 || pl.LN > LZ_MAX_LN) return false;
-  double lp = -1.0;
+  return !(off && off[0] == '1');
+}
+
+// Whether a class of plans (one K, LN and digit-width class; the digit width
+// and the base a >= 2 vary with N) runs on the short-prime path: its widest
+// digits have to fit.  A batch whose multipliers or digits turn out not to fit
+// is demoted to the long primes.
+static bool lz_class_fits(const Plan& pl) {
+  if (!lz_wanted() || pl.K < 3 || pl.LN < 8 || pl.LN > LZ_MAX_LN) return false;
+  double lp = -2.0;
   for (int k = 0; k < pl.K; ++k) lp += std::log2(double(PRIMES[k]));
   int cb = pl.cbits();
   for (int b = cb + pl.pck; (b >> 5) == (pl.cbits() >> 5) && pl.LN + 2 * b < lp; b += pl.pck) cb = b;
@@ -741,11 +748,26 @@ static size_t lz_slot_words(int K, size_t n) {
 
 static int32_t lz_signed(uint64_t v, uint32_t p) { return v > p / 2 ? int32_t(v) - int32_t(p) : int32_t(v); }
 
-static int lz_elements(const Ctx& c) {
-  if (const char* e = std::getenv("ANNIE_LZ_LR")) return std::atoi(e);
-  // Lines of 2^9 and shorter would leave half a wave idle at sixteen.
-  const int M = c.pl.LN <= 13 ? c.pl.LN : c.pl.LN - c.pl.LN / 2;
-  return (c.nslots_alloc << c.pl.LN) >= (size_t(1) << 17) && M >= 10 ? 4 : 3;
+// Geometry of the transforms.  A launch of few slots leaves most CUs idle and is
+// bound by the chain of one workgroup, so the transform is split over two or
+// four workgroups (lz_branch, lz_join in lazy.hip) while their number is small;
+// the lines are drawn where both sides measured equal.  us per squaring, not
+// split / two / four: 2^12, one slot 20.0 / 18.1 / 20.1, 16 slots 28.4 / 27.3 /
+// 33.7; 2^13, one slot 30.4 / 22.1 / 22.3, 24 slots 50.2 / 46.8 / 52.1, 40 slots
+// (sixteen elements per thread) 65.0 / 67.9 / 75.3; 2^14 in two passes / four,
+// one slot 32.5 / 31.3 (K = 5), 31.8 / 27.6 (K = 4), 24 slots 85 / 79, 40 slots
+// 121 / 129; 2^11 and 2^15 are no faster split.
+static void lz_geometry(Ctx& c) {
+  Lazy& z = c.lz;
+  const int LN = c.pl.LN;
+  const size_t slots = c.nslots_alloc;
+  z.sp = (LN == 12 && slots <= 16) || (LN == 13 && slots <= 32) ? 1 : (LN == 14 && slots <= 32) ? 2 : 0;
+  z.m1 = z.sp > 0 ? 0 : c.m1;
+  z.m2 = LN - z.m1 - z.sp;
+  // Sixteen elements per thread where the launch fills the GPU (fewer LDS
+  // exchanges), eight where it leaves CUs idle (shorter chains per thread), in
+  // split transforms and in lines of 2^9 and shorter (half a wave would idle).
+  z.LR = z.sp == 0 && z.m2 >= 10 && (slots << LN) >= (size_t(1) << 17) ? 4 : 3;
 }
 
 static int lz_setup(Ctx& c) {
@@ -755,9 +777,7 @@ static int lz_setup(Ctx& c) {
   z.sh = lz_shape(K);
   z.primes = lz_primes(LN, z.sh.KR);
   const int KR = z.sh.KR, KQ = z.sh.KQ, DL = z.sh.DL;
-  // Sixteen elements per thread where the launch fills the GPU (fewer LDS
-  // exchanges), eight where it leaves CUs idle (shorter chains per thread).
-  z.LR = lz_elements(c);
+  lz_geometry(c);
   z.stride = lz_slot_words(K, n);
   z.plane0 = size_t(NLZ) * size_t(DL) * n;
   if (hipMalloc(&z.mem, c.nslots_alloc * z.stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
@@ -799,33 +819,37 @@ static int lz_setup(Ctx& c) {
 
 typedef void (*LzKernel)(const LzNtt);
 
-template <int M, int LR, int SRC, int W>
+template <int M, int LR, int SRC, int W, int SP>
 static LzKernel lz_row_mode(int mode) {
-  return mode == LZ_SQR    ? k_lz_row<M, LR, LZ_SQR, SRC, W>
-         : mode == LZ_MULN ? k_lz_row<M, LR, LZ_MULN, SRC, W>
-                           : k_lz_row<M, LR, LZ_GEN, SRC, W>;
+  return mode == LZ_SQR    ? k_lz_row<M, LR, LZ_SQR, SRC, W, SP>
+         : mode == LZ_MULN ? k_lz_row<M, LR, LZ_MULN, SRC, W, SP>
+                           : k_lz_row<M, LR, LZ_GEN, SRC, W, SP>;
 }
 template <int M, int SRC>
 static LzKernel lz_row_kernel(int LR, int mode) {
-  return LR == 3 ? lz_row_mode<M, 3, SRC, 0>(mode) : lz_row_mode<M, 4, SRC, 0>(mode);
+  return LR == 3 ? lz_row_mode<M, 3, SRC, 0, 0>(mode) : lz_row_mode<M, 4, SRC, 0, 0>(mode);
+}
+template <int M, int SRC>
+static LzKernel lz_split_kernel(int sp, int mode) {
+  return sp == 1 ? lz_row_mode<M, 3, SRC, 0, 1>(mode) : lz_row_mode<M, 3, SRC, 0, 2>(mode);
 }
 
 // Rows of planes [A.pl0, A.pl0 + planes): the whole transform of a digit
 // register (single-pass lengths), or the row levels of planes in place.
 static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
   const Lazy& z = c.lz;
-  const bool single = c.m1 == 0;
-  const uint32_t S = 1u << c.m2, T = S >> z.LR, rows = 1u << c.m1;
+  const bool single = z.m1 == 0;
+  const uint32_t S = 1u << z.m2, T = S >> z.LR, rows = 1u << (z.m1 + z.sp);
   uint32_t lines = 1;
   if (T < 64 && !single) {
-    lines = row_lines_default(c.m1, c.m2);
+    lines = row_lines_default(z.m1, z.m2);
     if (c.sched_lines != 0) lines = c.sched_lines;  // checked by annie_hip_set_schedule
   }
   A.cols = int(lines);
   const dim3 grid(rows / lines, unsigned(c.nslots), unsigned(planes)), block(lines * T);
   const size_t shm = size_t(lines) * (S + (S >> 5)) * 4;
   LzKernel f = nullptr;
-  switch (single ? 100 * z.sh.DL + c.m2 : c.m2) {
+  switch ((single ? 100 * z.sh.DL + (z.sp > 0 ? 1000 : 0) : 0) + z.m2) {
 #define LZ_CASE1(M)                                           \
   case 200 + M: f = lz_row_kernel<M, 2>(z.LR, mode); break; \
   case 300 + M: f = lz_row_kernel<M, 3>(z.LR, mode); break;
@@ -836,23 +860,31 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
     LZ_CASE1(12)
     LZ_CASE1(13)
 #undef LZ_CASE1
+#define LZ_CASES(M)                                            \
+  case 1200 + M: f = lz_split_kernel<M, 2>(z.sp, mode); break; \
+  case 1300 + M: f = lz_split_kernel<M, 3>(z.sp, mode); break;
+    LZ_CASES(10)
+    LZ_CASES(11)
+    LZ_CASES(12)
+    LZ_CASES(13)
+#undef LZ_CASES
     case 7: f = lz_row_kernel<7, 0>(z.LR, mode); break;
     case 8: f = lz_row_kernel<8, 0>(z.LR, mode); break;
     case 9: f = lz_row_kernel<9, 0>(z.LR, mode); break;
     case 10: f = lz_row_kernel<10, 0>(z.LR, mode); break;
-    case 11: f = lz_width(lz_set(c.pl.LN)) == 1 ? lz_row_mode<11, 4, 0, 1>(mode) : lz_row_mode<11, 4, 0, 2>(mode); break;
+    case 11: f = lz_width(lz_set(c.pl.LN)) == 1 ? lz_row_mode<11, 4, 0, 1, 0>(mode) : lz_row_mode<11, 4, 0, 2, 0>(mode); break;
     default: return fail(ANNIE_ERR_SIZE, "no row kernel for this length");
   }
-  ProfScope ps(c, "k_lz_row", c.m2, mode == LZ_SQR ? "sqr" : mode == LZ_MULN ? "muln" : "gen", planes);
+  ProfScope ps(c, "k_lz_row", z.m2, mode == LZ_SQR ? "sqr" : mode == LZ_MULN ? "muln" : "gen", planes);
   hipLaunchKernelGGL(f, grid, block, shm, c.stream, A);
   HIPCHK(hipGetLastError());
   return ANNIE_OK;
 }
 
 static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
-  const bool wide = c.m1 >= 10;
-  const uint32_t S = 1u << c.m1, T = S / (wide ? 32u : 16u), n2 = uint32_t(c.n >> c.m1);
-  uint32_t C = col_cols_default(c.m1, c.pl.LN);
+  const bool wide = c.lz.m1 >= 10;
+  const uint32_t S = 1u << c.lz.m1, T = S / (wide ? 32u : 16u), n2 = uint32_t(c.n >> c.lz.m1);
+  uint32_t C = col_cols_default(c.lz.m1, c.pl.LN);
   if (c.sched_cols != 0 && !wide) C = c.sched_cols;  // checked by annie_hip_set_schedule
   if (wide && C != 8u) return fail(ANNIE_ERR_SIZE, "column pass geometry");
   A.cols = int(C);
@@ -863,7 +895,7 @@ static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
   const dim3 grid(n2 / C * (wide ? unsigned(planes) : 1u), unsigned(c.nslots), wide ? 1u : unsigned(planes)), block(C * T);
   const size_t shm = size_t(wide ? C : C + 1) * S * 4;
   LzKernel f = nullptr;
-  switch (100 * lz_width(lz_set(c.pl.LN)) + c.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
+  switch (100 * lz_width(lz_set(c.pl.LN)) + c.lz.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
 #define LZ_CASE(M, W)                                        \
   case 100 * W + M * 4: f = k_lz_coli<M, W>; break;          \
   case 100 * W + M * 4 + 2: f = k_lz_colf<M, 2, W>; break;   \
@@ -877,7 +909,7 @@ static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
 #undef LZ_CASE
     default: return fail(ANNIE_ERR_SIZE, "no column kernel for this length");
   }
-  ProfScope ps(c, inverse ? "k_lz_coli" : "k_lz_colf", c.m1, nullptr, planes);
+  ProfScope ps(c, inverse ? "k_lz_coli" : "k_lz_colf", c.lz.m1, nullptr, planes);
   hipLaunchKernelGGL(f, grid, block, shm, c.stream, A);
   HIPCHK(hipGetLastError());
   return ANNIE_OK;
@@ -888,9 +920,9 @@ static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
 static int lz_transform(Ctx& c, LzNtt& A, int mode, int pl0, int planes, int back) {
   int rc;
   A.pl0 = pl0;
-  if (c.m1 > 0 && (rc = lz_col(c, A, false, planes))) return rc;
+  if (c.lz.m1 > 0 && (rc = lz_col(c, A, false, planes))) return rc;
   if ((rc = lz_row(c, A, mode, planes))) return rc;
-  if (c.m1 > 0 && back > 0 && (rc = lz_col(c, A, true, back))) return rc;
+  if (c.lz.m1 > 0 && back > 0 && (rc = lz_col(c, A, true, back))) return rc;
   return ANNIE_OK;
 }
 
@@ -908,7 +940,7 @@ static LzNtt lz_args(const Ctx& c) {
   A.slot_ids = c.slot_ids;
   A.slot_stride = z.stride;
   A.LN = c.pl.LN;
-  A.m1 = c.m1;
+  A.m1 = z.m1;
   A.KR = z.sh.KR;
   A.mul.a = 1u;
   return A;
@@ -924,19 +956,25 @@ static int lz_carry(Ctx& c, LzCarry& A, bool cyc) {
   A.cbits = c.pl.cbits();
   A.cbits_slot = c.cbits_dev;
   ProfScope ps(c, cyc ? "k_lz_carryR" : "k_lz_carryQ", c.pl.K, nullptr, 1);
-  switch (10 * lz_set(c.pl.LN) + c.pl.K * 2 + (cyc ? 1 : 0) - 6) {
-#define LZ_CASE(SET)                                                                                                  \
-  case 10 * SET + 1: hipLaunchKernelGGL((k_lz_carry<SET, 6, 6, 5, 2, false>), grid, block, 0, c.stream, A); break; \
-  case 10 * SET + 0: hipLaunchKernelGGL((k_lz_carry<SET, 4, 4, 3, 2, true>), grid, block, 0, c.stream, A); break;  \
-  case 10 * SET + 3: hipLaunchKernelGGL((k_lz_carry<SET, 7, 7, 4, 2, false>), grid, block, 0, c.stream, A); break; \
-  case 10 * SET + 2: hipLaunchKernelGGL((k_lz_carry<SET, 5, 5, 3, 2, true>), grid, block, 0, c.stream, A); break;  \
-  case 10 * SET + 5: hipLaunchKernelGGL((k_lz_carry<SET, 9, 8, 4, 3, false>), grid, block, 0, c.stream, A); break; \
-  case 10 * SET + 4: hipLaunchKernelGGL((k_lz_carry<SET, 6, 6, 3, 3, true>), grid, block, 0, c.stream, A); break;
-    LZ_CASE(0)
-    LZ_CASE(1)
-    LZ_CASE(2)
-    LZ_CASE(3)
+  A.twi = c.lz.tw + (cyc ? size_t(c.lz.sh.KR) : 2 * size_t(c.lz.sh.KR) + size_t(c.lz.sh.KQ)) * c.n;
+  switch (100 * c.lz.sp + 10 * lz_set(c.pl.LN) + c.pl.K * 2 + (cyc ? 1 : 0) - 6) {
+#define LZ_CASE1(ID, SET, SP, ...) \
+  case 100 * SP + 10 * SET + ID: hipLaunchKernelGGL((k_lz_carry<SET, __VA_ARGS__, SP>), grid, block, 0, c.stream, A); break;
+#define LZ_CASE(SET, SP)                     \
+  LZ_CASE1(1, SET, SP, 6, 6, 5, 2, false) \
+  LZ_CASE1(0, SET, SP, 4, 4, 3, 2, true)  \
+  LZ_CASE1(3, SET, SP, 7, 7, 4, 2, false) \
+  LZ_CASE1(2, SET, SP, 5, 5, 3, 2, true)  \
+  LZ_CASE1(5, SET, SP, 9, 8, 4, 3, false) \
+  LZ_CASE1(4, SET, SP, 6, 6, 3, 3, true)
+    LZ_CASE(0, 0)
+    LZ_CASE(0, 1)
+    LZ_CASE(0, 2)
+    LZ_CASE(1, 0)
+    LZ_CASE(2, 0)
+    LZ_CASE(3, 0)
 #undef LZ_CASE
+#undef LZ_CASE1
     default: return fail(ANNIE_ERR_SIZE, "no carry kernel for this RNS size");
   }
   HIPCHK(hipGetLastError());
@@ -1243,7 +1281,7 @@ static int setup_long(Ctx& c) {
 
 // Device state shared by the slots of a context: stream, and the register
 // files, roots and kernel constants of `slots` slots of the path it takes.
-static int setup_device(Ctx& c, int device, size_t slots, bool want_lazy) {
+static int setup_device(Ctx& c, int device, size_t slots, bool lazy) {
   c.n = c.pl.n();
   c.m1 = (c.pl.LN <= 13) ? 0 : c.pl.LN / 2;
   c.m2 = c.pl.LN - c.m1;
@@ -1269,7 +1307,7 @@ static int setup_device(Ctx& c, int device, size_t slots, bool want_lazy) {
   c.nslots_alloc = slots;
   c.nbase.LN = c.cbase.LN = c.pl.LN;
   c.cbase.cbits = c.pl.cbits();
-  return (want_lazy && lz_class_fits(c.pl)) ? lz_setup(c) : setup_long(c);
+  return lazy ? lz_setup(c) : setup_long(c);
 }
 
 // Per-modulus constants of one slot: N_Q, the negacyclic transform of N, and
@@ -1534,7 +1572,7 @@ static int create(const uint64_t* Nl, size_t nl, int32_t a, int device, int min_
     return ANNIE_INIT_FAILED;
   }
   int rc;
-  if ((rc = setup_device(c, device, 1, lz_fits(c.pl, c.pl.cbits(), uint32_t(a), lz_primes(c.pl.LN, LZ_MAXP))))) return rc;
+  if ((rc = setup_device(c, device, 1, lz_wanted() && lz_fits(c.pl, c.pl.cbits(), uint32_t(a), lz_primes(c.pl.LN, LZ_MAXP))))) return rc;
   if ((rc = load_slot_consts(c, 0, c.N, t))) return rc;
   *out = h.release();
   return ANNIE_OK;
@@ -2050,7 +2088,7 @@ int annie_hip_batch_create(int K, int pck, int LN, int lbase, size_t slots, int 
   c.pl.LN = LN;
   c.pl.lbase = lbase;
   int rc;
-  if ((rc = setup_device(c, device, slots, true))) return rc;
+  if ((rc = setup_device(c, device, slots, lz_class_fits(c.pl)))) return rc;
   c.slotN.resize(slots);
   c.slot_cb.assign(slots, c.pl.cbits());
   c.slot_base.assign(slots, 1u);

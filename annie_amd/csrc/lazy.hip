@@ -249,12 +249,52 @@ __device__ __forceinline__ int32_t lz_digit(const uint32_t* x, size_t n, uint32_
   return int32_t(h - (br ? 1u : 0u) - __umulhi(lo * P.q, P.p));
 }
 
-__device__ __forceinline__ uint32_t lz_slot(const uint32_t* ids, uint32_t pos) { return ids ? ids[pos] : 0u; }
+__device__ __forceinline__ uint32_t lz_slot(const uint32_t* ids, uint32_t pos) {
+  return ids ? uint32_t(__builtin_amdgcn_readfirstlane(int(ids[pos]))) : 0u;
+}
+
+// Kernel arguments that a kernel needs in any case, read together at its
+// start: left to itself the compiler loads each one where a branch first
+// needs it, and the round trips follow one another (a dozen in the carry, a
+// quarter of its time at the shortest lengths).
+template <class T>
+__device__ __forceinline__ void lz_pin1(const T v) {
+  asm volatile("" : : "s"(v));
+}
+template <class... T>
+__device__ __forceinline__ void lz_pin(const T... v) {
+  (lz_pin1(v), ...);
+}
 
 __device__ __forceinline__ uint32_t lz_multiplier(const LzMult& m, uint32_t pos, uint32_t slot) {
   if (m.a_slot != nullptr) return m.a_slot[pos] & ~SLOT_SNAP;
   if (m.bits_mode == 1) return ((m.bits[pos >> 5] >> (pos & 31u)) & 1u) ? m.slot_base[slot] : 1u;
   return m.a;
+}
+
+// A transform of length 2^LN split over 2^SP workgroups (SP = LN - M > 0, the
+// single-pass kernels of short launches): workgroup `row` computes the node of
+// level SP it owns straight from the digits, position i of it from the 2^SP
+// digits i + t 2^M, so that no column pass and no exchange come before it; the
+// carry undoes those levels as it loads (lz_join).  Position i from digits x_t:
+// level 0 pairs t and t + 2^{SP - 1} with root r(0, 0), and so on; the sign of
+// each level's root is the branch that leads to `row`.  Within 1.5 p + 0.8 p SP.
+constexpr int lz_split_in(int SP) { return lz_in(0) + 205 * SP; }
+struct LzBranch {
+  int32_t r[2];
+  uint32_t rq[2];
+};
+template <int SP>
+__device__ __forceinline__ LzBranch lz_branch(const uint32_t* twf, uint32_t row, const LzP& P) {
+  LzBranch b{};
+#pragma unroll
+  for (int l = 0; l < SP; ++l) {
+    const uint32_t node = row >> (SP - l);
+    const int32_t r = int32_t(twf[(1u << l) + node]);
+    b.r[l] = ((row >> (SP - 1 - l)) & 1u) ? -r : r;
+    b.rq[l] = uint32_t(b.r[l]) * P.q;
+  }
+  return b;
 }
 
 // Lines of fewer than 64 threads run several to a block, up to 1,024 threads.
@@ -268,13 +308,15 @@ constexpr int lz_row_threads(int M, int LR) { return (1 << M >> LR) > 512 || (1 
 // Grid: (rows / lines, slots, planes), so that the cyclic planes, which go
 // forward and back, start before the negacyclic ones, which only go forward
 // here; block: lines of 2^M / 2^LR threads.
-template <int M, int LR, int MODE, int SRC, int W>
+template <int M, int LR, int MODE, int SRC, int W, int SP>
 __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A) {
   extern __shared__ uint32_t lds[];
   constexpr uint32_t S = 1u << M, T = S >> LR;
   constexpr int NR = Sched<M, LR>::NR, RL = Sched<M, LR>::template rr<NR - 1>();
   constexpr int ROOTS = LR <= 3 ? 2 : 1;
-  constexpr int S0 = SRC ? lz_in(W) : lz_lim(W);
+  lz_pin(A.slot_ids, A.slot_stride, A.LN, A.KR, A.pl0, A.x, A.wr, A.wq, A.fwdR, A.invR, A.fwdQ, A.invQ, A.nir, A.nq, A.tq, A.neg);
+  constexpr int S0 = SRC == 0 ? lz_lim(W) : SP > 0 ? lz_split_in(SP) : lz_in(W);
+  static_assert(lz_safe(W, M, LR, S0), "a forward line leaves its words");
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
   const int pl = A.pl0 + int(blockIdx.z);
@@ -283,17 +325,31 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
   const LzP P{A.c.p[k], A.c.q[k], A.c.bar[k]};
   constexpr bool ONE = T >= 64;
   const uint32_t line = ONE ? 0u : threadIdx.x / T, tg = ONE ? threadIdx.x : threadIdx.x % T;
-  const uint32_t row = SRC ? 0u : (ONE ? blockIdx.x : blockIdx.x * uint32_t(A.cols) + line);
-  const uint32_t lineRoot = SRC ? 1u : (1u << A.m1) + row;
+  const uint32_t row = (SRC && SP == 0) ? 0u : (ONE || SRC) ? blockIdx.x : blockIdx.x * uint32_t(A.cols) + line;
+  const uint32_t lineRoot = SRC ? (1u << SP) + row : (1u << A.m1) + row;
   const size_t base = so + size_t(k) * n + size_t(row) * S;
   uint32_t* X = lds + line * (S + (S >> 5));
   uint32_t* w = (cyc ? A.wr : A.wq) + base;
   const uint32_t* twf = (cyc ? A.fwdR : A.fwdQ) + size_t(k) * n;
   const uint32_t* twi = (cyc ? A.invR : A.invQ) + size_t(k) * n;
 
+  const LzBranch br = lz_branch<SP>(twf, row, P);
   auto gld = [&](uint32_t i) {
-    if constexpr (SRC == 0) return ld_w(w, i);
-    else return uint32_t(lz_digit<SRC>(A.x + so, n, i, P));
+    if constexpr (SRC == 0) {
+      return ld_w(w, i);
+    } else if constexpr (SP == 0) {
+      return uint32_t(lz_digit<SRC>(A.x + so, n, i, P));
+    } else {
+      int32_t d[1 << SP];
+#pragma unroll
+      for (int t = 0; t < (1 << SP); ++t) d[t] = lz_digit<SRC>(A.x + so, n, i + uint32_t(t) * S, P);
+#pragma unroll
+      for (int l = 0; l < SP; ++l)
+#pragma unroll
+        for (int t = 0; t < (1 << SP >> (l + 1)); ++t)
+          d[t] += lz_mulc(d[t + (1 << SP >> (l + 1))], br.r[l], br.rq[l], P.p);
+      return uint32_t(d[0]);
+    }
   };
   auto gst = [&](uint32_t i, uint32_t v) { st_w(w, i, v); };
   auto lld = [&](uint32_t i) { return X[lpad(i)]; };
@@ -354,8 +410,9 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
         x[e] = uint32_t(lz_mul(lz_mul(int32_t(x[e]), y, P), int32_t(op[e]), P));
       }
     }
-    // Single-pass values go to the carry; a column pass follows otherwise.
-    lz_inv<W, M, LR, NR - 1, ROOTS, SRC != 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
+    // Single-pass values go to the carry; a column pass or lz_join follows
+    // otherwise.
+    lz_inv<W, M, LR, NR - 1, ROOTS, SRC != 0 && SP == 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
   } else {
     int32_t c = A.scale[k];
     if (MODE == LZ_SQR || A.op != LZ_FWD) {
@@ -629,7 +686,7 @@ __device__ __forceinline__ LzDig<DL> lz_finish(uint32_t (&v)[LZ_MAXL], uint32_t 
 // (WIDE) the sums are kept in two halves of at most five products, below
 // 2^64.
 template <int SET, int KP, int L>
-__device__ __forceinline__ void lz_crt(const uint32_t* src, size_t n, uint32_t i, uint32_t (&v)[LZ_MAXL]) {
+__device__ __forceinline__ void lz_crt(const int32_t (&r)[KP], uint32_t (&v)[LZ_MAXL]) {
   constexpr LzCrt<KP, L> C = lz_make_crt<SET, KP, L>();
   constexpr bool WIDE = lz_width(SET) > 0;
   constexpr int H = WIDE ? 4 : KP;  // products of the first half: 4 2^(29.9 + 32) < 2^64
@@ -641,9 +698,6 @@ __device__ __forceinline__ void lz_crt(const uint32_t* src, size_t n, uint32_t i
     for (int l = 0; l < L; ++l) cob[l] = 0;
   }
   float f = 0.5f;
-  int32_t r[KP];
-#pragma unroll
-  for (int k = 0; k < KP; ++k) r[k] = int32_t(ld_w(src + size_t(k) * n, i));
 #pragma unroll
   for (int k = 0; k < KP; ++k) {
     int32_t y = lz_mulc(r[k], C.c[k], C.cq[k], C.p[k]);
@@ -673,10 +727,46 @@ __device__ __forceinline__ void lz_crt(const uint32_t* src, size_t n, uint32_t i
   }
 }
 
+// Residue of a plane at coefficient i: the word itself, or, after a transform
+// split over 2^SP workgroups, its last SP inverse levels: coefficient t 2^M + j
+// from the values y_b of position j (each within 1.6 p, so four sum up in a
+// word).  Both branches of a level are one product, by the root or by 1 (one:
+// 2^32 mod p), so that waves across a boundary take no detour; the roots are
+// entries 1 .. 3 of the plane's table, uniform loads.
+template <int SP>
+__device__ __forceinline__ int32_t lz_join(const uint32_t* src, uint32_t i, int LN, const uint32_t* twi, uint32_t q, uint32_t p,
+                                           int32_t one) {
+  if constexpr (SP == 0) {
+    return int32_t(ld_w(src, i));
+  } else {
+    const int M = LN - SP;
+    const uint32_t t = i >> M, j = i & ((1u << M) - 1u);
+    const uint4 w = *reinterpret_cast<const uint4*>(twi);
+    const uint32_t root[4] = {w.x, w.y, w.z, w.w};
+    int32_t y[1 << SP];
+#pragma unroll
+    for (int b = 0; b < (1 << SP); ++b) y[b] = int32_t(ld_w(src, j + (uint32_t(b) << M)));
+#pragma unroll
+    for (int l = SP - 1; l >= 0; --l) {
+      const bool odd = ((t >> (SP - 1 - l)) & 1u) != 0u;
+#pragma unroll
+      for (int b = 0; b < (1 << l); ++b) {
+        const int32_t r0 = int32_t(root[(1 << l) + b]);
+        const int32_t r = odd ? r0 : one;
+        const uint32_t rq = odd ? uint32_t(r0) * q : uint32_t(one) * q;
+        y[b] = lz_mulc(y[2 * b] + (odd ? -y[2 * b + 1] : y[2 * b + 1]), r, rq, p);
+      }
+    }
+    return y[0];
+  }
+}
+
 // Grid: (ceil(waves / 4), slots); block 256.
-template <int SET, int KP, int L, int ND, int DL, bool NEGA>
+template <int SET, int KP, int L, int ND, int DL, bool NEGA, int SP>
 __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   constexpr int W = 64 - ND;
+  lz_pin(A.src, A.dst, A.dst2, A.neg, A.slot_ids, A.slot_stride, A.LN, A.cbits, A.cbits_slot, A.snap, A.mul.a, A.mul.a_slot,
+         A.mul.bits_mode, A.mul.slot_base, A.mul.bits[blockIdx.y >> 5 & (INLINE_SLOTS / 32 - 1)]);
   const size_t n = size_t(1) << A.LN;
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride;
@@ -689,14 +779,19 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
                              : (A.mul.bits_mode == 2 && ((A.mul.bits[blockIdx.y >> 5] >> (blockIdx.y & 31u)) & 1u));
   }
   const int lane = int(threadIdx.x & 63u);
-  const int wave = int(blockIdx.x * 4u + (threadIdx.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * 4u + (threadIdx.x >> 6)));
   const int top = int((n - 1) / W);
   if (wave > top) return;
   for (int w = wave;; --w) {
     const int i = w * W + lane - ND;
     const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
+    int32_t r[KP];
+#pragma unroll
+    for (int k = 0; k < KP; ++k)
+      r[k] = lz_join<SP>(A.src + so + size_t(k) * n, idx, A.LN, A.twi + size_t(k) * n, cx_inv32(lz_prime(SET, k)),
+                         lz_prime(SET, k), int32_t((uint64_t(1) << 32) % lz_prime(SET, k)));
     uint32_t v[LZ_MAXL];
-    lz_crt<SET, KP, L>(A.src + so, n, idx, v);
+    lz_crt<SET, KP, L>(r, v);
     if (a != 1u) {
       uint64_t t = 0;
 #pragma unroll
@@ -868,28 +963,37 @@ __global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* 
 
 // Instantiations, looked up by the host engine.  Eight elements per thread
 // (LR = 3) for short launches, sixteen where they fill the GPU.
-#define LZ_ROW(M, LR, SRC, W)                                             \
-  template __global__ void k_lz_row<M, LR, LZ_SQR, SRC, W>(const LzNtt);  \
-  template __global__ void k_lz_row<M, LR, LZ_MULN, SRC, W>(const LzNtt); \
-  template __global__ void k_lz_row<M, LR, LZ_GEN, SRC, W>(const LzNtt);
-#define LZ_ROW1(M)   \
-  LZ_ROW(M, 3, 2, 0) \
-  LZ_ROW(M, 3, 3, 0) \
-  LZ_ROW(M, 4, 2, 0) \
-  LZ_ROW(M, 4, 3, 0)
+#define LZ_ROW(M, LR, SRC, W, SP)                                             \
+  template __global__ void k_lz_row<M, LR, LZ_SQR, SRC, W, SP>(const LzNtt);  \
+  template __global__ void k_lz_row<M, LR, LZ_MULN, SRC, W, SP>(const LzNtt); \
+  template __global__ void k_lz_row<M, LR, LZ_GEN, SRC, W, SP>(const LzNtt);
+#define LZ_ROW1(M)      \
+  LZ_ROW(M, 3, 2, 0, 0) \
+  LZ_ROW(M, 3, 3, 0, 0) \
+  LZ_ROW(M, 4, 2, 0, 0) \
+  LZ_ROW(M, 4, 3, 0, 0)
 LZ_ROW1(8)
 LZ_ROW1(9)
 LZ_ROW1(10)
 LZ_ROW1(11)
 LZ_ROW1(12)
 LZ_ROW1(13)
-#define LZ_ROW2(M) LZ_ROW(M, 3, 0, 0) LZ_ROW(M, 4, 0, 0)
+#define LZ_ROWS(M)      \
+  LZ_ROW(M, 3, 2, 0, 1) \
+  LZ_ROW(M, 3, 3, 0, 1) \
+  LZ_ROW(M, 3, 2, 0, 2) \
+  LZ_ROW(M, 3, 3, 0, 2)
+LZ_ROWS(10)
+LZ_ROWS(11)
+LZ_ROWS(12)
+LZ_ROWS(13)
+#define LZ_ROW2(M) LZ_ROW(M, 3, 0, 0, 0) LZ_ROW(M, 4, 0, 0, 0)
 LZ_ROW2(7)
 LZ_ROW2(8)
 LZ_ROW2(9)
 LZ_ROW2(10)
-LZ_ROW(11, 4, 0, 1)
-LZ_ROW(11, 4, 0, 2)
+LZ_ROW(11, 4, 0, 1, 0)
+LZ_ROW(11, 4, 0, 2, 0)
 #define LZ_COL(M, W)                                          \
   template __global__ void k_lz_colf<M, 2, W>(const LzNtt);   \
   template __global__ void k_lz_colf<M, 3, W>(const LzNtt);   \
@@ -900,17 +1004,19 @@ LZ_COL(9, 0)
 LZ_COL(10, 0)
 LZ_COL(10, 1)
 LZ_COL(11, 2)
-#define LZ_CARRY(SET)                                                            \
-  template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true>(const LzCarry);  \
-  template __global__ void k_lz_carry<SET, 7, 7, 4, 2, false>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true>(const LzCarry);  \
-  template __global__ void k_lz_carry<SET, 9, 8, 4, 3, false>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true>(const LzCarry);
-LZ_CARRY(0)
-LZ_CARRY(1)
-LZ_CARRY(2)
-LZ_CARRY(3)
+#define LZ_CARRY(SET, SP)                                                         \
+  template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true, SP>(const LzCarry);  \
+  template __global__ void k_lz_carry<SET, 7, 7, 4, 2, false, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true, SP>(const LzCarry);  \
+  template __global__ void k_lz_carry<SET, 9, 8, 4, 3, false, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true, SP>(const LzCarry);
+LZ_CARRY(0, 0)
+LZ_CARRY(0, 1)
+LZ_CARRY(0, 2)
+LZ_CARRY(1, 0)
+LZ_CARRY(2, 0)
+LZ_CARRY(3, 0)
 template __global__ void k_lz_pack<2>(const LzPack);
 template __global__ void k_lz_pack<3>(const LzPack);
 #define LZ_CONV(K, DL)                                        \

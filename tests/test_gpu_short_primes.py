@@ -19,7 +19,7 @@ P = [(125 << 25) + 1, (243 << 24) + 1, (235 << 24) + 1, (29 << 27) + 1, (13 << 2
 # Bits of N: K = 3, 4, 5 at the single-pass lengths 2^8 .. 2^13 and the two-pass
 # lengths from 2^14 (seven column levels) to 2^20 (ten); the wider primes of
 # 2^21 and 2^22.
-SIZES = [10000, 13000, 17500, 38000, 55000, 70000, 200000, 324619, 430000, 560000, 1000003, 3100000, 8600000, 27000000,
+SIZES = [10000, 13000, 17500, 38000, 55000, 70000, 200000, 324619, 430000, 560000, 1000003, 3100000, 8600000, 12000000, 27000000,
          50000000, 60000000, 100000000, 130000000, 200000000, 250000000]
 
 
@@ -167,5 +167,58 @@ def test_large_multiplier_moves_to_long_primes(gpu):
         got = [int.from_bytes(out[s].tobytes(), "little") for s in range(2)]
         assert got[0] == pow(pow(3, 4, Ns[0]) * big, 2, Ns[0])
         assert got[1] == pow(3, 13, Ns[1])
+    finally:
+        lib.annie_hip_destroy(h)
+
+
+# Batches on both sides of each rule of the transforms' geometry: split over two
+# or four workgroups, one workgroup of eight or sixteen elements per thread.
+@pytest.mark.parametrize("bits,slots", [(20000, 300), (50000, 130), (200000, 16), (200000, 17), (200000, 40), (332000, 32),
+                                        (332000, 33), (560000, 3), (560000, 33), (1000003, 8)])
+def test_batch_geometries(gpu, bits, slots):
+    """Three moduli over all slots, squared together and one slot at a time:
+    every slot holds its power."""
+    lib = annie_amd.load_library()
+    Ns, seed = [], bits
+    while len(Ns) < 3:
+        N = usable_N(bits, seed, 3)
+        seed += 1
+        if not Ns or annie_amd.select_plan(N, 3) == annie_amd.select_plan(Ns[0], 3):
+            Ns.append(N)
+    K, pck, LN, lbase = annie_amd.select_plan(Ns[0], 3)
+    print(f"case batch bits={bits} slots={slots} K={K} LN={LN}", flush=True)
+    u32 = ctypes.c_uint32
+    h = ctypes.c_void_p()
+    assert lib.annie_hip_batch_create(K, pck, LN, lbase, slots, 0, ctypes.byref(h)) == 0, annie_amd._err(lib)
+    try:
+        for s in range(slots):
+            arr, n = annie_amd.int_to_limbs(Ns[s % 3])
+            f, nf = (ctypes.c_uint64 * (n + 1))(), ctypes.c_size_t()
+            assert lib.annie_hip_batch_load(h, s, arr, n, 3, f, n + 1, ctypes.byref(nf)) == 0, annie_amd._err(lib)
+        ids = (u32 * slots)(*range(slots))
+        rng = random.Random(slots)
+        e = [0, 0, 0]
+        assert lib.annie_hip_batch_set1(h, ids, slots) == 0
+        for _ in range(bits.bit_length() + 3):
+            b = [rng.getrandbits(1) for _ in range(3)]
+            e = [2 * x + y for x, y in zip(e, b)]
+            m = (u32 * slots)(*[3 if b[s % 3] else 1 for s in range(slots)])
+            assert lib.annie_hip_batch_square_mul(h, ids, m, slots) == 0
+        one = [slots - 1, slots // 2]  # two slots further on their own, and back by nothing
+        for s in one:
+            assert lib.annie_hip_batch_copy(h, 1, 0, (u32 * 1)(s), 1) == 0
+            assert lib.annie_hip_batch_mul(h, 1, 0, (u32 * 1)(s), 1) == 0
+        L = bits // 64 + 4
+        out = np.zeros((slots, L), dtype=np.uint64)
+        nout = (ctypes.c_size_t * slots)()
+        p64 = ctypes.POINTER(ctypes.c_uint64)
+        assert lib.annie_hip_batch_get(h, 0, ids, slots, out.ctypes.data_as(p64), L, nout) == 0
+        want = [oracle.powm(3, x, N) for x, N in zip(e, Ns)]
+        for s in range(slots):
+            assert int.from_bytes(out[s].tobytes(), "little") == want[s % 3], f"slot {s}"
+        pick = (u32 * 2)(*one)
+        assert lib.annie_hip_batch_get(h, 1, pick, 2, out.ctypes.data_as(p64), L, nout) == 0
+        for j, s in enumerate(one):
+            assert int.from_bytes(out[j].tobytes(), "little") == want[s % 3] ** 2 % Ns[s % 3], f"product of slot {s}"
     finally:
         lib.annie_hip_destroy(h)
