@@ -42,9 +42,9 @@ template <int M, int K, int QS>
 __global__ void k_sqr_run(const RunArgs R);
 template <int M, int LR, int MODE, int SRC, int W, int SP>
 __global__ void k_lz_row(const LzNtt A);
-template <int M, int DL, int W>
+template <int M, int LR, int DL, int W>
 __global__ void k_lz_colf(const LzNtt A);
-template <int M, int W>
+template <int M, int LR, int W>
 __global__ void k_lz_coli(const LzNtt A);
 template <int SET, int KP, int L, int ND, int DL, bool NEGA, int SP>
 __global__ void k_lz_carry(const LzCarry A);
@@ -119,6 +119,7 @@ struct Lazy {
   // Levels of the column passes (0: single-pass), or of a single-pass transform
   // split over 2^sp workgroups, and of the rows.
   int m1 = 0, sp = 0, m2 = 0;
+  uint32_t cols = 16;  // columns per workgroup (columns of up to 2^9)
   std::vector<uint32_t> primes;
   LzPrimes pc{};
   int32_t scaleR[LZ_MAXP] = {}, scaleQ[LZ_MAXP] = {};  // of the transforms of N^-1 mod R and N
@@ -762,12 +763,20 @@ static void lz_geometry(Ctx& c) {
   const int LN = c.pl.LN;
   const size_t slots = c.nslots_alloc;
   z.sp = (LN == 12 && slots <= 16) || (LN == 13 && slots <= 32) ? 1 : (LN == 14 && slots <= 32) ? 2 : 0;
-  z.m1 = z.sp > 0 ? 0 : c.m1;
+  // Short columns and long rows: a row keeps its 2^m2 elements in LDS for the
+  // forward and the inverse levels, a column pass goes through memory twice.
+  // us per squaring with m1 = LN / 2 / as here: 2^16 (8 / 7 columns levels) 37.3 /
+  // 35.6, 2^18 (9 / 8) 70.9 / 64.3, 2^19 (9 / 8) 95.1 / 86.5, 2^20 (10 / 8) 149.5 /
+  // 140.9, 2^22 (11 / 10) 737 / 627; 2^17 at 7 instead of 8 50.3 / 46.0, 2^22 at 9
+  // instead of 10 705 / 627.
+  z.m1 = z.sp > 0 || LN <= 13 ? 0 : LN <= 16 ? 7 : LN <= 20 ? 8 : 10;
   z.m2 = LN - z.m1 - z.sp;
+  z.cols = LN == 20 ? 32 : 16;
   // Sixteen elements per thread where the launch fills the GPU (fewer LDS
   // exchanges), eight where it leaves CUs idle (shorter chains per thread), in
-  // split transforms and in lines of 2^9 and shorter (half a wave would idle).
-  z.LR = z.sp == 0 && z.m2 >= 10 && (slots << LN) >= (size_t(1) << 17) ? 4 : 3;
+  // split transforms, in lines of 2^9 and shorter (half a wave would idle) and at
+  // 2^19 (86.5 against 89.2 us).
+  z.LR = z.sp == 0 && z.m2 >= 10 && LN != 19 && (slots << LN) >= (size_t(1) << 17) ? 4 : 3;
 }
 
 static int lz_setup(Ctx& c) {
@@ -825,15 +834,6 @@ static LzKernel lz_row_mode(int mode) {
          : mode == LZ_MULN ? k_lz_row<M, LR, LZ_MULN, SRC, W, SP>
                            : k_lz_row<M, LR, LZ_GEN, SRC, W, SP>;
 }
-template <int M, int SRC>
-static LzKernel lz_row_kernel(int LR, int mode) {
-  return LR == 3 ? lz_row_mode<M, 3, SRC, 0, 0>(mode) : lz_row_mode<M, 4, SRC, 0, 0>(mode);
-}
-template <int M, int SRC>
-static LzKernel lz_split_kernel(int sp, int mode) {
-  return sp == 1 ? lz_row_mode<M, 3, SRC, 0, 1>(mode) : lz_row_mode<M, 3, SRC, 0, 2>(mode);
-}
-
 // Rows of planes [A.pl0, A.pl0 + planes): the whole transform of a digit
 // register (single-pass lengths), or the row levels of planes in place.
 static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
@@ -849,30 +849,33 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
   const dim3 grid(rows / lines, unsigned(c.nslots), unsigned(planes)), block(lines * T);
   const size_t shm = size_t(lines) * (S + (S >> 5)) * 4;
   LzKernel f = nullptr;
-  switch ((single ? 100 * z.sh.DL + (z.sp > 0 ? 1000 : 0) : 0) + z.m2) {
-#define LZ_CASE1(M)                                           \
-  case 200 + M: f = lz_row_kernel<M, 2>(z.LR, mode); break; \
-  case 300 + M: f = lz_row_kernel<M, 3>(z.LR, mode); break;
-    LZ_CASE1(8)
-    LZ_CASE1(9)
-    LZ_CASE1(10)
-    LZ_CASE1(11)
-    LZ_CASE1(12)
-    LZ_CASE1(13)
+  const int W = lz_width(lz_set(c.pl.LN)), src = single ? z.sh.DL : 0;
+  switch (10000 * src + 1000 * W + 100 * z.sp + 10 * (z.m2 - 6) + z.LR) {
+#define LZ_CASE(M, LR, SRC, W, SP) \
+  case 10000 * SRC + 1000 * W + 100 * SP + 10 * (M - 6) + LR: f = lz_row_mode<M, LR, SRC, W, SP>(mode); break;
+#define LZ_CASE1(M, LR, SP) LZ_CASE(M, LR, 2, 0, SP) LZ_CASE(M, LR, 3, 0, SP)
+    LZ_CASE1(8, 3, 0)
+    LZ_CASE1(9, 3, 0)
+    LZ_CASE1(10, 3, 0)
+    LZ_CASE1(11, 3, 0)
+    LZ_CASE1(12, 3, 0)
+    LZ_CASE1(10, 4, 0)
+    LZ_CASE1(11, 4, 0)
+    LZ_CASE1(12, 4, 0)
+    LZ_CASE1(13, 4, 0)
+    LZ_CASE1(11, 3, 1)
+    LZ_CASE1(12, 3, 1)
+    LZ_CASE1(12, 3, 2)
+    LZ_CASE(7, 3, 0, 0, 0)
+    LZ_CASE(8, 3, 0, 0, 0)
+    LZ_CASE(9, 3, 0, 0, 0)
+    LZ_CASE(10, 4, 0, 0, 0)
+    LZ_CASE(11, 3, 0, 0, 0)
+    LZ_CASE(12, 4, 0, 0, 0)
+    LZ_CASE(11, 4, 0, 1, 0)
+    LZ_CASE(12, 4, 0, 2, 0)
 #undef LZ_CASE1
-#define LZ_CASES(M)                                            \
-  case 1200 + M: f = lz_split_kernel<M, 2>(z.sp, mode); break; \
-  case 1300 + M: f = lz_split_kernel<M, 3>(z.sp, mode); break;
-    LZ_CASES(10)
-    LZ_CASES(11)
-    LZ_CASES(12)
-    LZ_CASES(13)
-#undef LZ_CASES
-    case 7: f = lz_row_kernel<7, 0>(z.LR, mode); break;
-    case 8: f = lz_row_kernel<8, 0>(z.LR, mode); break;
-    case 9: f = lz_row_kernel<9, 0>(z.LR, mode); break;
-    case 10: f = lz_row_kernel<10, 0>(z.LR, mode); break;
-    case 11: f = lz_width(lz_set(c.pl.LN)) == 1 ? lz_row_mode<11, 4, 0, 1, 0>(mode) : lz_row_mode<11, 4, 0, 2, 0>(mode); break;
+#undef LZ_CASE
     default: return fail(ANNIE_ERR_SIZE, "no row kernel for this length");
   }
   ProfScope ps(c, "k_lz_row", z.m2, mode == LZ_SQR ? "sqr" : mode == LZ_MULN ? "muln" : "gen", planes);
@@ -881,35 +884,34 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
   return ANNIE_OK;
 }
 
+template <int M, int LR, int W>
+static LzKernel lz_col_kernel(bool inverse, int DL) {
+  return inverse ? k_lz_coli<M, LR, W> : DL == 2 ? k_lz_colf<M, LR, 2, W> : k_lz_colf<M, LR, 3, W>;
+}
+
 static int lz_col(Ctx& c, LzNtt& A, bool inverse, int planes) {
-  const bool wide = c.lz.m1 >= 10;
-  const uint32_t S = 1u << c.lz.m1, T = S / (wide ? 32u : 16u), n2 = uint32_t(c.n >> c.lz.m1);
-  uint32_t C = col_cols_default(c.lz.m1, c.pl.LN);
+  const Lazy& z = c.lz;
+  const bool wide = z.m1 >= 10;
+  const uint32_t S = 1u << z.m1, n2 = uint32_t(c.n >> z.m1);
+  uint32_t C = wide ? 16u : z.cols;
   if (c.sched_cols != 0 && !wide) C = c.sched_cols;  // checked by annie_hip_set_schedule
-  if (wide && C != 8u) return fail(ANNIE_ERR_SIZE, "column pass geometry");
+  const int LR = wide ? 5 : 4;
+  // At 2^10 the planes go with the column groups (lz_tile in lazy.hip, in units
+  // of 32 columns over eight XCDs).
+  if (C * (S >> LR) > 1024u || (wide && n2 % 256u != 0)) return fail(ANNIE_ERR_SIZE, "column pass geometry");
   A.cols = int(C);
-  // From 2^10 on the planes go with the column groups (lz_tile in lazy.hip, in
-  // units of four groups over eight XCDs: n2 >= 2^10 columns are whole units).
-  if (wide && n2 % 256u != 0) return fail(ANNIE_ERR_SIZE, "column pass geometry");
   A.planes = planes;
-  const dim3 grid(n2 / C * (wide ? unsigned(planes) : 1u), unsigned(c.nslots), wide ? 1u : unsigned(planes)), block(C * T);
+  const dim3 grid(n2 / C * (wide ? unsigned(planes) : 1u), unsigned(c.nslots), wide ? 1u : unsigned(planes)), block(C * (S >> LR));
   const size_t shm = size_t(wide ? C : C + 1) * S * 4;
   LzKernel f = nullptr;
-  switch (100 * lz_width(lz_set(c.pl.LN)) + c.lz.m1 * 4 + (inverse ? 0 : c.lz.sh.DL)) {
-#define LZ_CASE(M, W)                                        \
-  case 100 * W + M * 4: f = k_lz_coli<M, W>; break;          \
-  case 100 * W + M * 4 + 2: f = k_lz_colf<M, 2, W>; break;   \
-  case 100 * W + M * 4 + 3: f = k_lz_colf<M, 3, W>; break;
-    LZ_CASE(7, 0)
-    LZ_CASE(8, 0)
-    LZ_CASE(9, 0)
-    LZ_CASE(10, 0)
-    LZ_CASE(10, 1)
-    LZ_CASE(11, 2)
-#undef LZ_CASE
+  switch (100 * lz_width(lz_set(c.pl.LN)) + z.m1) {
+    case 7: f = lz_col_kernel<7, 4, 0>(inverse, z.sh.DL); break;
+    case 8: f = lz_col_kernel<8, 4, 0>(inverse, z.sh.DL); break;
+    case 110: f = lz_col_kernel<10, 5, 1>(inverse, z.sh.DL); break;
+    case 210: f = lz_col_kernel<10, 5, 2>(inverse, z.sh.DL); break;
     default: return fail(ANNIE_ERR_SIZE, "no column kernel for this length");
   }
-  ProfScope ps(c, inverse ? "k_lz_coli" : "k_lz_colf", c.lz.m1, nullptr, planes);
+  ProfScope ps(c, inverse ? "k_lz_coli" : "k_lz_colf", z.m1, nullptr, planes);
   hipLaunchKernelGGL(f, grid, block, shm, c.stream, A);
   HIPCHK(hipGetLastError());
   return ANNIE_OK;

@@ -63,7 +63,7 @@ constexpr bool lz_fwd_red(int W, int M, int LR, int s, int I) {
 constexpr bool lz_safe(int W, int M, int LR, int s) { return lz_walk(W, M, LR, s, -1) <= lz_lim(W); }
 static_assert(lz_safe(0, 13, 3, lz_in(0)) && lz_safe(0, 13, 4, lz_in(0)) && lz_safe(0, 10, 5, lz_in(0)) &&
                   lz_safe(0, 10, 4, lz_lim(0)) && lz_safe(0, 10, 3, lz_lim(0)) && lz_safe(1, 10, 5, lz_in(1)) &&
-                  lz_safe(1, 11, 4, lz_lim(1)) && lz_safe(2, 11, 5, lz_in(2)) && lz_safe(2, 11, 4, lz_lim(2)),
+                  lz_safe(1, 11, 4, lz_lim(1)) && lz_safe(2, 10, 5, lz_in(2)) && lz_safe(2, 12, 4, lz_lim(2)),
               "a forward line leaves its words");
 
 struct LzP {
@@ -436,18 +436,21 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
 }
 
 // Column passes of lengths from 2^14 on: the first M = m1 levels on columns of
-// stride n2 = n / 2^M, A.cols (8 for M >= 10) consecutive columns per block,
+// stride n2 = n / 2^M, A.cols (16 for M = 10) consecutive columns per block,
 // interleaved and XOR-swizzled in LDS as the passes over the long primes.
-// Grid: (column groups, slots, planes); from 2^10 on (column groups x planes,
-// slots): a unit of four column groups covers whole 128-byte lines and goes to
-// one XCD (id mod 8) with all its planes in turn, so that the digits are read
-// from memory once for all planes (25 MB instead of 15 times that at 2^21).
-template <int M>
+// Grid: (column groups, slots, planes); at 2^10 (column groups x planes, slots):
+// a unit of two column groups covers whole 128-byte lines and goes to one XCD
+// (id mod 8) with all its planes in turn, so that the digits are read from
+// memory once for all planes (25 MB instead of 15 times that at 2^21).
+// Sixteen columns of 2^10 take 64 KiB of LDS, two workgroups a CU; eight read
+// and wrote 1.4 times the data (half-used lines left L2 before the neighbouring
+// group came; nine planes of 2^21 back 60 -> 43 us, fifteen forward 77 -> 66).
+template <int M, int LR>
 struct LzCol {
-  static constexpr int LR = (M >= 10) ? 5 : 4;
-  static constexpr bool LDS_ROOTS = (LR == 4);
-  static constexpr int THREADS = (M >= 10) ? (8 << (M - LR)) : 1024;
-  static constexpr int WAVES = (M >= 10) ? 4 : 4;
+  static constexpr bool LDS_ROOTS = M < 10;
+  static constexpr int C = 16;  // columns per block at M = 10
+  static constexpr int THREADS = (M >= 10) ? (C << (M - LR)) : 1024;
+  static constexpr int WAVES = 4;
 };
 
 struct LzTile {
@@ -459,21 +462,22 @@ __device__ __forceinline__ LzTile lz_tile(const LzNtt& A, uint32_t C) {
   if constexpr (M < 10) {
     return {A.pl0 + int(blockIdx.z), col_group(C) * C};
   } else {
-    const uint32_t per = 4u * uint32_t(A.planes), t = blockIdx.x >> 3;
+    constexpr uint32_t G = 32u / LzCol<M, 5>::C;  // column groups of a 128-byte line
+    const uint32_t per = G * uint32_t(A.planes), t = blockIdx.x >> 3;
     const uint32_t unit = (t / per) * 8u + (blockIdx.x & 7u), r = t % per;
-    return {A.pl0 + int(r >> 2), (unit * 4u + (r & 3u)) * C};
+    return {A.pl0 + int(r / G), (unit * G + r % G) * C};
   }
 }
 
-template <int M, int DL, int W>
-__global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(const LzNtt A) {
+template <int M, int LR, int DL, int W>
+__global__ void __launch_bounds__((LzCol<M, LR>::THREADS), (LzCol<M, LR>::WAVES)) k_lz_colf(const LzNtt A) {
   extern __shared__ uint32_t lds[];
-  constexpr int LR = LzCol<M>::LR;
+  lz_pin(A.slot_ids, A.slot_stride, A.LN, A.KR, A.pl0, A.planes, A.cols, A.x, A.wr, A.wq, A.fwdR, A.invR, A.fwdQ, A.invQ, A.neg);
   constexpr uint32_t S = 1u << M;
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride, n = size_t(1) << A.LN;
-  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const uint32_t C = (M >= 10) ? uint32_t(LzCol<M, LR>::C) : uint32_t(A.cols);
   const LzTile tile = lz_tile<M>(A, C);
   const int pl = tile.pl;
   const bool cyc = pl < A.KR;
@@ -490,8 +494,7 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
   auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
 
-  // Roots of 2^10 one round ahead from the table; 2^11 would spill.
-  constexpr int ROOTS = M == 10 ? 1 : 0;
+  constexpr int ROOTS = LzCol<M, LR>::LDS_ROOTS ? 0 : 1;  // 2^10: one round ahead, from the table
   uint32_t x[1 << LR];
   LzRoots<M, LR, 0> none;
   SchedTw<M, LR, 0> t0;
@@ -499,7 +502,7 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   round_load<LR, Sched<M, LR>::template rr<0>()>(x, M, 0, tg, gld);
   if (A.neg != nullptr && threadIdx.x == 0u && col0 == 0u && A.neg[so] == 0u)
     x[0] = uint32_t(lz_red(int32_t(x[0] + 2u * uint32_t(A.c.one[k])), P));  // m' + 2, as in k_lz_row
-  if constexpr (LzCol<M>::LDS_ROOTS) {
+  if constexpr (LzCol<M, LR>::LDS_ROOTS) {
     uint32_t* roots = lds + C * S;
     for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twf[i];
     __syncthreads();
@@ -510,14 +513,14 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_colf(
   round_store<LR, RL>(x, M, DLV, tg, gst);
 }
 
-template <int M, int W>
-__global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(const LzNtt A) {
+template <int M, int LR, int W>
+__global__ void __launch_bounds__((LzCol<M, LR>::THREADS), (LzCol<M, LR>::WAVES)) k_lz_coli(const LzNtt A) {
   extern __shared__ uint32_t lds[];
-  constexpr int LR = LzCol<M>::LR;
+  lz_pin(A.slot_ids, A.slot_stride, A.LN, A.KR, A.pl0, A.planes, A.cols, A.x, A.wr, A.wq, A.fwdR, A.invR, A.fwdQ, A.invQ, A.neg);
   constexpr uint32_t S = 1u << M;
   constexpr int NR = Sched<M, LR>::NR, DLV = LR * (NR - 1), RL = Sched<M, LR>::template rr<NR - 1>();
   const size_t so = size_t(lz_slot(A.slot_ids, blockIdx.y)) * A.slot_stride, n = size_t(1) << A.LN;
-  const uint32_t C = (LR == 5) ? 8u : uint32_t(A.cols);
+  const uint32_t C = (M >= 10) ? uint32_t(LzCol<M, LR>::C) : uint32_t(A.cols);
   const LzTile tile = lz_tile<M>(A, C);
   const int pl = tile.pl;
   const bool cyc = pl < A.KR;
@@ -533,13 +536,12 @@ __global__ void __launch_bounds__(LzCol<M>::THREADS, LzCol<M>::WAVES) k_lz_coli(
   auto lld = [&](uint32_t i) { return lds[i * C + (line ^ ((i >> LR) & (C - 1u)))]; };
   auto lst = [&](uint32_t i, uint32_t v) { lds[i * C + (line ^ ((i >> LR) & (C - 1u)))] = v; };
 
-  // Roots of 2^10 one round ahead from the table; 2^11 would spill.
-  constexpr int ROOTS = M == 10 ? 1 : 0;
+  constexpr int ROOTS = LzCol<M, LR>::LDS_ROOTS ? 0 : 1;  // 2^10: one round ahead, from the table
   uint32_t x[1 << LR];
   LzRoots<M, LR, 0> none;
   SchedTw<M, LR, NR - 1> ti;
   round_load<LR, RL>(x, M, DLV, tg, gld);
-  if constexpr (LzCol<M>::LDS_ROOTS) {
+  if constexpr (LzCol<M, LR>::LDS_ROOTS) {
     uint32_t* roots = lds + C * S;
     for (uint32_t i = threadIdx.x; i < S; i += blockDim.x) roots[i] = twi[i];
     __syncthreads();
@@ -961,49 +963,41 @@ __global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* 
   }
 }
 
-// Instantiations, looked up by the host engine.  Eight elements per thread
-// (LR = 3) for short launches, sixteen where they fill the GPU.
+// Instantiations, looked up by the host engine (lz_geometry chooses among
+// them): whole transforms, split ones, row passes, column passes.
 #define LZ_ROW(M, LR, SRC, W, SP)                                             \
   template __global__ void k_lz_row<M, LR, LZ_SQR, SRC, W, SP>(const LzNtt);  \
   template __global__ void k_lz_row<M, LR, LZ_MULN, SRC, W, SP>(const LzNtt); \
   template __global__ void k_lz_row<M, LR, LZ_GEN, SRC, W, SP>(const LzNtt);
-#define LZ_ROW1(M)      \
-  LZ_ROW(M, 3, 2, 0, 0) \
-  LZ_ROW(M, 3, 3, 0, 0) \
-  LZ_ROW(M, 4, 2, 0, 0) \
-  LZ_ROW(M, 4, 3, 0, 0)
-LZ_ROW1(8)
-LZ_ROW1(9)
-LZ_ROW1(10)
-LZ_ROW1(11)
-LZ_ROW1(12)
-LZ_ROW1(13)
-#define LZ_ROWS(M)      \
-  LZ_ROW(M, 3, 2, 0, 1) \
-  LZ_ROW(M, 3, 3, 0, 1) \
-  LZ_ROW(M, 3, 2, 0, 2) \
-  LZ_ROW(M, 3, 3, 0, 2)
-LZ_ROWS(10)
-LZ_ROWS(11)
-LZ_ROWS(12)
-LZ_ROWS(13)
-#define LZ_ROW2(M) LZ_ROW(M, 3, 0, 0, 0) LZ_ROW(M, 4, 0, 0, 0)
-LZ_ROW2(7)
-LZ_ROW2(8)
-LZ_ROW2(9)
-LZ_ROW2(10)
+#define LZ_ROW1(M, LR, SP) LZ_ROW(M, LR, 2, 0, SP) LZ_ROW(M, LR, 3, 0, SP)
+LZ_ROW1(8, 3, 0)
+LZ_ROW1(9, 3, 0)
+LZ_ROW1(10, 3, 0)
+LZ_ROW1(11, 3, 0)
+LZ_ROW1(12, 3, 0)
+LZ_ROW1(10, 4, 0)
+LZ_ROW1(11, 4, 0)
+LZ_ROW1(12, 4, 0)
+LZ_ROW1(13, 4, 0)
+LZ_ROW1(11, 3, 1)
+LZ_ROW1(12, 3, 1)
+LZ_ROW1(12, 3, 2)
+LZ_ROW(7, 3, 0, 0, 0)
+LZ_ROW(8, 3, 0, 0, 0)
+LZ_ROW(9, 3, 0, 0, 0)
+LZ_ROW(10, 4, 0, 0, 0)
+LZ_ROW(11, 3, 0, 0, 0)
+LZ_ROW(12, 4, 0, 0, 0)
 LZ_ROW(11, 4, 0, 1, 0)
-LZ_ROW(11, 4, 0, 2, 0)
-#define LZ_COL(M, W)                                          \
-  template __global__ void k_lz_colf<M, 2, W>(const LzNtt);   \
-  template __global__ void k_lz_colf<M, 3, W>(const LzNtt);   \
-  template __global__ void k_lz_coli<M, W>(const LzNtt);
-LZ_COL(7, 0)
-LZ_COL(8, 0)
-LZ_COL(9, 0)
-LZ_COL(10, 0)
-LZ_COL(10, 1)
-LZ_COL(11, 2)
+LZ_ROW(12, 4, 0, 2, 0)
+#define LZ_COL(M, LR, W)                                        \
+  template __global__ void k_lz_colf<M, LR, 2, W>(const LzNtt); \
+  template __global__ void k_lz_colf<M, LR, 3, W>(const LzNtt); \
+  template __global__ void k_lz_coli<M, LR, W>(const LzNtt);
+LZ_COL(7, 4, 0)
+LZ_COL(8, 4, 0)
+LZ_COL(10, 5, 1)
+LZ_COL(10, 5, 2)
 #define LZ_CARRY(SET, SP)                                                         \
   template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false, SP>(const LzCarry); \
   template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true, SP>(const LzCarry);  \
