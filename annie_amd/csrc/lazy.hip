@@ -26,7 +26,7 @@ constexpr int lz_lim(int W) { return W == 0 ? 1766 : W == 1 ? 828 : 545; }   // 
 constexpr int lz_gain(int W) { return W == 0 ? 37 : W == 1 ? 80 : 121; }     // 1024 p / 2^33
 constexpr int LZ_RED = 264;                                                   // lz_red: [0, 1.03 p)
 constexpr int lz_in(int W) { return W == 0 ? 384 : 262; }                     // a digit's residue as loaded
-constexpr int lz_out(int W) { return W == 0 ? 410 : 256; }                    // what an inverse round starts from
+constexpr int lz_out(int W) { return W == 0 ? 410 : W == 1 ? 270 : 256; }     // what an inverse round starts from
 constexpr int lz_less(int s) { return s > 512 ? s - 256 : 256; }              // lz_cond of a value within s
 
 // Forward bounds: lz_level is the bound after one level from bound s (the
@@ -82,9 +82,61 @@ __device__ __forceinline__ int32_t lz_red(int32_t x, const LzP& P) {
   return x - int32_t(uint32_t(__mulhi(x, int32_t(P.bar)) >> 26) * P.p);
 }
 
+// Inverse bounds: before a sum and difference leave their words, one or both
+// operands are reduced by lz_cond, once or twice, or by lz_red (codes 1, 2, 3;
+// 0: not at all), whichever takes the fewest issue slots (2.3 and 3.6 each);
+// after the last level of a round all elements are brought back within lz_out.
+// Compared with one lz_cond for every sum: 55 instead of 74 slots per 32
+// butterflies for W = 1.
+template <int RR, int W>
+struct LzPlan {
+  uint8_t op[RR][1 << RR], end[1 << RR];
+};
+constexpr int lz_reduced(int W, int s, int op) {
+  return op == 0 ? s : op == 3 ? (s < LZ_RED ? s : LZ_RED) : op == 1 ? lz_less(s) : lz_less(lz_less(s));
+}
+constexpr int lz_cost(int op) { return op == 0 ? 0 : op == 1 ? 23 : op == 2 ? 46 : 36; }
+template <int RR, int W>
+constexpr LzPlan<RR, W> lz_inv_plan() {
+  LzPlan<RR, W> pl{};
+  int bd[1 << RR] = {};
+  for (int j = 0; j < (1 << RR); ++j) bd[j] = lz_out(W);
+  const int first = W == 0 ? 3 : 1;  // W = 0: lz_red only
+  for (int e = RR - 1; e >= 0; --e) {
+    const int half = (1 << RR) >> (e + 1);
+    for (int j = 0; j < (1 << RR); ++j) {
+      if (j & half) continue;
+      const int i = j + half;
+      if (bd[j] + bd[i] > lz_lim(W)) {
+        int best = 1 << 30;
+        for (int a = 0; a < 4; ++a)
+          for (int b = 0; b < 4; ++b) {
+            if ((a > 0 && a < first) || (b > 0 && b < first)) continue;
+            const int s = lz_reduced(W, bd[j], a) + lz_reduced(W, bd[i], b), cost = (lz_cost(a) + lz_cost(b)) * 4096 + s;
+            if (s <= lz_lim(W) && cost < best) {
+              best = cost;
+              pl.op[e][j] = uint8_t(a);
+              pl.op[e][i] = uint8_t(b);
+            }
+          }
+        bd[j] = lz_reduced(W, bd[j], pl.op[e][j]);
+        bd[i] = lz_reduced(W, bd[i], pl.op[e][i]);
+      }
+      const int s = bd[j] + bd[i];
+      bd[j] = s;
+      bd[i] = 130 + s * lz_gain(W) / 1024;
+    }
+  }
+  for (int j = 0; j < (1 << RR); ++j)
+    if (bd[j] > lz_out(W))
+      for (int a : {1, 3, 2})
+        if (a >= first && lz_reduced(W, bd[j], a) <= lz_out(W) && pl.end[j] == 0) pl.end[j] = uint8_t(a);
+  return pl;
+}
+
 // x - p or x + p by the sign: within max(p, |x| - p).
 __device__ __forceinline__ uint32_t lz_cond(uint32_t x, const LzP& P) {
-  return x + (uint32_t(int32_t(x) >> 31) & (2u * P.p)) - P.p;
+  return x + (int32_t(x) < 0 ? P.p : 0u - P.p);
 }
 
 // The levels of one round from elements within s.
@@ -116,21 +168,18 @@ __device__ __forceinline__ void lz_round_fwd(uint32_t (&x)[1 << LR], const Round
 }
 
 // Inverse levels of a round; the elements start within lz_out, and end there
-// too unless LAST (then within their words).  bd: the bound of each element, a
-// compile-time constant after unrolling.
-template <int W>
-__device__ __forceinline__ void lz_less_inv(uint32_t& x, int& bd, const LzP& P) {
-  if (W == 0 && bd > LZ_RED) x = uint32_t(lz_red(int32_t(x), P)), bd = LZ_RED;
-  if (W > 0 && bd > 256) x = lz_cond(x, P), bd = lz_less(bd);
+// too unless LAST (then within their words).
+__device__ __forceinline__ void lz_apply(uint32_t& x, int op, const LzP& P) {
+  if (op == 3) x = uint32_t(lz_red(int32_t(x), P));
+  if (op == 1 || op == 2) x = lz_cond(x, P);
+  if (op == 2) x = lz_cond(x, P);
 }
 
 template <int LR, int RR, int W, bool LAST>
 __device__ __forceinline__ void lz_round_inv(uint32_t (&x)[1 << LR], const RoundTw<LR, RR>& T, const LzP& P) {
+  constexpr LzPlan<RR, W> PL = lz_inv_plan<RR, W>();
 #pragma unroll
   for (int s = 0; s < RoundTw<LR, RR>::G; ++s) {
-    int bd[1 << RR];
-#pragma unroll
-    for (int j = 0; j < (1 << RR); ++j) bd[j] = lz_out(W);
     uint32_t* v = &x[s * (1 << RR)];
 #pragma unroll
     for (int e = RR - 1; e >= 0; --e) {
@@ -141,23 +190,17 @@ __device__ __forceinline__ void lz_round_inv(uint32_t (&x)[1 << LR], const Round
 #pragma unroll
         for (int jj = 0; jj < half; ++jj) {
           const int j = blk * 2 * half + jj, i = j + half;
-          if (bd[j] + bd[i] > lz_lim(W)) {
-            lz_less_inv<W>(v[j], bd[j], P);
-            lz_less_inv<W>(v[i], bd[i], P);
-          }
+          lz_apply(v[j], PL.op[e][j], P);
+          lz_apply(v[i], PL.op[e][i], P);
           const uint32_t d = v[j] - v[i];
           v[j] = v[j] + v[i];
           v[i] = uint32_t(lz_mulc(int32_t(d), int32_t(r), rq, P.p));
-          const int sum = bd[j] + bd[i];
-          bd[j] = sum;
-          bd[i] = 130 + sum * lz_gain(W) / 1024;
         }
       }
     }
     if constexpr (!LAST) {
 #pragma unroll
-      for (int j = 0; j < (1 << RR); ++j)
-        if (bd[j] > lz_out(W)) lz_less_inv<W>(v[j], bd[j], P);
+      for (int j = 0; j < (1 << RR); ++j) lz_apply(v[j], PL.end[j], P);
     }
   }
 }
