@@ -1526,7 +1526,7 @@ static int lz_get_values(Ctx& c, int src, const size_t* slots, const mpz_t* cons
       mpz_t& v = *zs[i0 + i];
       const mpz_t& N = *mods[i0 + i];
       const size_t words = (c.n / 32) * size_t(slot_cbits(c, slots[i0 + i]));
-      mpz_import(v, words, -1, 4, 0, 0, z.pack_host + i * per);
+      mpz_import(v, words / 2, -1, 8, 0, 0, z.pack_host + i * per);  // whole limbs: GMP copies them
       if (mpz_tstbit(v, mp_bitcnt_t(words) * 32 - 1)) {  // negative: only from a register that holds no residue
         Mpz top;
         mpz_setbit(top.v, mp_bitcnt_t(words) * 32);
