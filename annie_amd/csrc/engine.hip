@@ -46,7 +46,7 @@ template <int M, int LR, int DL, int W>
 __global__ void k_lz_colf(const LzNtt A);
 template <int M, int LR, int W>
 __global__ void k_lz_coli(const LzNtt A);
-template <int SET, int KP, int L, int ND, int DL, bool NEGA, int SP>
+template <int SET, int KP, int L, int ND, int DL, bool NEGA, int EX, int SP>
 __global__ void k_lz_carry(const LzCarry A);
 __global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
 template <int DL>
@@ -948,8 +948,9 @@ static LzNtt lz_args(const Ctx& c) {
   return A;
 }
 
-static int lz_carry(Ctx& c, LzCarry& A, bool cyc) {
-  const int nd = cyc ? (c.pl.K == 3 ? 5 : 4) : 3;
+// external: A.dst receives the plan's K residue planes instead of digits (k_lz_carry's EX).
+static int lz_carry(Ctx& c, LzCarry& A, bool cyc, bool external = false) {
+  const int nd = cyc ? (c.pl.K == 3 ? 5 : 4) : external ? 6 : 3;  // halo lanes of a wave
   const size_t waves = (c.n + size_t(63 - nd)) / size_t(64 - nd);
   const dim3 grid(unsigned((waves + 3) / 4), unsigned(c.nslots)), block(256);
   A.slot_ids = c.slot_ids;
@@ -959,16 +960,19 @@ static int lz_carry(Ctx& c, LzCarry& A, bool cyc) {
   A.cbits_slot = c.cbits_dev;
   ProfScope ps(c, cyc ? "k_lz_carryR" : "k_lz_carryQ", c.pl.K, nullptr, 1);
   A.twi = c.lz.tw + (cyc ? size_t(c.lz.sh.KR) : 2 * size_t(c.lz.sh.KR) + size_t(c.lz.sh.KQ)) * c.n;
-  switch (100 * c.lz.sp + 10 * lz_set(c.pl.LN) + c.pl.K * 2 + (cyc ? 1 : 0) - 6) {
+  switch (100 * c.lz.sp + 20 * lz_set(c.pl.LN) + c.pl.K * 3 + (cyc ? 1 : external ? 2 : 0) - 9) {
 #define LZ_CASE1(ID, SET, SP, ...) \
-  case 100 * SP + 10 * SET + ID: hipLaunchKernelGGL((k_lz_carry<SET, __VA_ARGS__, SP>), grid, block, 0, c.stream, A); break;
+  case 100 * SP + 20 * SET + ID: hipLaunchKernelGGL((k_lz_carry<SET, __VA_ARGS__, SP>), grid, block, 0, c.stream, A); break;
 #define LZ_CASE(SET, SP)                     \
-  LZ_CASE1(1, SET, SP, 6, 6, 5, 2, false) \
-  LZ_CASE1(0, SET, SP, 4, 4, 3, 2, true)  \
-  LZ_CASE1(3, SET, SP, 7, 7, 4, 2, false) \
-  LZ_CASE1(2, SET, SP, 5, 5, 3, 2, true)  \
-  LZ_CASE1(5, SET, SP, 9, 8, 4, 3, false) \
-  LZ_CASE1(4, SET, SP, 6, 6, 3, 3, true)
+  LZ_CASE1(1, SET, SP, 6, 6, 5, 2, false, 0) \
+  LZ_CASE1(0, SET, SP, 4, 4, 3, 2, true, 0)  \
+  LZ_CASE1(2, SET, SP, 4, 4, 3, 2, true, 3)  \
+  LZ_CASE1(4, SET, SP, 7, 7, 4, 2, false, 0) \
+  LZ_CASE1(3, SET, SP, 5, 5, 3, 2, true, 0)  \
+  LZ_CASE1(5, SET, SP, 5, 5, 3, 2, true, 4)  \
+  LZ_CASE1(7, SET, SP, 9, 8, 4, 3, false, 0) \
+  LZ_CASE1(6, SET, SP, 6, 6, 3, 3, true, 0)  \
+  LZ_CASE1(8, SET, SP, 6, 6, 3, 3, true, 5)
     LZ_CASE(0, 0)
     LZ_CASE(0, 1)
     LZ_CASE(0, 2)
@@ -998,9 +1002,10 @@ static LzBufs lz_bufs(const Ctx& c, const uint32_t* x, uint32_t* y) {
 // MMGW product y = a x v: v = x (LZ_SQR), or with LZ_GEN the register whose
 // transforms are in PYR / PYQ (op LZ_MULY) or 1 (LZ_MUL1).  mul: the multiplier
 // of each list position; snap / snapbits: positions whose result also goes to
-// LZ_SNAP.
+// LZ_SNAP.  external: y receives the register format of the callers' buffers
+// instead of digits.
 static int lz_product(Ctx& c, const LzBufs& B, int mode, int op, const LzMult& mul, const uint32_t* snap = nullptr,
-                      const uint32_t* snapbits = nullptr) {
+                      const uint32_t* snapbits = nullptr, bool external = false) {
   const int KR = c.lz.sh.KR, KQ = c.lz.sh.KQ;
   int rc;
   c.staged = false;
@@ -1032,7 +1037,7 @@ static int lz_product(Ctx& c, const LzBufs& B, int mode, int op, const LzMult& m
   Q.mul.a = 1u;
   Q.mul.bits_mode = snapbits != nullptr ? 2 : 0;
   if (snapbits != nullptr) std::memcpy(Q.mul.bits, snapbits, sizeof(Q.mul.bits));
-  return lz_carry(c, Q, false);
+  return lz_carry(c, Q, false, external);
 }
 
 static LzMult lz_by(uint32_t a) {
@@ -1649,9 +1654,9 @@ static bool ready(const annie_hip_t* h) {
 // `scratch` only names the symbol; its device address on each GPU comes from
 // hipGetSymbolAddress, looked up once per device with that device current.
 constexpr size_t NOALLOC_KN_MAX = ANNIE_HIP_NOALLOC_MAX_KN;
-// Short primes: three digit registers, a block of flags and the work planes
-// (23 n words at K = 4, the largest: n <= 2^17 there, 2^16 at K = 5).
-constexpr size_t SCRATCH_WORDS = 23 * (NOALLOC_KN_MAX / 4) + LZ_FLAGS;
+// Short primes: two digit registers, a block of flags and the work planes (21 n
+// words at K = 4, the largest: n <= 2^17 there, 2^16 at K = 5).
+constexpr size_t SCRATCH_WORDS = 22 * (NOALLOC_KN_MAX / 4) + LZ_FLAGS;
 static_assert(SCRATCH_WORDS >= 4 * NOALLOC_KN_MAX + size_t(DIGIT_LIMBS) * (NOALLOC_KN_MAX / 2), "long-prime work registers");
 static __device__ __align__(256) uint32_t scratch[SCRATCH_WORDS];
 
@@ -1779,12 +1784,10 @@ int annie_hip_square_mul_noalloc(annie_hip_t* h, const uint32_t* x, uint32_t* y,
   if (c.lz.on && !lz_takes(c, uint32_t(a)) && (rc = lz_demote(c))) return rc;
   if (c.lz.on) {
     const size_t n = c.n, dig = size_t(c.lz.sh.DL) * n, kr = size_t(c.lz.sh.KR) * n, kq = size_t(c.lz.sh.KQ) * n;
-    if (3 * dig + kr + 2 * kq + LZ_FLAGS > SCRATCH_WORDS) return fail(ANNIE_ERR_SIZE, "no-allocation work registers");
-    uint32_t *dx = w, *dy = w + dig, *mp = w + 2 * dig, *wr = w + 3 * dig, *wq = wr + kr, *mq = wq + kq, *neg = mq + kq;
+    if (2 * dig + kr + 2 * kq + LZ_FLAGS > SCRATCH_WORDS) return fail(ANNIE_ERR_SIZE, "no-allocation work registers");
+    uint32_t *dx = w, *mp = w + dig, *wr = w + 2 * dig, *wq = wr + kr, *mq = wq + kq, *neg = mq + kq;
     if ((rc = lz_import(c, x, dx, c.pl.cbits()))) return rc;
-    const LzBufs B{dx, dy, mp, neg, wr, wq, mq};
-    if ((rc = lz_product(c, B, LZ_SQR, 0, lz_by(uint32_t(a))))) return rc;
-    return lz_export(c, dy, y, c.pl.cbits());
+    return lz_product(c, LzBufs{dx, y, mp, neg, wr, wq, mq}, LZ_SQR, 0, lz_by(uint32_t(a)), nullptr, nullptr, true);
   }
   const SqBufs B{x, y, w, w + kn, w + 2 * kn, w + 3 * kn, w + 4 * kn};
   // One stream: the two-stream squaring is only used above this size limit.

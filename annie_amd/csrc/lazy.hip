@@ -756,6 +756,35 @@ __device__ __forceinline__ LzDig<DL> lz_finish(uint32_t (&v)[LZ_MAXL], uint32_t 
   return lz_add(s, lz_small(s, c));
 }
 
+// The lane's digit brought into [-B/2, B/2): three carry steps (a longer run of
+// carries would need three digits at the edge of their range in a row, and
+// keeps the value all the same).  The LZ_BALANCE lowest lanes are not final.
+constexpr int LZ_BALANCE = 3;
+template <int DL>
+__device__ __forceinline__ LzDig<DL> lz_balance(LzDig<DL> s, uint32_t sh, bool flip) {
+#pragma unroll
+  for (int step = 0; step < LZ_BALANCE; ++step) {
+    const int32_t q = lz_split(s, sh);
+    int32_t c = int32_t(lz_shr1(uint32_t(q)));
+    if (flip) c = -c;
+    s = lz_add(s, lz_small(s, c));
+  }
+  return s;
+}
+
+// A digit as residues of the plan's first K primes.
+template <int K, int DL>
+__device__ __forceinline__ void lz_store_residues(uint32_t* dst, size_t n, uint32_t i, const LzDig<DL>& s) {
+  uint32_t d[DIGIT_LIMBS];
+  const uint64_t u = uint64_t(s.v);
+  d[0] = uint32_t(u);
+  d[1] = uint32_t(u >> 32);
+  if constexpr (DL == 3) d[2] = uint32_t(s.h);
+  else d[2] = uint32_t(int32_t(d[1]) >> 31);
+#pragma unroll
+  for (int k = 0; k < K; ++k) st_w(dst + size_t(k) * n, i, digit_residue_wide(d, k));
+}
+
 // The coefficient as two's complement limbs.  Column l sums KP products below p
 // 2^32: 9 2^(28.2 + 32) < 2^63.4 for the shortest primes; with the wider ones
 // (WIDE) the sums are kept in two halves of at most five products, below
@@ -837,9 +866,13 @@ __device__ __forceinline__ int32_t lz_join(const uint32_t* src, uint32_t i, int 
 }
 
 // Grid: (ceil(waves / 4), slots); block 256.
-template <int SET, int KP, int L, int ND, int DL, bool NEGA, int SP>
+// EX > 0: the result leaves in the external format, EX residue planes at dst (one
+// slot), by waves with the three more halo lanes that the balancing takes. One
+// launch and a pass over the digits less than k_lz_export behind it: a call on 2^10 coefficients 32.5 -> 30.4 us
+// with its synchronisation, on 2^16 55.0 -> 53.9.
+template <int SET, int KP, int L, int ND, int DL, bool NEGA, int EX, int SP>
 __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
-  constexpr int W = 64 - ND;
+  constexpr int H = EX > 0 ? ND + LZ_BALANCE : ND, W = 64 - H;
   lz_pin(A.src, A.dst, A.dst2, A.neg, A.slot_ids, A.slot_stride, A.LN, A.cbits, A.cbits_slot, A.snap, A.mul.a, A.mul.a_slot,
          A.mul.bits_mode, A.mul.slot_base, A.mul.bits[blockIdx.y >> 5 & (INLINE_SLOTS / 32 - 1)]);
   const size_t n = size_t(1) << A.LN;
@@ -858,7 +891,7 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   const int top = int((n - 1) / W);
   if (wave > top) return;
   for (int w = wave;; --w) {
-    const int i = w * W + lane - ND;
+    const int i = w * W + lane - H;
     const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
     int32_t r[KP];
 #pragma unroll
@@ -877,7 +910,12 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
       }
     }
     const LzDig<DL> d = lz_finish<DL, L, ND, NEGA>(v, sh, i == 0);
-    const bool own = lane >= ND && uint32_t(i) < n;
+    const bool own = lane >= H && uint32_t(i) < n;
+    if constexpr (EX > 0) {
+      const LzDig<DL> b = lz_balance<DL>(d, sh, NEGA && i == 0);
+      if (own) lz_store_residues<EX, DL>(A.dst, n, uint32_t(i), b);
+      return;
+    }
     if (w == wave && own) {
       lz_store_digit<DL>(A.dst + so, n, uint32_t(i), d);
       if (snap) lz_store_digit<DL>(A.dst2 + so, n, uint32_t(i), d);
@@ -915,14 +953,11 @@ __global__ void __launch_bounds__(256) k_lz_import(const LzConv A) {
   if (lane >= ND && uint32_t(i) < n) lz_store_digit<DL>(A.dst, n, uint32_t(i), d);
 }
 
-// Digits -> residues of the plan's K primes, of the balanced digits in
-// [-B/2, B/2) (three carry steps: a longer run of carries would need three
-// digits at the edge of their range in a row, and keeps the value all the
-// same).  neg: the register is m' (mod B^n - 1) of that sign, exported as the
+// Digits -> residues of the plan's K primes, of the balanced digits.  neg: the register is m' (mod B^n - 1) of that sign, exported as the
 // squaring defines it: m' + 2, plus R = B^n - 1 when negative.
 template <int K, int DL>
 __global__ void __launch_bounds__(256) k_lz_export(const LzConv A) {
-  constexpr int H = 3, W = 64 - H;
+  constexpr int H = LZ_BALANCE, W = 64 - H;
   const size_t n = size_t(1) << A.LN;
   const int lane = int(threadIdx.x & 63u), w = int(blockIdx.x * 4u + (threadIdx.x >> 6));
   const int i = w * W + lane - H;
@@ -930,13 +965,7 @@ __global__ void __launch_bounds__(256) k_lz_export(const LzConv A) {
   const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
   const uint32_t sh = uint32_t(A.cbits) & 31u;
   LzDig<DL> s = lz_load_digit<DL>(A.src, n, idx);
-#pragma unroll
-  for (int step = 0; step < H; ++step) {
-    const int32_t q = lz_split(s, sh);
-    int32_t c = int32_t(lz_shr1(uint32_t(q)));
-    if (A.neg == nullptr && i == 0) c = -c;
-    s = lz_add(s, lz_small(s, c));
-  }
+  s = lz_balance<DL>(s, sh, A.neg == nullptr && i == 0);
   if (lane < H || uint32_t(i) >= n) return;
   if (A.neg != nullptr) {
     const bool neg = A.neg[0] != 0u;
@@ -946,14 +975,7 @@ __global__ void __launch_bounds__(256) k_lz_export(const LzConv A) {
       else s.h += int32_t(1) << sh;
     }
   }
-  uint32_t d[DIGIT_LIMBS];
-  const uint64_t u = uint64_t(s.v);
-  d[0] = uint32_t(u);
-  d[1] = uint32_t(u >> 32);
-  if constexpr (DL == 3) d[2] = uint32_t(s.h);
-  else d[2] = uint32_t(int32_t(d[1]) >> 31);
-#pragma unroll
-  for (int k = 0; k < K; ++k) st_w(A.dst + size_t(k) * n, uint32_t(i), digit_residue_wide(d, k));
+  lz_store_residues<K, DL>(A.dst, n, uint32_t(i), s);
 }
 
 // A register that holds a non-negative number below B^n / 2, as binary words: 2
@@ -1071,13 +1093,16 @@ LZ_COL(7, 4, 0)
 LZ_COL(8, 4, 0)
 LZ_COL(10, 5, 1)
 LZ_COL(10, 5, 2)
-#define LZ_CARRY(SET, SP)                                                         \
-  template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false, SP>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true, SP>(const LzCarry);  \
-  template __global__ void k_lz_carry<SET, 7, 7, 4, 2, false, SP>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true, SP>(const LzCarry);  \
-  template __global__ void k_lz_carry<SET, 9, 8, 4, 3, false, SP>(const LzCarry); \
-  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true, SP>(const LzCarry);
+#define LZ_CARRY(SET, SP)                                                            \
+  template __global__ void k_lz_carry<SET, 6, 6, 5, 2, false, 0, SP>(const LzCarry);\
+  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true, 0, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 4, 4, 3, 2, true, 3, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 7, 7, 4, 2, false, 0, SP>(const LzCarry);\
+  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true, 0, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 5, 5, 3, 2, true, 4, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 9, 8, 4, 3, false, 0, SP>(const LzCarry);\
+  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true, 0, SP>(const LzCarry); \
+  template __global__ void k_lz_carry<SET, 6, 6, 3, 3, true, 5, SP>(const LzCarry);
 LZ_CARRY(0, 0)
 LZ_CARRY(0, 1)
 LZ_CARRY(0, 2)

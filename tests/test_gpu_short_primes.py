@@ -12,6 +12,7 @@ import pytest
 import annie_amd
 import oracle
 from tests.helpers import assert_same_words, usable_N
+from tests.test_zz_no_alloc import DevBuf, hip  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 P = [(125 << 25) + 1, (243 << 24) + 1, (235 << 24) + 1, (29 << 27) + 1, (13 << 28) + 1]
@@ -222,3 +223,29 @@ def test_batch_geometries(gpu, bits, slots):
             assert int.from_bytes(out[j].tobytes(), "little") == want[s % 3] ** 2 % Ns[s % 3], f"product of slot {s}"
     finally:
         lib.annie_hip_destroy(h)
+
+
+# The result of a squaring on the caller's buffers leaves the last carry in the
+# external format: the same words as the register holds after the same squaring.
+@pytest.mark.parametrize("bits", [10000, 17500, 55000, 200000, 324619, 560000, 1000003])
+def test_squaring_on_caller_buffers(hip, bits):
+    a = 3
+    N = usable_N(bits, bits, a)
+    t = annie_amd.Transform(N, a, min_ln=5)
+    print(f"case bits={bits} K={t.K} LN={t.LN}", flush=True)
+    x, y = DevBuf(hip, t.K * t.n), DevBuf(hip, t.K * t.n)
+    try:
+        values = _edge_values(N, t, random.Random(bits))
+        for j, v in enumerate(values if bits < 100000 else values[-3:]):
+            w = _words(v, t)
+            x.write(w)
+            for m in (1, 3):
+                t.write_register(0, w)
+                t.square_mul(m)
+                t.square_mul_noalloc(x.ptr.value, y.ptr.value, m)
+                t.sync()
+                assert_same_words(y.read(), t.read_register(0), f"value {j}", t.n)
+    finally:
+        x.free()
+        y.free()
+        t.close()
