@@ -48,7 +48,7 @@ template <int M, int LR, int W>
 __global__ void k_lz_coli(const LzNtt A);
 template <int SET, int KP, int L, int ND, int DL, bool NEGA, int EX, int SP>
 __global__ void k_lz_carry(const LzCarry A);
-__global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C);
+__global__ void k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int SP, int KR, int KQ, const LzPrimes C);
 template <int DL>
 __global__ void k_lz_pack(const LzPack A);
 template <int K, int DL>
@@ -751,18 +751,20 @@ static int32_t lz_signed(uint64_t v, uint32_t p) { return v > p / 2 ? int32_t(v)
 
 // Geometry of the transforms.  A launch of few slots leaves most CUs idle and is
 // bound by the chain of one workgroup, so the transform is split over two or
-// four workgroups (lz_branch, lz_join in lazy.hip) while their number is small;
+// four workgroups (lz_branch, LzJoin in lazy.hip) while their number is small;
 // the lines are drawn where both sides measured equal.  us per squaring, not
-// split / two / four: 2^12, one slot 20.0 / 18.1 / 20.1, 16 slots 28.4 / 27.3 /
-// 33.7; 2^13, one slot 30.4 / 22.1 / 22.3, 24 slots 50.2 / 46.8 / 52.1, 40 slots
+// split / two / four: 2^12, one slot 20.0 / 17.8 / 17.8, 16 slots 28.4 / 23.6 /
+// 28.3; 2^13, one slot 30.4 / 21.5 / 19.7, 4 slots - / 24.0 / 22.0, 9 slots - /
+// 28.5 / 28.3, 16 slots - / 33.1 / 35.3, 24 slots 50.2 / 46.8 / 52.1, 40 slots
 // (sixteen elements per thread) 65.0 / 67.9 / 75.3; 2^14 in two passes / four,
-// one slot 32.5 / 31.3 (K = 5), 31.8 / 27.6 (K = 4), 24 slots 85 / 79, 40 slots
-// 121 / 129; 2^11 and 2^15 are no faster split.
+// one slot 30.7 / 27.5 (K = 5), 29.2 / 24.2 (K = 3), 32 slots 81.5 / 76.6, 48
+// slots 105 / 117; 2^11 (16.6 / 16.6 / 17.3) and 2^15 (31.0 / - / 43.2) are no
+// faster split.
 static void lz_geometry(Ctx& c) {
   Lazy& z = c.lz;
   const int LN = c.pl.LN;
   const size_t slots = c.nslots_alloc;
-  z.sp = (LN == 12 && slots <= 16) || (LN == 13 && slots <= 32) ? 1 : (LN == 14 && slots <= 32) ? 2 : 0;
+  z.sp = (LN == 13 && slots <= 8) || (LN == 14 && slots <= 32) ? 2 : (LN == 12 && slots <= 16) || (LN == 13 && slots <= 32) ? 1 : 0;
   // Short columns and long rows: a row keeps its 2^m2 elements in LDS for the
   // forward and the inverse levels, a column pass goes through memory twice.
   // us per squaring with m1 = LN / 2 / as here: 2^16 (8 / 7 columns levels) 37.3 /
@@ -790,7 +792,8 @@ static int lz_setup(Ctx& c) {
   z.stride = lz_slot_words(K, n);
   z.plane0 = size_t(NLZ) * size_t(DL) * n;
   if (hipMalloc(&z.mem, c.nslots_alloc * z.stride * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "register file");
-  if (hipMalloc(&z.tw, (2 * size_t(KR) + 2 * size_t(KQ)) * n * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "roots");
+  const size_t roots = 2 * size_t(KR + KQ) * n + 8 * size_t(KR + KQ);  // tables and LzJoin's constants
+  if (hipMalloc(&z.tw, roots * 4) != hipSuccess) return fail(ANNIE_ERR_NOMEM, "roots");
   HIPCHK(hipMemsetAsync(z.mem, 0, c.nslots_alloc * z.stride * 4, c.stream));
   // Powers psi^i, i < 2^s, and psi^{i 2^s} of a primitive 2n-th root psi of
   // each prime; the device multiplies them into the tables.
@@ -818,8 +821,8 @@ static int lz_setup(Ctx& c) {
   }
   uint32_t* dpw = c.lzplane(PWR);  // scratch: per < n words for every length of this path
   HIPCHK(hipMemcpyAsync(dpw, pw.data(), pw.size() * 4, hipMemcpyHostToDevice, c.stream));
-  hipLaunchKernelGGL(k_lz_roots, dim3(unsigned((n + 255) / 256), unsigned(KR)), dim3(256), 0, c.stream, z.tw, dpw, LN, KR, KQ,
-                     z.pc);
+  hipLaunchKernelGGL(k_lz_roots, dim3(unsigned((n + 255) / 256), unsigned(KR)), dim3(256), 0, c.stream, z.tw, dpw, LN, z.sp, KR,
+                     KQ, z.pc);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c.stream));
   z.on = true;
@@ -865,6 +868,7 @@ static int lz_row(Ctx& c, LzNtt& A, int mode, int planes) {
     LZ_CASE1(13, 4, 0)
     LZ_CASE1(11, 3, 1)
     LZ_CASE1(12, 3, 1)
+    LZ_CASE1(11, 3, 2)
     LZ_CASE1(12, 3, 2)
     LZ_CASE(7, 3, 0, 0, 0)
     LZ_CASE(8, 3, 0, 0, 0)
@@ -959,7 +963,7 @@ static int lz_carry(Ctx& c, LzCarry& A, bool cyc, bool external = false) {
   A.cbits = c.pl.cbits();
   A.cbits_slot = c.cbits_dev;
   ProfScope ps(c, cyc ? "k_lz_carryR" : "k_lz_carryQ", c.pl.K, nullptr, 1);
-  A.twi = c.lz.tw + (cyc ? size_t(c.lz.sh.KR) : 2 * size_t(c.lz.sh.KR) + size_t(c.lz.sh.KQ)) * c.n;
+  A.join = c.lz.tw + 2 * size_t(c.lz.sh.KR + c.lz.sh.KQ) * c.n + (cyc ? 0 : 8 * size_t(c.lz.sh.KR));
   switch (100 * c.lz.sp + 20 * lz_set(c.pl.LN) + c.pl.K * 3 + (cyc ? 1 : external ? 2 : 0) - 9) {
 #define LZ_CASE1(ID, SET, SP, ...) \
   case 100 * SP + 20 * SET + ID: hipLaunchKernelGGL((k_lz_carry<SET, __VA_ARGS__, SP>), grid, block, 0, c.stream, A); break;

@@ -116,7 +116,7 @@ struct LzNtt {
 // CRT of the planes and carry.
 struct LzCarry {
   const uint32_t* src;                        // planes
-  const uint32_t* twi;                        // inverse roots of a split transform, prime k at + k n
+  const uint32_t* join;                       // constants of a split transform (LzJoin), prime k at + 8 k
   uint32_t* dst;                              // digits
   uint32_t* dst2;                             // snapshot of flagged positions, or null
   uint32_t* neg;                              // receives the sign of the number, or null

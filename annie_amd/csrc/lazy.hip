@@ -347,7 +347,7 @@ __device__ __forceinline__ uint32_t lz_multiplier(const LzMult& m, uint32_t pos,
 // single-pass kernels of short launches): workgroup `row` computes the node of
 // level SP it owns straight from the digits, position i of it from the 2^SP
 // digits i + t 2^M, so that no column pass and no exchange come before it; the
-// carry undoes those levels as it loads (lz_join).  Position i from digits x_t:
+// carry undoes those levels as it loads (LzJoin).  Position i from digits x_t:
 // level 0 pairs t and t + 2^{SP - 1} with root r(0, 0), and so on; the sign of
 // each level's root is the branch that leads to `row`.  Within 1.5 p + 0.8 p SP.
 constexpr int lz_split_in(int SP) { return lz_in(0) + 205 * SP; }
@@ -483,7 +483,7 @@ __global__ void __launch_bounds__(lz_row_threads(M, LR)) k_lz_row(const LzNtt A)
         x[e] = uint32_t(lz_mul(lz_mul(int32_t(x[e]), y, P), int32_t(op[e]), P));
       }
     }
-    // Single-pass values go to the carry; a column pass or lz_join follows
+    // Single-pass values go to the carry; a column pass or LzJoin follows
     // otherwise.
     lz_inv<W, M, LR, NR - 1, ROOTS, SRC != 0 && SP == 0>(x, tg, lineRoot, twi, P, gst, lld, lst, ti, ri);
   } else {
@@ -833,37 +833,36 @@ __device__ __forceinline__ void lz_crt(const int32_t (&r)[KP], uint32_t (&v)[LZ_
 
 // Residue of a plane at coefficient i: the word itself, or, after a transform
 // split over 2^SP workgroups, its last SP inverse levels: coefficient t 2^M + j
-// from the values y_b of position j (each within 1.6 p, so four sum up in a
-// word).  Both branches of a level are one product, by the root or by 1 (one:
-// 2^32 mod p), so that waves across a boundary take no detour; the roots are
-// entries 1 .. 3 of the plane's table, uniform loads.
+// from the values y_b of position j (each within 1.6 p).  The signs of a level
+// hang on bits of t alone and its roots multiply out, so two sums times two
+// constants of (plane, t) and one reduction do: join holds them, a pair per t
+// (one for SP = 1), filled by k_lz_roots.  |sum| <= 2 3.2 p p / 2 and the result
+// is within 0.8 p.  Level by level, with a reduced product for each of three
+// butterflies, the two carries of 2^13 coefficients split four ways took 5.4 and
+// 4.2 us, now 4.0 and 3.4; a squaring of 2^14 coefficients 30.7 us, now 27.2.
 template <int SP>
-__device__ __forceinline__ int32_t lz_join(const uint32_t* src, uint32_t i, int LN, const uint32_t* twi, uint32_t q, uint32_t p,
-                                           int32_t one) {
-  if constexpr (SP == 0) {
-    return int32_t(ld_w(src, i));
-  } else {
+struct LzJoin {
+  uint32_t y[1 << SP];
+  uint2 c;
+  __device__ __forceinline__ void load(const uint32_t* src, uint32_t i, int LN, const uint32_t* join) {
     const int M = LN - SP;
-    const uint32_t t = i >> M, j = i & ((1u << M) - 1u);
-    const uint4 w = *reinterpret_cast<const uint4*>(twi);
-    const uint32_t root[4] = {w.x, w.y, w.z, w.w};
-    int32_t y[1 << SP];
+    const uint32_t j = SP == 0 ? i : i & ((1u << M) - 1u);
 #pragma unroll
-    for (int b = 0; b < (1 << SP); ++b) y[b] = int32_t(ld_w(src, j + (uint32_t(b) << M)));
-#pragma unroll
-    for (int l = SP - 1; l >= 0; --l) {
-      const bool odd = ((t >> (SP - 1 - l)) & 1u) != 0u;
-#pragma unroll
-      for (int b = 0; b < (1 << l); ++b) {
-        const int32_t r0 = int32_t(root[(1 << l) + b]);
-        const int32_t r = odd ? r0 : one;
-        const uint32_t rq = odd ? uint32_t(r0) * q : uint32_t(one) * q;
-        y[b] = lz_mulc(y[2 * b] + (odd ? -y[2 * b + 1] : y[2 * b + 1]), r, rq, p);
-      }
-    }
-    return y[0];
+    for (int b = 0; b < (1 << SP); ++b) y[b] = ld_w(src + (size_t(b) << M), j);
+    if constexpr (SP == 1) c.x = ld_w(join, 2u * (i >> M));
+    if constexpr (SP == 2) c = *reinterpret_cast<const uint2*>(join + 2u * (i >> M));
   }
-}
+  // neg: minus the lowest bit of t, the sign of the first level.
+  __device__ __forceinline__ int32_t value(uint32_t neg, uint32_t q, uint32_t p) const {
+    if constexpr (SP == 0) {
+      return int32_t(y[0]);
+    } else {
+      int64_t v = int64_t(int32_t(y[0] + (y[1] ^ neg) - neg)) * int32_t(c.x);
+      if constexpr (SP == 2) v += int64_t(int32_t(y[2] + (y[3] ^ neg) - neg)) * int32_t(c.y);
+      return int32_t(v >> 32) - __mulhi(int32_t(uint32_t(v) * q), int32_t(p));
+    }
+  }
+};
 
 // Grid: (ceil(waves / 4), slots); block 256.
 // EX > 0: the result leaves in the external format, EX residue planes at dst (one
@@ -878,14 +877,6 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   const size_t n = size_t(1) << A.LN;
   const uint32_t slot = lz_slot(A.slot_ids, blockIdx.y);
   const size_t so = size_t(slot) * A.slot_stride;
-  const uint32_t cbits = A.cbits_slot ? A.cbits_slot[slot] : uint32_t(A.cbits);
-  const uint32_t sh = cbits & 31u;
-  const uint32_t a = lz_multiplier(A.mul, blockIdx.y, slot);
-  bool snap = false;
-  if (A.dst2 != nullptr) {
-    snap = A.snap != nullptr ? (A.snap[blockIdx.y] & SLOT_SNAP) != 0u
-                             : (A.mul.bits_mode == 2 && ((A.mul.bits[blockIdx.y >> 5] >> (blockIdx.y & 31u)) & 1u));
-  }
   const int lane = int(threadIdx.x & 63u);
   const int wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * 4u + (threadIdx.x >> 6)));
   const int top = int((n - 1) / W);
@@ -893,11 +884,23 @@ __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   for (int w = wave;; --w) {
     const int i = w * W + lane - H;
     const uint32_t idx = i < 0 ? uint32_t(i + int(n)) : (uint32_t(i) < n ? uint32_t(i) : uint32_t(n - 1));
-    int32_t r[KP];
+    // Everything that comes from memory is asked for before the first wait.
+    LzJoin<SP> in[KP];
 #pragma unroll
-    for (int k = 0; k < KP; ++k)
-      r[k] = lz_join<SP>(A.src + so + size_t(k) * n, idx, A.LN, A.twi + size_t(k) * n, cx_inv32(lz_prime(SET, k)),
-                         lz_prime(SET, k), int32_t((uint64_t(1) << 32) % lz_prime(SET, k)));
+    for (int k = 0; k < KP; ++k) in[k].load(A.src + so + size_t(k) * n, idx, A.LN, A.join + 8 * k);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t cbits = A.cbits_slot ? A.cbits_slot[slot] : uint32_t(A.cbits);
+    const uint32_t sh = cbits & 31u;
+    const uint32_t a = lz_multiplier(A.mul, blockIdx.y, slot);
+    bool snap = false;
+    if (A.dst2 != nullptr) {
+      snap = A.snap != nullptr ? (A.snap[blockIdx.y] & SLOT_SNAP) != 0u
+                               : (A.mul.bits_mode == 2 && ((A.mul.bits[blockIdx.y >> 5] >> (blockIdx.y & 31u)) & 1u));
+    }
+    int32_t r[KP];
+    const uint32_t neg = SP == 0 ? 0u : 0u - ((idx >> (A.LN - SP)) & 1u);
+#pragma unroll
+    for (int k = 0; k < KP; ++k) r[k] = in[k].value(neg, cx_inv32(lz_prime(SET, k)), lz_prime(SET, k));
     uint32_t v[LZ_MAXL];
     lz_crt<SET, KP, L>(r, v);
     if (a != 1u) {
@@ -1032,8 +1035,11 @@ __global__ void __launch_bounds__(256) k_lz_pack(const LzPack A) {
 // Root tables (heap-indexed as make_tables in plan.h) in signed Montgomery form,
 // |w| <= p / 2: entry 2^l + b is psi^e with e = 2 h brv_l(b) (cyclic) or h (2
 // brv_l(b) + 1) (negacyclic), h = n / 2^{l+1}, or its inverse psi^{2n - e}.  pw
-// holds psi^i for i < 2^s, then psi^{i 2^s}, per prime (s = ceil(LN / 2)).
-__global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int KR, int KQ, const LzPrimes C) {
+// holds psi^i for i < 2^s, then psi^{i 2^s}, per prime (s = ceil(LN / 2)).  Behind
+// the tables, for a transform split over 2^SP workgroups, eight words per plane
+// (KR cyclic, KQ negacyclic) for LzJoin.
+__global__ void __launch_bounds__(256)
+k_lz_roots(uint32_t* tw, const uint32_t* pw, int LN, int SP, int KR, int KQ, const LzPrimes C) {
   const uint32_t n = 1u << LN, idx = blockIdx.x * 256u + threadIdx.x;
   const int k = int(blockIdx.y);
   if (idx >= n) return;
@@ -1056,6 +1062,17 @@ __global__ void __launch_bounds__(256) k_lz_roots(uint32_t* tw, const uint32_t* 
     tw[(2 * size_t(KR) + k) * n + idx] = root(eQ);
     tw[(2 * size_t(KR) + KQ + k) * n + idx] = root((2u * n - eQ) & mask);
   }
+  if (SP > 0 && idx < (2u << SP)) {
+    // Of coefficient block t: the factor of y_0 (idx even) or y_2, inverse roots
+    // of entries 1 (the last level) and 2 or 3, and -1 = psi^n where the last
+    // level subtracts.
+    const uint32_t t = idx >> 1, j = idx & 1u, last = t >> (SP - 1), first = SP == 2 ? t & 1u : 0u;
+    uint32_t* join = tw + (2 * size_t(KR) + 2 * size_t(KQ)) * n;
+    const uint32_t sign = last != 0u && j != 0u ? n : 0u;
+    const uint32_t cyc = first * j * (n / 2u), nega = last * (n / 2u) + first * (n / 4u) * (1u + 2u * j);
+    join[8 * k + idx] = root((2u * n - cyc + sign) & mask);
+    if (k < KQ) join[8 * (KR + k) + idx] = root((2u * n - nega + sign) & mask);
+  }
 }
 
 // Instantiations, looked up by the host engine (lz_geometry chooses among
@@ -1076,6 +1093,7 @@ LZ_ROW1(12, 4, 0)
 LZ_ROW1(13, 4, 0)
 LZ_ROW1(11, 3, 1)
 LZ_ROW1(12, 3, 1)
+LZ_ROW1(11, 3, 2)
 LZ_ROW1(12, 3, 2)
 LZ_ROW(7, 3, 0, 0, 0)
 LZ_ROW(8, 3, 0, 0, 0)

@@ -174,8 +174,8 @@ def test_large_multiplier_moves_to_long_primes(gpu):
 
 # Batches on both sides of each rule of the transforms' geometry: split over two
 # or four workgroups, one workgroup of eight or sixteen elements per thread.
-@pytest.mark.parametrize("bits,slots", [(20000, 300), (50000, 130), (200000, 16), (200000, 17), (200000, 40), (332000, 32),
-                                        (332000, 33), (560000, 3), (560000, 33), (1000003, 8)])
+@pytest.mark.parametrize("bits,slots", [(20000, 300), (50000, 130), (200000, 16), (200000, 17), (200000, 40), (332000, 8),
+                                        (332000, 9), (332000, 32), (332000, 33), (560000, 3), (560000, 33), (1000003, 8)])
 def test_batch_geometries(gpu, bits, slots):
     """Three moduli over all slots, squared together and one slot at a time:
     every slot holds its power."""
@@ -220,7 +220,8 @@ def test_batch_geometries(gpu, bits, slots):
         pick = (u32 * 2)(*one)
         assert lib.annie_hip_batch_get(h, 1, pick, 2, out.ctypes.data_as(p64), L, nout) == 0
         for j, s in enumerate(one):
-            assert int.from_bytes(out[j].tobytes(), "little") == want[s % 3] ** 2 % Ns[s % 3], f"product of slot {s}"
+            got = int.from_bytes(out[j, :nout[j]].tobytes(), "little")  # words from nout on are not written
+            assert got == want[s % 3] ** 2 % Ns[s % 3], f"product of slot {s}"
     finally:
         lib.annie_hip_destroy(h)
 
