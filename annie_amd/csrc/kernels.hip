@@ -180,7 +180,7 @@ __device__ __forceinline__ void inv_rounds(uint32_t (&x)[1 << LR], uint32_t tg, 
 // 16 elements per thread (LR = 4 levels per register round; 32 elements per
 // thread at rows of 2^11 measured no faster).
 // Grid: (rows / lines-per-block, K, jobs).  Block: lines * 2^M / 16 threads.
-// Rows of 2^11 (the 40M-digit length): five waves per SIMD, so that a one-job
+// Rows of 2^11 (2^21 and 2^22 in two passes): five waves per SIMD, so that a one-job
 // pass over five planes (10,240 waves) is exactly two resident rounds and a
 // two-job pass four, instead of 2.5 and 5 at four waves (the half round left
 // half the chip idle at the end of every one-job pass).

@@ -13,17 +13,18 @@
 // inverse transform and the carry of T_Q out (src/transformGPU.h:523-568 does
 // each product on its own).
 //
-// The primes are below 2^28.2 (slightly wider above 2^20), so that a signed
-// 32-bit word holds +-6.9 p and a butterfly needs no correction: see lazy.hip.  More planes (7 + 5 instead of
-// 4 per transform at K = 4) and fewer transforms come to 29 plane transforms a
-// squaring instead of 32, each at half the instructions, in four launches
-// (lengths up to 2^13) or eight instead of six or twelve.
+// The primes are below 2^28.2 (2^29.9 at 2^22), so that a signed 32-bit word
+// holds +-6.9 p (2.1 p) and a butterfly needs no correction: see lazy.hip.  More
+// planes (7 + 5 instead of 4 per transform at K = 4) and fewer transforms come to
+// 29 plane transforms a squaring instead of 32, each at half the instructions, in
+// four launches (lengths up to 2^13) or eight instead of six or twelve.
 //
-// Measured against the passes over the long primes, one squaring: 2^10 (K =
-// 4) 43.9 -> 16.8 us, 2^13 61.7 -> 31.5, 2^14 (K = 5) 77.4 -> 35.5, 2^16 78.7
-// -> 41.7, 2^19 154 -> 101; one tick of a batch: 130 slots of 2^12 138 -> 89,
-// 300 slots of 2^9 (K = 5) 124 -> 82, nine of 2^13 71 -> 39.  2^23 has
-// too few such primes and stays on the long ones.
+// Measured against the passes over the long primes, us per squaring: 2^10 (K = 4)
+// 43.9 -> 14.0, 2^13 61.9 -> 19.7, 2^14 (K = 5) 77.4 -> 27.1, 2^16 78.6 -> 35.6,
+// 2^19 154 -> 85.5, 2^21 (K = 5) 473 -> 339, 2^22 810 -> 595; one tick of a batch
+// with its read-back: 130 slots of 2^12 138 -> 60, 300 slots of 2^9 (K = 5) 124 ->
+// 33.5, nine of 2^13 71 -> 28.  2^23 has too few such primes and stays on the long
+// ones.
 #pragma once
 #include <cmath>
 #include <cstddef>

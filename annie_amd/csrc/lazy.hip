@@ -866,9 +866,10 @@ struct LzJoin {
 
 // Grid: (ceil(waves / 4), slots); block 256.
 // EX > 0: the result leaves in the external format, EX residue planes at dst (one
-// slot), by waves with the three more halo lanes that the balancing takes. One
-// launch and a pass over the digits less than k_lz_export behind it: a call on 2^10 coefficients 32.5 -> 30.4 us
-// with its synchronisation, on 2^16 55.0 -> 53.9.
+// slot), by waves with the three more halo lanes that the balancing takes.  One
+// launch and a pass over the digits less than k_lz_export behind it: a call on
+// 2^10 coefficients 32.5 -> 30.4 us with its synchronisation, on 2^16 55.0 ->
+// 53.9.
 template <int SET, int KP, int L, int ND, int DL, bool NEGA, int EX, int SP>
 __global__ void __launch_bounds__(256) k_lz_carry(const LzCarry A) {
   constexpr int H = EX > 0 ? ND + LZ_BALANCE : ND, W = 64 - H;

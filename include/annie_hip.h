@@ -73,13 +73,14 @@ int annie_hip_square_mul(annie_hip_t* ctx, int32_t a);
  * annie_hip_square_mul on caller-owned device buffers: x and y hold K planes of
  * n u32 residues (plane-major, the layout of annie_hip_read_register), 16-byte
  * aligned; y may equal x.  Its work registers live in a static device array
- * of the library (one per GPU, 4 K n + 3 n words at the largest size, held
- * until the process ends) instead of the context's own, so the context's
- * registers are untouched.  Limit: K * n <= ANNIE_HIP_NOALLOC_MAX_KN words per
+ * of the library (one per GPU, 11.5 MiB, held until the process ends) instead
+ * of the context's own, so the context's registers are untouched.  Limit: K * n <= ANNIE_HIP_NOALLOC_MAX_KN words per
  * register (ANNIE_ERR_SIZE above it).  Enqueued on the context's stream and
  * returns without waiting.  Every call on one GPU shares that array: calls
  * whose work overlaps on one GPU (other threads, other contexts' streams)
- * race; calls on one stream are ordered. */
+ * race; calls on one stream are ordered.  A multiplier above 4,095 on a context
+ * created for a smaller base moves the context to its larger primes first,
+ * which allocates and waits, once: make such a call before capturing. */
 #define ANNIE_HIP_NOALLOC_MAX_KN ((size_t)1 << 19)
 int annie_hip_square_mul_noalloc(annie_hip_t* ctx, const uint32_t* x, uint32_t* y, int32_t a);
 
@@ -180,9 +181,10 @@ int annie_hip_batch_mul(annie_hip_t* b, size_t dst, size_t src, const uint32_t* 
  * iterations): for each listed slot i, r0 = m * r0^2 for m = mult[i * steps + t],
  * t = 0, 1, ..., up to the slot's first m = 0 (zeros only as a suffix); bit 31
  * of m as in annie_hip_batch_square_mul, allowed on the last squaring of the
- * slot's run only.  One workgroup per slot runs the whole squaring sequence;
- * the registers end equal, word for word, to those of the same squarings
- * issued one by one.  steps <= ANNIE_HIP_RUN_MAX_STEPS.  ANNIE_ERR_SIZE when
+ * slot's run only.  One workgroup per slot runs the whole squaring sequence
+ * (on the short primes the squarings are issued launch by launch); the
+ * registers end equal, word for word, to those of the same squarings issued
+ * one by one.  steps <= ANNIE_HIP_RUN_MAX_STEPS.  ANNIE_ERR_SIZE when
  * the batch's plan has no run kernel (annie_hip_batch_run_supported == 0:
  * transform lengths outside 2^9 .. 2^13, other RNS sizes or digit widths). */
 #define ANNIE_HIP_RUN_MAX_STEPS 256
