@@ -21,7 +21,7 @@
 //
 // Measured against the passes over the long primes, us per squaring: 2^10 (K = 4)
 // 43.9 -> 14.0, 2^13 61.9 -> 19.7, 2^14 (K = 5) 77.4 -> 27.1, 2^16 78.6 -> 35.6,
-// 2^19 154 -> 85.5, 2^21 (K = 5) 473 -> 339, 2^22 810 -> 595; one tick of a batch
+// 2^19 154 -> 85.5, 2^21 (K = 5) 473 -> 347, 2^22 810 -> 599; one tick of a batch
 // with its read-back: 130 slots of 2^12 138 -> 60, 300 slots of 2^9 (K = 5) 124 ->
 // 33.5, nine of 2^13 71 -> 28.  2^23 has too few such primes and stays on the long
 // ones.
